@@ -1281,6 +1281,14 @@ hgdt_status hgdt_operator_instance_stats(hgdt_operator op, int64_t* iterations, 
   });
 }
 
+hgdt_status hgdt_operator_solve_workgroups(hgdt_operator op, int32_t* workgroups)
+{
+  return guarded([&] {
+    require(op && workgroups, HGDT_ERR_INVALID_ARGUMENT, "NULL argument");
+    *workgroups = op->op->last_workgroups;
+  });
+}
+
 hgdt_status hgdt_operator_instance_true_residuals(hgdt_operator op, double* relres)
 {
   return guarded([&] {

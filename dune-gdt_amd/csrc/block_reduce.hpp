@@ -25,11 +25,41 @@ __device__ __forceinline__ int active_block(int nb, const int32_t* __restrict__ 
   return (L < 0 || !list) ? L : list[L];
 }
 
+// v + (v of lane ^ 32 | ^ 16) without LDS: the swap exchanges the upper half (odd rows of 16) of one operand
+// with the lower half (even rows) of the other
+template <bool HALVES>
+__device__ __forceinline__ double add_swapped(double v)
+{
+  const unsigned lo = unsigned(__double2loint(v)), hi = unsigned(__double2hiint(v));
+  if constexpr (HALVES) {
+    const auto a = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+    const auto b = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+    return __hiloint2double(int(b[0]), int(a[0])) + __hiloint2double(int(b[1]), int(a[1]));
+  } else {
+    const auto a = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+    const auto b = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+    return __hiloint2double(int(b[0]), int(a[0])) + __hiloint2double(int(b[1]), int(a[1]));
+  }
+}
+template <int CTRL>
+__device__ __forceinline__ double add_dpp(double v)
+{
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true);
+  return v + __hiloint2double(hi, lo);
+}
+
+// sum over the wave, in every lane: pairs of lanes 32, 16, 8, 4, 2, 1 apart.  After the step of distance d all
+// lanes equal modulo d hold the same value, so a rotation of the row of 16 by 8 or 4 gives the partner's.
+// All six exchanges are vector instructions; as LDS permutes they were a chain of six LDS round trips.
 __device__ __forceinline__ double wave_sum(double v)
 {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1)
-    v += __shfl_xor(v, off, 64);
+  v = add_swapped<true>(v);
+  v = add_swapped<false>(v);
+  v = add_dpp<0x128>(v); // row_ror:8
+  v = add_dpp<0x124>(v); // row_ror:4
+  v = add_dpp<0x4e>(v);  // quad_perm:[2,3,0,1]
+  v = add_dpp<0xb1>(v);  // quad_perm:[1,0,3,2]
   return v;
 }
 

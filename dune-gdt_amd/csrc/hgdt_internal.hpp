@@ -470,6 +470,7 @@ struct Operator {
   std::vector<int64_t> last_iters;
   std::vector<double> last_relres;
   std::vector<double> last_true_relres; // |b - A x| / |b| at exit (-1: not computed)
+  int32_t last_workgroups = 0;          // of the last solve in one launch (0: kernels per iteration)
 
   // Structured assembly (P1 on the Kuhn tetrahedra of axis-parallel lattices with Laplace element forms and
   // constant or per-element sources): the symmetric DIA storage of the solver (diagonal and upper diagonals),

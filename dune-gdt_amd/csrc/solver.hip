@@ -48,6 +48,7 @@
 
 #include "hgdt_internal.hpp"
 #include "block_reduce.hpp"
+#include "resident.hpp"
 
 namespace hgdt {
 namespace {
@@ -1382,6 +1383,7 @@ struct SolverCache {
   int graph_chunk = 0;
   int64_t graph_version = -1;
   int64_t version = 0;
+  ResidentPlan resident;
   ~SolverCache()
   {
     for (auto& h : host_scalars)
@@ -2382,6 +2384,36 @@ static void launch_iteration(const Operator& op, const PcgParams& P, int par, hi
   });
 }
 
+// plan of the solve in one launch (resident.hip) for the operator's storage and launch shapes
+static ResidentPlan& resident_plan(Operator& op)
+{
+  SolverCache& C = cache_of(op);
+  ResidentPlan& plan = C.resident;
+  if (plan.version != C.version) {
+    plan.usable = false;
+    if (kernel_format(op) == FMT_DIAS && op.fmt.format == HGDT_FORMAT_DIA)
+      resident_plan_dia(plan, op, C.s_offs, C.s_nu);
+    plan.version = C.version;
+  }
+  return plan;
+}
+
+static bool resident_solve(Operator& op, const PcgParams& P, hipStream_t stream)
+{
+  const SolverFormat& F = op.fmt;
+  SolverCache& C = cache_of(op);
+  ResidentParams R{};
+  R.n = op.n, R.ninst = P.ninst, R.inst_row0 = P.inst_row0;
+  R.a_block = F.A.block, R.v_block = F.V.block;
+  while ((1 << R.v_lg_items) < F.V.items)
+    ++R.v_lg_items;
+  R.s_nu = P.s_nu, R.s_off = P.s_off, R.scaled = P.scaled, R.dsq = P.dsq;
+  R.r = P.r, R.x = P.x, R.r_pub = P.p, R.part2 = P.part2;
+  R.n_a = F.A.nblocks, R.n_v = F.V.nblocks;
+  R.S = P.S, R.max_iter = P.max_iter;
+  return resident_run(C.resident, R, stream, C.host_scalars[0]);
+}
+
 void Operator::apply_inverse(const double* b, double* x, const hgdt_solver_options& opt, hgdt_solver_stats& st,
                              hipStream_t user_stream)
 {
@@ -2455,7 +2487,10 @@ void Operator::apply_inverse(const double* b, double* x, const hgdt_solver_optio
   // current scalars in record 0 after each chunk; the last step of a solve runs in the chunk after the
   // one whose update met the tolerance (the stopping test is the first thing a step does)
   const int chunk = opt.check_every + (opt.check_every & 1);
-  if (graph && (C.graph == nullptr || C.graph_x != x || C.graph_chunk != chunk || C.graph_version != C.version
+  // in one launch where the vectors fit on the chip (a timed solve issues the kernel that is timed)
+  const bool solved = !opt.time_spmv && resident_plan(*this).usable && resident_solve(*this, P, stream);
+  last_workgroups = solved ? C.resident.workgroups : 0;
+  if (!solved && graph && (C.graph == nullptr || C.graph_x != x || C.graph_chunk != chunk || C.graph_version != C.version
                 || C.graph_b != b || C.graph_maxit != opt.max_iter)) {
     if (C.graph)
       HGDT_HIP(hipGraphExecDestroy(C.graph));
@@ -2565,33 +2600,42 @@ void Operator::apply_inverse(const double* b, double* x, const hgdt_solver_optio
   const int64_t max_chunks = (opt.max_iter + 1 + chunk - 1) / chunk + 1;
   int cur = 0;
   int64_t launched = 0;
-  launch_chunk();
-  ++launched;
-  HGDT_HIP(hipMemcpyAsync(C.host_scalars[cur], d_scalars.ptr, sizeof(PcgScalars) * ninst, hipMemcpyDeviceToHost,
-                          stream));
-  HGDT_HIP(hipEventRecord(C.copied[cur], stream));
-  while (true) {
-    const int nxt = cur ^ 1;
-    bool queued = false;
-    if (launched < max_chunks) {
-      launch_chunk();
-      ++launched;
-      HGDT_HIP(hipMemcpyAsync(C.host_scalars[nxt], d_scalars.ptr, sizeof(PcgScalars) * ninst,
-                              hipMemcpyDeviceToHost, stream));
-      HGDT_HIP(hipEventRecord(C.copied[nxt], stream));
-      queued = true;
-    }
-    HGDT_HIP(hipEventSynchronize(C.copied[cur]));
-    if (all_done(C.host_scalars[cur]) || !queued) {
-      if (!queued)
-        break;
-      cur = nxt;
+  if (!solved) {
+    launch_chunk();
+    ++launched;
+    HGDT_HIP(hipMemcpyAsync(C.host_scalars[cur], d_scalars.ptr, sizeof(PcgScalars) * ninst, hipMemcpyDeviceToHost,
+                            stream));
+    HGDT_HIP(hipEventRecord(C.copied[cur], stream));
+    while (true) {
+      const int nxt = cur ^ 1;
+      bool queued = false;
+      if (launched < max_chunks) {
+        launch_chunk();
+        ++launched;
+        HGDT_HIP(hipMemcpyAsync(C.host_scalars[nxt], d_scalars.ptr, sizeof(PcgScalars) * ninst,
+                                hipMemcpyDeviceToHost, stream));
+        HGDT_HIP(hipEventRecord(C.copied[nxt], stream));
+        queued = true;
+      }
       HGDT_HIP(hipEventSynchronize(C.copied[cur]));
-      break;
+      if (all_done(C.host_scalars[cur]) || !queued) {
+        if (!queued)
+          break;
+        cur = nxt;
+        HGDT_HIP(hipEventSynchronize(C.copied[cur]));
+        break;
+      }
+      if (ninst > 1)
+        compact(C.host_scalars[cur]);
+      cur = nxt;
     }
-    if (ninst > 1)
-      compact(C.host_scalars[cur]);
-    cur = nxt;
+  } else if (ninst > 1) {
+    // the workgroups of an instance end with it: counted as narrowings while others went on
+    int64_t most = 0;
+    for (int i = 0; i < ninst; ++i)
+      most = std::max<int64_t>(most, C.host_scalars[0][i].iters);
+    for (int i = 0; i < ninst; ++i)
+      compactions += C.host_scalars[0][i].iters < most;
   }
   hipLaunchKernelGGL(k_cg_finish, dim3(blocks_for(n, 256)), dim3(256), 0, stream, n, fmt.d_dh.ptr, x);
   HGDT_HIP(hipGetLastError());

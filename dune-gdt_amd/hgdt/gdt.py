@@ -1047,6 +1047,12 @@ class MatrixOperator:
         L.call("hgdt_operator_instance_stats", self._h, it.ctypes.data_as(L._pi64), rr.ctypes.data_as(L._pdbl))
         return it, rr
 
+    def solve_workgroups(self):
+        """workgroups of the launch that ran the last apply_inverse as a whole (0: kernels per iteration)"""
+        w = ctypes.c_int32()
+        L.call("hgdt_operator_solve_workgroups", self._h, ctypes.byref(w))
+        return int(w.value)
+
     def adjoint_log_diffusion_gradient(self, u, lam, form_index=0, stream=None):
         """grad_e = -kappa_e lambda_e^T Khat_e u_e (no reference counterpart)."""
         u = _dvec(u, self.shape[0], "u")

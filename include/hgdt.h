@@ -431,7 +431,8 @@ typedef struct hgdt_solver_stats {
   int64_t step_bytes;     /* algorithmic bytes of the solver's operator application (the kernel timed
                              by time_spmv) */
   int64_t compactions;    /* batches: times the launches were narrowed to the blocks of the instances
-                             still iterating */
+                             still iterating (a solve in one launch: instances that ended, and with them
+                             their workgroups, before the last one) */
   double true_relres;     /* max over instances of |b - A x| / |b| at exit, recomputed from the returned x
                              (-1 when options.true_residual is 0) */
   int32_t column_staged;  /* 1: the solver's operator application ran with column staging (see
@@ -457,6 +458,8 @@ hgdt_status hgdt_operator_instance_stats(hgdt_operator op, int64_t* iterations, 
  * -1 when it was not computed).  The reference's apply_inverse checks the solver's result the same way
  * (operators/matrix-based.hh:148-159 with XT::LA::Solver's post-check of the residual). */
 hgdt_status hgdt_operator_instance_true_residuals(hgdt_operator op, double* relres);
+/* workgroups of the launch that ran the last apply_inverse as a whole (0: it issued kernels per iteration) */
+hgdt_status hgdt_operator_solve_workgroups(hgdt_operator op, int32_t* workgroups);
 
 /* Adjoint element kernel (no reference counterpart): for the Laplace form appended at position
  * `form_index` among the element forms, with per-element diffusion kappa_e,
