@@ -10,23 +10,31 @@
 // Exchange: every block partial has a slot in global memory that holds a sentinel until its workgroup has
 // stored it; every workgroup of the instance reads all slots, again until none holds the sentinel, and adds
 // them in block order.  So the values are their own flags: one store and one load between the slowest
-// workgroup and all others (2.4-3.5 us with 256 workgroups, 1-1.3 us with 16).  Two sets of slots alternate, by the
-// parity of the step: a workgroup puts the sentinel back into its slots of the other set when it stores to one;
-// by then every workgroup has read that other set (it stored to the exchange in between afterwards), and none
-// polls it again before this workgroup has stored to that exchange, which it does after waiting for its
-// earlier stores.  Slots, published rows and polls are relaxed atomics at agent scope (the XCDs' L2 caches
-// are coherent for these); a workgroup waits for its published rows (vmcnt 0) before the barrier ahead of the
-// store of its partials, so whoever has seen the partials sees the rows.
+// workgroup and all others (2.4-3.5 us with 256 workgroups, 1-1.3 us with 16).  The sets of slots rotate,
+// three for p.q and two for the norms: a workgroup empties its slots of the set that comes up next but one (norms:
+// next) when it stores to one.  By then every workgroup has read what they held (it has stored to an exchange since),
+// and none polls them again before this workgroup has stored to the p.q exchange in between, which it does after
+// waiting for its earlier stores (vmcnt 0).  The rows of r that other workgroups read go the same way, through two
+// arrays with the sentinel.  Slot accesses are relaxed atomics at agent scope, for which the XCDs' L2
+// caches are coherent; as every value is its own flag, no order between different addresses is needed beyond that.
 //
 // Every value is computed by the operations of the three kernels in their order (row sums, block partials in
 // the operator's and the vector partition, sums over the partials), so a solve gives the same bits on either path,
 // alone or in a batch.
+//
+// Measured (us per iteration, three kernels -> one launch, before and after the default row blocks became those of a
+// workgroup's lanes): Q1 128^2 14 -> 4.5, 701x523 18 -> 8.6, 1023^2 33 -> 10.7, P1 48^3 x 6 19 -> 7.3, eight of these in a
+// batch 33 -> 9.4; SELL: P1 triangles of a mesh with 160 401 vertices 18 -> 7.5, P2 triangles with 90 201 DoFs 18 -> 8.2.
+// What is left of an iteration: two exchanges of 1-2.5 us, the barriers and sums around them, and for 4096 rows per
+// workgroup LDS (13 reads of 8 bytes per row at 128 B per clock: 1.4 us).
 //
 // All workgroups of a team must be on the chip together: the host launches at most one per CU and counts the
 // CUs of all running launches of the process.  A wait that outlasts its limit (another process holds the
 // CUs) sets a flag at which every workgroup ends; the caller then solves with the three kernels.
 
 #include <algorithm>
+#include <atomic>
+#include <cmath>
 #include <condition_variable>
 #include <cstring>
 #include <map>
@@ -38,8 +46,9 @@
 namespace hgdt {
 namespace {
 
-constexpr int RES_LANES = 512, RES_WAVES = RES_LANES / 64;
+constexpr int RES_LANES = RES_BLOCK, RES_WAVES = RES_LANES / 64;
 constexpr int RES_MAX_SLOTS = 16;
+constexpr int RES_HALO = 3; // halo rows a lane asks for while the residual norms are exchanged
 constexpr int RES_GROUPS = RES_WAVES * RES_MAX_SLOTS; // 64-row groups of a workgroup
 constexpr int64_t RES_LDS = 150 * 1024;               // dynamic LDS of a workgroup, of 160 KB
 
@@ -61,37 +70,38 @@ __device__ __forceinline__ unsigned long long slot_load(const double* p)
 {
   return __hip_atomic_load(reinterpret_cast<const unsigned long long*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ __forceinline__ void publish(double* p, double v)
-{
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ double published(const double* p)
-{
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// waits until the slot holds a value; false when the wait is over its limit or another workgroup gave up
-__device__ bool slot_wait(const double* p, int* gave_up, int64_t ticks, unsigned long long& u)
-{
-  const long long t0 = wall_clock64();
-  for (int k = 1;; ++k) {
-    __builtin_amdgcn_s_sleep(1);
-    u = slot_load(p);
-    if (u != RES_EMPTY)
-      return true;
-    if ((k & 255) == 0 && (__hip_atomic_load(gave_up, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ||
-                           wall_clock64() - t0 > ticks)) {
-      __hip_atomic_store(gave_up, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+// limit of a wait: over() after each failed look, true when the wait is to end (its limit is reached, or another
+// workgroup gave up).  The first looks follow each other at once; later ones sleep and watch the clock.
+struct Patience {
+  int looks = 0;
+  long long since = 0;
+  __device__ __forceinline__ bool over(int* gave_up, int64_t ticks)
+  {
+    if (++looks < 256)
       return false;
-    }
+    __builtin_amdgcn_s_sleep(2);
+    if (looks == 256)
+      since = wall_clock64();
+    if (looks & 255)
+      return false;
+    if (!__hip_atomic_load(gave_up, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) && wall_clock64() - since <= ticks)
+      return false;
+    __hip_atomic_store(gave_up, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return true;
   }
+};
+
+// a value that is the same in all lanes, as a scalar
+__device__ __forceinline__ int uniform(int v)
+{
+  return __builtin_amdgcn_readfirstlane(v);
 }
 
 // element `i` of an array whose base is the same for the whole wave: a 32-bit byte offset per lane
 template <class T>
 __device__ __forceinline__ T* at(T* base, unsigned i)
 {
-  return reinterpret_cast<T*>(reinterpret_cast<uintptr_t>(base) + i * unsigned(sizeof(T)));
+  return reinterpret_cast<T*>(reinterpret_cast<char*>(const_cast<std::remove_const_t<T>*>(base)) + i * unsigned(sizeof(T)));
 }
 
 // sums of `count` partials of NV values as Partials::sum adds them (lane t of `block` lanes adds the partials t,
@@ -103,7 +113,6 @@ __device__ __forceinline__ bool exchange_sum(const double* slots, const double (
                                              int block, double (*red)[RES_WAVES], int* failed, int* gave_up,
                                              int64_t ticks, double (&tot)[NV])
 {
-  constexpr int U = 4 / NV;
   const int t = threadIdx.x;
 #pragma unroll
   for (int k = 0; k < NV; ++k)
@@ -114,61 +123,86 @@ __device__ __forceinline__ bool exchange_sum(const double* slots, const double (
       for (int k = 0; k < NV; ++k)
         tot[k] += own[k];
   } else if (t < block) {
-    bool ok = true;
-    for (int b = t; b < count && ok; b += U * block) {
-      unsigned long long u[U][NV];
+    for (int b = t; b < count; b += block) {
+      unsigned long long u[NV];
+      Patience wait;
+      while (true) {
+        bool empty = false;
 #pragma unroll
-      for (int j = 0; j < U; ++j)
-        if (b + j * block < count)
+        for (int k = 0; k < NV; ++k)
+          u[k] = slot_load(at(slots, unsigned(b) * NV + k));
 #pragma unroll
-          for (int k = 0; k < NV; ++k)
-            u[j][k] = slot_load(at(slots, unsigned(b + j * block) * NV + k));
+        for (int k = 0; k < NV; ++k)
+          empty = empty || u[k] == RES_EMPTY;
+        if (!empty)
+          break;
+        if (wait.over(gave_up, ticks)) {
+          *failed = 1;
+          break;
+        }
+      }
+      if (*failed)
+        break;
 #pragma unroll
-      for (int j = 0; j < U; ++j)
-        if (b + j * block < count)
-#pragma unroll
-          for (int k = 0; k < NV; ++k) {
-            if (u[j][k] == RES_EMPTY)
-              ok = ok && slot_wait(at(slots, unsigned(b + j * block) * NV + k), gave_up, ticks, u[j][k]);
-            tot[k] += __longlong_as_double((long long)u[j][k]);
-          }
+      for (int k = 0; k < NV; ++k)
+        tot[k] += __longlong_as_double((long long)u[k]);
     }
-    if (!ok)
-      *failed = 1;
   }
-  const int nw = block >> 6;
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
-    const double w = wave_sum(tot[k]);
+    const double w = wave_sum(tot[k]); // (0 in the waves past `block`: added below without a change)
     if ((t & 63) == 0)
       red[k][t >> 6] = w;
   }
   __syncthreads();
-  if (*failed)
+  if (uniform(*failed))
     return false;
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
     double s = 0.;
-    for (int w = 0; w < nw; ++w)
+#pragma unroll
+    for (int w = 0; w < RES_WAVES; ++w)
       s += red[k][w];
     tot[k] = s;
   }
   return true;
 }
 
-// PCG of the tasks of one workgroup, one after the other.  S rows per lane; lane t holds row j of its layer
-// s >> lg (layers of RES_LANES << lg rows, lg the vector blocks' items): the rows of vector block (layer,
-// t / v_block), lane t % v_block.  NU: strict upper slots compiled for (missing ones have zero values).  KEEP: the
-// matrix rows stay in registers, else they are read every iteration.
-template <int S, int NU, bool KEEP>
+// g consecutive LDS values added in order (g a power of two up to 16), four loads at a time
+__device__ __forceinline__ double add_run(const double* v, int g)
+{
+  double s = 0.;
+  if (g == 1)
+    return s + v[0];
+  if (g == 2)
+    return s + v[0] + v[1];
+  for (int w = 0; w < g; w += 4) {
+    const double a = v[w], b = v[w + 1], c = v[w + 2], d = v[w + 3];
+    s += a, s += b, s += c, s += d;
+  }
+  return s;
+}
+
+// PCG of the tasks of one workgroup, one after the other.  Lane t holds rows t, t + RES_LANES, ... of the workgroup,
+// one per slot.  Vector blocks have 1 << LG rows per lane: RES_LANES lanes, or (LG = 0) any number that divides it.  So
+// a slot's rows are a constant away from slot 0's and LDS is read at constant offsets.  Rows past the end of the instance
+// hold zeros and take part like others.  NU: strict upper slots compiled for (missing ones have zero values).
+// KEEP != 0: the matrix rows stay in registers, else they are read every iteration.
+// SAME: the operator blocks are the vector blocks; else they have one row per lane (64-row sums combined by threads).
+// NU = 0: SELL-64 storage; p of the own rows is followed by the halo, a list of rows, and the entries hold positions
+// in that; KEEP: entries of a row that registers hold (at least the widest slice's).
+template <int S, int LG, bool SAME, int NU, int KEEP>
 __global__ void __launch_bounds__(RES_LANES) k_pcg_resident(ResidentParams P)
 {
   extern __shared__ double pl[]; // p of the own rows and `reach` rows to either side (0 outside the instance)
   __shared__ double ga[RES_GROUPS], gv[2][RES_GROUPS];
   __shared__ double red1[1][RES_WAVES], red2[2][RES_WAVES];
   __shared__ int failed;
+  constexpr int ITEMS = 1 << LG, R = S * RES_LANES;
+  constexpr bool SELL = NU == 0;
+  constexpr bool LEAN = S > 8; // registers hold r only: q lies in LDS, x and D^{1/2} are read (x written) in every step
+  constexpr int MU = SELL ? 1 : NU;
   const int t = threadIdx.x, wave = t >> 6;
-  const int lg = P.v_lg_items, items = 1 << lg;
   const int vwaves = P.v_block >> 6;
   if (t == 0)
     failed = 0;
@@ -181,36 +215,68 @@ __global__ void __launch_bounds__(RES_LANES) k_pcg_resident(ResidentParams P)
     const int64_t* __restrict__ so = P.s_off + int64_t(K.inst) * ku;
     const bool alone = K.team == 1;
     const int rows = K.rows;
-    int off[NU];
-    int reach = 0;
+    int off[MU];
+    int reach = 0; // rows ahead of the own ones in pl
 #pragma unroll
     for (int u = 0; u < NU; ++u) {
       const int64_t o = u < ku ? so[u] : 0; // padding slots: values 0, offset 0
       off[u] = o < hi - lo ? int(o) : 0;
       reach = max(reach, off[u]);
     }
-    // row of slot s relative to the own rows: a lane's part and the slot's (the same in all lanes).  The lane's part
-    // is made opaque in every step, so that the compiler does not keep S addresses of every array in registers
-    int tb = (((t / P.v_block) * P.v_block) << lg) + t % P.v_block;
-    auto row = [&](int s) { return (((s >> lg) * RES_LANES) << lg) + (s & (items - 1)) * P.v_block + tb; };
     const int below = int(min(K.row0 - lo, int64_t(reach)));        // rows of the instance below the own ones
     const int above = int(min(hi - K.row0 - rows, int64_t(reach))); // and above, at most `reach`
-    double r[S], x[S], sq[S];
-    double au[KEEP ? S : 1][NU], al[KEEP ? S : 1][NU];
+    const int nhalo = SELL ? K.nhalo : below + above;
+    // row of halo entry e, and its place in pl
+    const int32_t* const hrow = P.halo_rows + (SELL ? K.halo0 : 0);
+    auto halo_row = [&](int e) { return SELL ? int64_t(hrow[e]) : K.row0 - below + (e < below ? e : rows + e); };
+    auto halo_place = [&](int e) { return SELL ? R + e : reach - below + (e < below ? e : rows + e); };
+    double r[S], x[LEAN ? 1 : S], sq[LEAN ? 1 : S];
+    double au[!SELL && KEEP ? S : 1][MU], al[!SELL && KEEP ? S : 1][MU];
+    constexpr int KW = SELL && KEEP ? KEEP : 2; // (even)
+    double mv[SELL && KEEP ? S : 1][KW];
+    uint32_t mi[SELL && KEEP ? S : 1][KW / 2];
+    int width[SELL ? S : 1];
     __syncthreads(); // the previous task's last reads of LDS
-    for (int e = t; e < rows + 2 * reach; e += RES_LANES) {
+    for (int e = t; e < R + 2 * reach; e += RES_LANES) {
       const int o = e - reach;
       pl[e] = (o >= -below && o < rows + above) ? P.r[K.row0 + o] : 0.;
     }
+    if constexpr (SELL)
+      for (int e = t; e < nhalo; e += RES_LANES)
+        pl[R + e] = P.r[halo_row(e)];
 #pragma unroll
     for (int s = 0; s < S; ++s) {
-      const int o = row(s);
+      const int o = t + s * RES_LANES;
       const int64_t i = K.row0 + o;
       const bool in = o < rows;
       r[s] = in ? P.r[i] : 0.;
-      x[s] = in ? P.x[i] : 0.;
-      sq[s] = in ? P.dsq[i] : 0.;
-      if constexpr (KEEP)
+      if constexpr (LEAN) {
+        if (in)
+          P.x_work[i] = P.x[i];
+      } else {
+        x[s] = in ? P.x[i] : 0.;
+        sq[s] = in ? P.dsq[i] : 0.;
+      }
+      if constexpr (SELL) {
+        width[s] = 0;
+        if constexpr (KEEP != 0)
+#pragma unroll
+          for (int k = 0; k < KW; ++k)
+            mv[s][k] = 0., mi[s][k / 2] = 0u;
+        if (uniform((s * RES_WAVES + wave) * 64) < rows) {
+          const int64_t* sp = P.slice_ptr + K.slice0 + s * RES_WAVES + uniform(wave);
+          const int64_t first = sp[0];
+          width[s] = int((sp[1] - first) >> 6);
+          if constexpr (KEEP != 0)
+#pragma unroll
+            for (int k = 0; k < KW; ++k)
+              if (k < width[s]) {
+                mv[s][k] = P.scaled[first + k * 64 + (t & 63)];
+                mi[s][k / 2] |= uint32_t(P.sell_local[first + k * 64 + (t & 63)]) << (k % 2 ? 16 : 0);
+              }
+        }
+      }
+      if constexpr (!SELL && KEEP)
 #pragma unroll
         for (int u = 0; u < NU; ++u) {
           const bool on = in && u < ku && off[u] > 0;
@@ -219,10 +285,12 @@ __global__ void __launch_bounds__(RES_LANES) k_pcg_resident(ResidentParams P)
         }
     }
     const double tol2 = P.S[K.inst].tol2;
-    const int own_na = (rows + P.a_block - 1) / P.a_block;
-    const int own_nv = (rows + (P.v_block << lg) - 1) / (P.v_block << lg);
-    // own rows [0, pub_lo) and [pub_hi, rows) are read by other workgroups of the team
-    const int pub_lo = K.rank > 0 ? reach : 0, pub_hi = K.rank + 1 < K.team ? rows - reach : rows;
+    const int own_na = (rows + P.a_rows - 1) / P.a_rows;
+    const int own_nv = (rows + P.v_block * ITEMS - 1) / (P.v_block * ITEMS);
+    // own rows [0, pub_lo) and [pub_hi, ...) are read by other workgroups of the team
+    // (SELL: the slots in `pub`)
+    const uint32_t pub = SELL ? P.publish[int64_t(K.mask) * RES_LANES + t] : 0u;
+    const int pub_lo = K.rank > 0 ? min(reach, rows) : 0, pub_hi = K.rank + 1 < K.team ? rows - reach : R;
     double rn[2], rho_prev = 0., beta = 0.;
     {
       // the initial residual's partials are complete: summed from memory, in the same order
@@ -237,131 +305,288 @@ __global__ void __launch_bounds__(RES_LANES) k_pcg_resident(ResidentParams P)
           red2[k][wave] = w;
       }
       __syncthreads();
+#pragma unroll
       for (int k = 0; k < 2; ++k) {
-        double s = 0.;
-        for (int w = 0; w < vwaves; ++w)
-          s += red2[k][w];
-        rn[k] = s;
+        rn[k] = 0.;
+#pragma unroll
+        for (int w = 0; w < RES_WAVES; ++w)
+          rn[k] += red2[k][w];
       }
     }
     int it = 0, begun = 0;
     int state = 0;
     double alpha = 0., pq = 0.;
+    unsigned long long halo[RES_HALO]; // rows of r of the halo, entries t, t + RES_LANES, ...
+    int hr[RES_HALO];                  // SELL: which rows these are
+    if constexpr (SELL)
+#pragma unroll
+      for (int k = 0; k < RES_HALO; ++k)
+        hr[k] = t + k * RES_LANES < nhalo ? hrow[t + k * RES_LANES] : 0;
     const int max_iter = int(min(P.max_iter, int64_t(0x7ffffff0)));
     for (;; ++it) {
-      asm volatile("" : "+v"(tb));
+      // the lane, opaque in every step: the addresses made from it are not kept in registers across steps
+      int l = t;
+      asm volatile("" : "+v"(l));
       // direction update: stopping test, p = r + beta p on the own rows and on the halo
-      state = (rn[1] <= tol2) ? 1 : (it >= max_iter) ? 2 : 0;
+      state = uniform((rn[1] <= tol2) ? 1 : (it >= max_iter) ? 2 : 0);
       begun = state ? it : it + 1;
       const double rho = rn[0];
       if (state)
         break;
+      double* const pt = pl + reach + l; // p of the lane's row in slot 0
       if (it > 0) {
         beta = rho / rho_prev;
-        for (int e = t; e < below + above; e += RES_LANES) {
-          const int o = e < below ? e - below : rows + e - below;
-          pl[reach + o] = fma(beta, pl[reach + o], published(P.r_pub + K.row0 + o));
-        }
 #pragma unroll
-        for (int s = 0; s < S; ++s) {
-          const int o = row(s);
-          if (o < rows)
-            pl[reach + o] = fma(beta, pl[reach + o], r[s]);
+        for (int s = 0; s < S; ++s)
+          pt[s * RES_LANES] = fma(beta, pt[s * RES_LANES], r[s]);
+        if (!alone) {
+          const double* from = P.r_pub[(it & 1) ^ 1] + (SELL ? 0 : K.row0 - below);
+          for (int e0 = l; e0 < nhalo; e0 += RES_HALO * RES_LANES) {
+            Patience wait;
+            const bool later = e0 >= RES_HALO * RES_LANES; // entries not asked for yet
+            unsigned src[RES_HALO];
+#pragma unroll
+            for (int k = 0; k < RES_HALO; ++k) {
+              const int e = e0 + k * RES_LANES;
+              if (later)
+                halo[k] = RES_EMPTY;
+              if constexpr (SELL)
+                src[k] = later ? (e < nhalo ? hrow[e] : 0) : hr[k];
+              else
+                src[k] = e < below ? e : rows + e;
+            }
+            bool empty;
+            do {
+              empty = false;
+#pragma unroll
+              for (int k = 0; k < RES_HALO; ++k)
+                if (e0 + k * RES_LANES < nhalo && halo[k] == RES_EMPTY)
+                  halo[k] = slot_load(at(from, src[k]));
+#pragma unroll
+              for (int k = 0; k < RES_HALO; ++k)
+                empty = empty || (e0 + k * RES_LANES < nhalo && halo[k] == RES_EMPTY);
+              if (empty && wait.over(P.gave_up, P.wait_ticks)) {
+                failed = 1;
+                break;
+              }
+            } while (empty);
+#pragma unroll
+            for (int k = 0; k < RES_HALO; ++k) {
+              const int e = e0 + k * RES_LANES;
+              if (e < nhalo) {
+                double& pe = pl[halo_place(e)];
+                pe = fma(beta, pe, __longlong_as_double((long long)halo[k]));
+              }
+            }
+          }
         }
       }
       rho_prev = rho;
       __syncthreads();
-      // q = Ah p, and p.q of every group of 64 rows
-      double q[S];
+      if (uniform(failed))
+        return;
+      // q = Ah p, and p.q of the operator blocks: per 64 rows of one slot, or as the vector blocks
+      double q[LEAN ? 1 : S], dot = 0.;
+      double* const ql = pl + R + 2 * reach + l;
+      auto take = [&](int s, double p, double a) { // the product's row of slot s
+        if constexpr (LEAN)
+          ql[s * RES_LANES] = a;
+        else
+          q[s] = a;
+        dot = fma(p, a, dot);
+        if (!SAME || s % ITEMS == ITEMS - 1) {
+          const double w = wave_sum(dot);
+          if ((l & 63) == 0)
+            ga[(SAME ? s >> LG : s) * RES_WAVES + wave] = w;
+          dot = 0.;
+        }
+      };
+      if constexpr (SELL && KEEP != 0) {
+        constexpr int W = 4; // positions read together
 #pragma unroll
-      for (int s = 0; s < S; ++s) {
-        const int o = row(s);
-        const bool in = o < rows;
-        const int oc = min(o, rows - 1);
-        const int c = reach + oc;
-        double bl[NU], bu[NU];
-        if constexpr (!KEEP) {
+        for (int s = 0; s < S; ++s) {
+          double a = 0.;
+#pragma unroll
+          for (int k0 = 0; k0 < KW; k0 += W)
+            if (k0 < width[s]) {
+              double x[W];
+#pragma unroll
+              for (int k = 0; k < W; ++k)
+                x[k] = pl[k % 2 ? mi[s][(k0 + k) / 2] >> 16 : mi[s][(k0 + k) / 2] & 0xffffu];
+#pragma unroll
+              for (int k = 0; k < W; ++k)
+                a = fma(mv[s][k0 + k], x[k], a);
+            }
+          take(s, pt[s * RES_LANES], a);
+        }
+      } else if constexpr (SELL) {
+        // a wave's rows of a slot are one slice; the first entries of the next slice are asked for ahead of the sums
+        constexpr int W = 8;
+        double m[2][W];
+        int c[2][W];
+        int64_t first[2];
+        auto ask = [&](int s) {
+          if (width[s] > 0) {
+            first[s & 1] = P.slice_ptr[K.slice0 + s * RES_WAVES + uniform(wave)];
+#pragma unroll
+            for (int k = 0; k < W; ++k) {
+              const unsigned e = unsigned(min(k, width[s] - 1) * 64 + (l & 63));
+              c[s & 1][k] = *at(P.sell_local + first[s & 1], e);
+              m[s & 1][k] = *at(P.scaled + first[s & 1], e);
+            }
+          }
+        };
+        ask(0);
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+          if (s + 1 < S)
+            ask(s + 1);
+          double a = 0.;
+          if (width[s] > 0) {
+            double x[W];
+#pragma unroll
+            for (int k = 0; k < W; ++k)
+              x[k] = pl[c[s & 1][k]];
+#pragma unroll
+            for (int k = 0; k < W; ++k)
+              if (k < width[s])
+                a = fma(m[s & 1][k], x[k], a);
+            for (int k = W; k < width[s]; ++k) {
+              const unsigned e = unsigned(k * 64 + (l & 63));
+              a = fma(*at(P.scaled + first[s & 1], e), pl[*at(P.sell_local + first[s & 1], e)], a);
+            }
+          }
+          take(s, pt[s * RES_LANES], a);
+        }
+      } else {
+      const double *pd[MU], *pu[MU];
+#pragma unroll
+      for (int u = 0; u < NU; ++u)
+        pd[u] = pt - off[u], pu[u] = pt + off[u];
+      constexpr int G = S < 2 ? S : 2; // slots whose loads are in flight together
+#pragma unroll
+      for (int s0 = 0; s0 < S; s0 += G) {
+        double ml[G][MU], mu[G][MU], xl[G][MU], xu[G][MU], xc[G];
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+          const int s = s0 + g, oc = KEEP ? 0 : min(l + s * RES_LANES, rows - 1);
 #pragma unroll
           for (int u = 0; u < NU; ++u) {
-            // (rows whose partner lies below the instance read the first valid entry, times p = 0)
-            const double* __restrict__ col = P.scaled + int64_t(u < ku ? u : 0) * n + K.row0;
-            bl[u] = *at(col - min(off[u], below), unsigned(max(oc - max(off[u] - below, 0), 0)));
-            bu[u] = *at(col, unsigned(oc));
+            if constexpr (KEEP) {
+              ml[g][u] = al[s][u], mu[g][u] = au[s][u];
+            } else {
+              // (rows whose partner lies below the instance read the first valid entry, times p = 0)
+              const double* col = P.scaled + int64_t(u < ku ? u : 0) * n + K.row0;
+              ml[g][u] = *at(col - min(off[u], below), unsigned(max(oc - max(off[u] - below, 0), 0)));
+              mu[g][u] = *at(col, unsigned(oc));
+            }
+            xl[g][u] = pd[u][s * RES_LANES], xu[g][u] = pu[u][s * RES_LANES];
           }
+          xc[g] = pt[s * RES_LANES];
         }
-        double a = 0.;
 #pragma unroll
-        for (int u = NU - 1; u >= 0; --u) {
-          const double m = KEEP ? al[KEEP ? s : 0][u] : (off[u] > 0 ? bl[u] : 0.);
-          a = fma(m, pl[c - off[u]], a);
-        }
-        const double pi = pl[c];
-        a += pi;
+        for (int g = 0; g < G; ++g) {
+          const int s = s0 + g;
+          double a = 0.;
 #pragma unroll
-        for (int u = 0; u < NU; ++u) {
-          const double m = KEEP ? au[KEEP ? s : 0][u] : (off[u] > 0 ? bu[u] : 0.);
-          a = fma(m, pl[c + off[u]], a);
+          for (int u = NU - 1; u >= 0; --u)
+            a = fma((KEEP || off[u] > 0) ? ml[g][u] : 0., xl[g][u], a);
+          a += xc[g];
+#pragma unroll
+          for (int u = 0; u < NU; ++u)
+            a = fma((KEEP || off[u] > 0) ? mu[g][u] : 0., xu[g][u], a);
+          if constexpr (!KEEP)
+            a = l + s * RES_LANES < rows ? a : 0.;
+          take(s, xc[g], a);
         }
-        q[s] = a;
-        const double w = wave_sum(in ? pi * a : 0.);
-        if ((t & 63) == 0)
-          ga[o >> 6] = w;
+        if constexpr (!KEEP)
+          asm volatile("" ::: "memory"); // no more matrix loads in flight than there are registers for
+      }
       }
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // the slots cleared by the last exchange are empty
       __syncthreads();
       double own1[1] = {0.};
-      const int par = it & 1;
-      if (t < own_na) {
-        const int g = P.a_block >> 6;
-        for (int w = 0; w < g; ++w)
-          own1[0] += ga[t * g + w];
+      const int par = it & 1, set = it % 3;
+      if (l < own_na) {
+        const int g = SAME ? vwaves : P.a_rows >> 6;
+        own1[0] = add_run(ga + l * g, g);
         if (!alone) {
-          slot_clear(at(P.g1 + (par ^ 1) * P.n_a + K.own_a, unsigned(t)));
-          slot_store(at(P.g1 + par * P.n_a + K.own_a, unsigned(t)), own1[0]);
+          slot_store(at(P.g1 + set * P.n_a + K.own_a, unsigned(l)), own1[0]);
+          slot_clear(at(P.g1 + (it + 2) % 3 * P.n_a + K.own_a, unsigned(l)));
         }
       }
+      double sv[LEAN ? S : 1];
+      if constexpr (LEAN)
+#pragma unroll
+        for (int s = 0; s < S; ++s)
+          sv[s] = *at(P.dsq + K.row0, unsigned(min(l + s * RES_LANES, rows - 1)));
       double tot1[1];
-      if (!exchange_sum<1>(P.g1 + par * P.n_a + K.a0, own1, alone, K.na, P.v_block, red1, &failed, P.gave_up,
+      if (!exchange_sum<1>(P.g1 + set * P.n_a + K.a0, own1, alone, K.na, P.v_block, red1, &failed, P.gave_up,
                            P.wait_ticks, tot1))
         return;
       pq = tot1[0];
-      if (!(pq > 0.)) { // breakdown: the iterate holds every earlier step
+      if (!uniform(pq > 0.)) { // breakdown: the iterate holds every earlier step
         state = 3;
         break;
       }
-      // update: x and r, the partials of the residual norms, the rows other workgroups read
+      // update of r, the partials of the residual norms, the rows other workgroups read
       alpha = rho / pq;
       double v[2] = {0., 0.};
 #pragma unroll
       for (int s = 0; s < S; ++s) {
-        const int o = row(s);
-        if (o < rows) {
-          x[s] = fma(alpha, pl[reach + o], x[s]);
-          const double ri = fma(-alpha, q[s], r[s]);
-          r[s] = ri;
-          const double ru = sq[s] * ri;
-          v[0] = fma(ri, ri, v[0]), v[1] = fma(ru, ru, v[1]);
-          if (!alone && (o < pub_lo || o >= pub_hi))
-            publish(at(P.r_pub + K.row0, unsigned(o)), ri);
-        }
-        if ((s & (items - 1)) == items - 1) {
+        const double ri = fma(-alpha, LEAN ? ql[s * RES_LANES] : q[LEAN ? 0 : s], r[s]);
+        r[s] = ri;
+        const double ru = (LEAN ? sv[LEAN ? s : 0] : sq[LEAN ? 0 : s]) * ri;
+        v[0] = fma(ri, ri, v[0]), v[1] = fma(ru, ru, v[1]);
+        if (s % ITEMS == ITEMS - 1) {
           const double w0 = wave_sum(v[0]), w1 = wave_sum(v[1]);
-          if ((t & 63) == 0)
-            gv[0][(s >> lg) * RES_WAVES + wave] = w0, gv[1][(s >> lg) * RES_WAVES + wave] = w1;
+          if ((l & 63) == 0)
+            gv[0][(s >> LG) * RES_WAVES + wave] = w0, gv[1][(s >> LG) * RES_WAVES + wave] = w1;
           v[0] = v[1] = 0.;
         }
       }
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // the published rows have arrived
       __syncthreads();
       double own2[2] = {0., 0.};
-      if (t < own_nv) {
-        for (int w = 0; w < vwaves; ++w)
-          own2[0] += gv[0][t * vwaves + w], own2[1] += gv[1][t * vwaves + w];
+      if (l < own_nv) {
+        own2[0] = add_run(gv[0] + l * vwaves, vwaves), own2[1] = add_run(gv[1] + l * vwaves, vwaves);
         if (!alone) {
-          double* mine = at(P.g2 + 2 * (par * P.n_v + K.own_v), 2u * unsigned(t));
-          double* other = at(P.g2 + 2 * ((par ^ 1) * P.n_v + K.own_v), 2u * unsigned(t));
-          slot_clear(other), slot_clear(other + 1);
+          double* mine = at(P.g2 + 2 * (par * P.n_v + K.own_v), 2u * unsigned(l));
+          double* other = at(P.g2 + 2 * ((par ^ 1) * P.n_v + K.own_v), 2u * unsigned(l));
           slot_store(mine, own2[0]), slot_store(mine + 1, own2[1]);
+          slot_clear(other), slot_clear(other + 1);
+        }
+      }
+      if (!alone) {
+        double *to = P.r_pub[par] + K.row0, *old = P.r_pub[par ^ 1] + K.row0;
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+          const int o = l + s * RES_LANES;
+          if (SELL ? (pub >> s) & 1u : o < pub_lo || o >= pub_hi)
+            slot_store(at(to, unsigned(o)), r[s]), slot_clear(at(old, unsigned(o)));
+        }
+      }
+      // in the time the exchange takes: x, and the halo's rows of r (empty where their workgroup is not that far)
+      if constexpr (LEAN) {
+        double xv[S];
+#pragma unroll
+        for (int s = 0; s < S; ++s)
+          xv[s] = *at(P.x_work + K.row0, unsigned(min(l + s * RES_LANES, rows - 1)));
+#pragma unroll
+        for (int s = 0; s < S; ++s)
+          if (l + s * RES_LANES < rows)
+            *at(P.x_work + K.row0, unsigned(l + s * RES_LANES)) = fma(alpha, pt[s * RES_LANES], xv[s]);
+      } else {
+#pragma unroll
+        for (int s = 0; s < S; ++s)
+          x[s] = fma(alpha, pt[s * RES_LANES], x[s]);
+      }
+      if (!alone) {
+        const double* from = P.r_pub[par] + (SELL ? 0 : K.row0 - below);
+#pragma unroll
+        for (int k = 0; k < RES_HALO; ++k) {
+          const int e = l + k * RES_LANES;
+          if (e < nhalo)
+            halo[k] = slot_load(at(from, unsigned(SELL ? hr[k] : e < below ? e : rows + e)));
         }
       }
       if (!exchange_sum<2>(P.g2 + 2 * (par * P.n_v + K.v0), own2, alone, K.nv, P.v_block, red2, &failed, P.gave_up,
@@ -370,51 +595,88 @@ __global__ void __launch_bounds__(RES_LANES) k_pcg_resident(ResidentParams P)
     }
 #pragma unroll
     for (int s = 0; s < S; ++s) {
-      const int o = row(s);
+      const int o = t + s * RES_LANES;
       if (o < rows)
-        P.x[K.row0 + o] = x[s];
+        P.x[K.row0 + o] = LEAN ? P.x_work[K.row0 + o] : x[LEAN ? 0 : s];
     }
     if (K.rank == 0 && t == 0) {
-      PcgScalars* R = P.S + K.inst;
-      R->rz = rn[0], R->rr = rn[1], R->beta = beta, R->alpha = alpha, R->alpha_prev = alpha, R->pq = pq;
-      R->iters = begun;
-      R->done = state;
-      R->brk = 0;
+      PcgScalars* D = P.S + K.inst;
+      D->rz = rn[0], D->rr = rn[1], D->beta = beta, D->alpha = alpha, D->alpha_prev = alpha, D->pq = pq;
+      D->iters = begun;
+      D->done = state;
+      D->brk = 0;
     }
   }
 }
 
-__global__ void k_resident_clear(int64_t n, double* __restrict__ slots, int* gave_up)
+// every slot and published row empty
+__global__ void __launch_bounds__(256) k_resident_clear(ResidentParams P, int64_t slots)
 {
-  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i < n)
-    slots[i] = __longlong_as_double((long long)RES_EMPTY);
+  const double empty = __longlong_as_double((long long)RES_EMPTY);
+  const int64_t i = xcd_index(max(P.n, slots));
+  if (i < slots)
+    P.g1[i] = empty;
+  if (i < P.n)
+    P.r_pub[0][i] = empty, P.r_pub[1][i] = empty;
   if (i == 0)
-    *gave_up = 0;
+    *P.gave_up = 0;
 }
 
 using Kernel = void (*)(ResidentParams);
 
+// compiled variants: vector and operator blocks of 512 lanes with as many rows per lane as there are slots (the
+// default shapes); any vector and operator blocks with one row per lane (shapes set by the caller)
 template <int NU>
-Kernel kernel_for(int slots)
+Kernel kernel_for(int slots, int lg, bool same)
 {
-  switch (slots) {
-    case 1:
-      return k_pcg_resident<1, NU, true>;
-    case 2:
-      return k_pcg_resident<2, NU, true>;
-    case 4:
-      return k_pcg_resident<4, NU, true>;
-    case 8:
-      return k_pcg_resident<8, NU, true>;
-    default:
-      return k_pcg_resident<16, NU, false>;
-  }
+  if (same)
+    switch (slots * 16 + lg) {
+      case 16:
+        return k_pcg_resident<1, 0, true, NU, 1>;
+      case 33:
+        return k_pcg_resident<2, 1, true, NU, 1>;
+      case 66:
+        return k_pcg_resident<4, 2, true, NU, 1>;
+      case 131:
+        return k_pcg_resident<8, 3, true, NU, 1>;
+      case 259:
+        return k_pcg_resident<16, 3, true, NU, 0>;
+    }
+  if (lg == 0)
+    switch (slots) {
+      case 1:
+        return k_pcg_resident<1, 0, false, NU, 1>;
+      case 2:
+        return k_pcg_resident<2, 0, false, NU, 1>;
+      case 4:
+        return k_pcg_resident<4, 0, false, NU, 1>;
+      case 8:
+        return k_pcg_resident<8, 0, false, NU, 1>;
+    }
+  return nullptr;
 }
 
-Kernel kernel_of(int slots, int nu)
+// nu < 0: SELL, slices of at most -nu entries per row
+Kernel kernel_of(int slots, int lg, bool same, int nu)
 {
-  return nu <= 3 ? kernel_for<3>(slots) : kernel_for<4>(slots);
+  if (nu < 0) {
+    if (!same || (1 << lg) != slots)
+      return nullptr;
+    const int w = -nu;
+    switch (slots) {
+      case 1:
+        return w <= 28 ? k_pcg_resident<1, 0, true, 0, 28> : k_pcg_resident<1, 0, true, 0, 0>;
+      case 2:
+        return w <= 12 ? k_pcg_resident<2, 1, true, 0, 12> : w <= 28 ? k_pcg_resident<2, 1, true, 0, 28>
+                                                                       : k_pcg_resident<2, 1, true, 0, 0>;
+      case 4:
+        return w <= 12 ? k_pcg_resident<4, 2, true, 0, 12> : k_pcg_resident<4, 2, true, 0, 0>;
+      case 8:
+        return k_pcg_resident<8, 3, true, 0, 0>;
+    }
+    return nullptr;
+  }
+  return nu <= 3 ? kernel_for<3>(slots, lg, same) : kernel_for<4>(slots, lg, same);
 }
 
 // CUs of a device in use by resident launches of this process
@@ -453,90 +715,323 @@ int device_cus()
 
 } // namespace
 
-void resident_plan_dia(ResidentPlan& plan, const Operator& op, const std::vector<std::vector<int64_t>>& s_offs,
-                       int s_nu)
+static int64_t team_of(int64_t rows, int slots)
 {
-  plan.usable = false;
-  const SolverFormat& F = op.fmt;
-  const int ba = F.A.block, bv = F.V.block, iv = F.V.items;
-  if (s_nu < 0 || s_nu > 4 || F.A.items != 1 || ba > 1024 || (ba & (ba - 1)) != 0 || RES_LANES % bv != 0)
-    return;
-  const std::vector<int64_t>& row0 = op.space->inst_dof;
-  const int ninst = int(row0.size()) - 1;
-  const int cus = device_cus();
-  int64_t largest = 0, reach = 0;
-  std::vector<int64_t> reaches(ninst, 0);
-  for (int in = 0; in < ninst; ++in) {
-    const int64_t ni = row0[in + 1] - row0[in];
-    if (ni == 0)
-      return;
-    largest = std::max(largest, ni);
-    for (int64_t o : s_offs[in])
-      if (o < ni)
-        reaches[in] = std::max(reaches[in], o);
-    reach = std::max(reach, reaches[in]);
-  }
-  // rows per lane: the fewest with which all instances fit on the chip together
-  int slots = 0;
-  int64_t total = 0, lds = 0;
-  for (int s : {1, 2, 4, 8, 16}) {
-    if (s % iv)
-      continue;
-    const int64_t R = int64_t(s) * RES_LANES;
-    if (R % ba)
-      continue;
-    total = 0;
-    for (int in = 0; in < ninst; ++in)
-      total += (row0[in + 1] - row0[in] + R - 1) / R;
-    lds = (std::min(R, largest) + 2 * reach) * int64_t(sizeof(double));
-    if (total <= cus && lds <= RES_LDS) {
-      slots = s;
-      break;
-    }
-  }
-  if (!slots || (s_nu == 0 && slots == RES_MAX_SLOTS)) // (a diagonal matrix holds no slot to stream)
-    return;
   const int64_t R = int64_t(slots) * RES_LANES;
-  std::vector<ResidentTask> tasks;
-  std::vector<int32_t> start;
-  for (int in = 0; in < ninst; ++in) {
+  return (rows + R - 1) / R;
+}
+
+// Whether a single instance takes `slots` rows per lane (the smallest are asked first): few workgroups keep the exchanges
+// short, few rows the steps between them.  Measured (Q1, us per iteration with 1 / 2 / 4 / 8 rows per lane): 1 089 rows
+// 4.5 / 4.2 / 2.7 / 4.3 (one workgroup: no exchange); 4 096 4.2 / 3.9 / 4.3 / 4.4; 16 384 5.0 / 4.4 / 5.0 / 6.2; 65 536 6.4 / 5.3 / 5.3 / 6.7; 131 044 8.0 / 7.9 / 5.7 / 7.1;
+// 262 144 - / - / 7.8 / 7.5.  SELL: 160 401 rows of 7 entries - / 8.5 / 7.6 / 13.4, 90 201 of 11 8.6 / 8.0 / 14.8 / 23
+static bool enough_rows(int64_t rows, int slots, int cus, bool sell)
+{
+  const int64_t w = team_of(rows, slots);
+  if (sell) // (a row costs more: 9 to 20 scattered reads of LDS)
+    return slots == 1 ? w <= cus / 16 : slots <= 4 ? w <= cus / 2 : w <= cus;
+  return slots == 1 ? w <= 1 : slots == 2 ? w <= (rows <= 4 * RES_LANES ? 1 : cus / 8) : slots == 4 ? w <= cus / 4 : w <= cus;
+}
+
+// Instances of a batch in the order of their size, each on the workgroups that are free first: the estimated time until
+// the last one ends, and (order, groups) which instance is next and on which workgroups.  A workgroup takes its instances
+// in this order, so the first unfinished one always has all of its workgroups.  Negative: an instance does not fit.
+static double schedule(const std::vector<int64_t>& row0, int slots, int cus, std::vector<int>* order,
+                       std::vector<std::vector<int>>* groups)
+{
+  // us per iteration of one workgroup with 1, 2, 4, 8, 16 rows per lane (measured), and of the exchanges
+  const double step = slots == 1 ? 1.8 : slots == 2 ? 2.1 : slots == 4 ? 2.7 : slots == 8 ? 4.3 : 10.;
+  const int ninst = int(row0.size()) - 1;
+  std::vector<int> by_size(ninst);
+  for (int i = 0; i < ninst; ++i)
+    by_size[i] = i;
+  std::stable_sort(by_size.begin(), by_size.end(),
+                   [&](int a, int b) { return row0[a + 1] - row0[a] > row0[b + 1] - row0[b]; });
+  std::vector<std::pair<double, int>> load(cus); // (time it is free, workgroup)
+  for (int w = 0; w < cus; ++w)
+    load[w] = {0., w};
+  if (groups)
+    groups->assign(ninst, {});
+  double last = 0.;
+  for (int i : by_size) {
+    const int64_t n = row0[i + 1] - row0[i], team = team_of(n, slots);
+    if (team > cus)
+      return -1.;
+    std::partial_sort(load.begin(), load.begin() + team, load.end());
+    // iterations grow like the square root of the size (two dimensions)
+    const double end = load[team - 1].first + std::sqrt(double(n)) * (step + (team > 1 ? 2.6 + 0.01 * double(team) : 0.));
+    for (int64_t k = 0; k < team; ++k) {
+      load[k].first = end;
+      if (groups)
+        (*groups)[i].push_back(load[k].second);
+    }
+    last = std::max(last, end);
+  }
+  if (order)
+    *order = by_size;
+  return last;
+}
+
+// rows per lane: -1 when no choice of `fits` (LDS, compiled variant) takes all instances
+template <class F>
+static int choose_slots(const std::vector<int64_t>& row0, bool sell, F fits)
+{
+  const int cus = device_cus();
+  int best = -1;
+  double time = 0.;
+  for (int s : {1, 2, 4, 8, 16}) {
+    if (row0.size() == 2) {
+      if (enough_rows(row0[1] - row0[0], s, cus, sell) && fits(s))
+        return s;
+      continue;
+    }
+    const double t = schedule(row0, s, cus, nullptr, nullptr);
+    if (t >= 0. && (best < 0 || t < time) && fits(s))
+      best = s, time = t;
+  }
+  return best;
+}
+
+// doubles a stencil reaches to either side of a row
+static int64_t reach_of(const std::vector<int64_t>& row0, const std::vector<std::vector<int64_t>>& s_offs)
+{
+  int64_t reach = 0;
+  for (size_t in = 0; in + 1 < row0.size(); ++in)
+    for (int64_t o : s_offs[in])
+      if (o < row0[in + 1] - row0[in])
+        reach = std::max(reach, o);
+  return reach;
+}
+
+static int64_t lds_of(int slots, int64_t reach)
+{
+  return (int64_t(slots) * RES_LANES * (slots > 8 ? 2 : 1) + 2 * reach) * int64_t(sizeof(double)); // (LEAN: q)
+}
+
+int resident_items(const std::vector<int64_t>& row0, const std::vector<std::vector<int64_t>>& s_offs, int s_nu)
+{
+  if (s_nu < 0 || s_nu > 4)
+    return 0;
+  const int64_t reach = reach_of(row0, s_offs);
+  const int s = choose_slots(row0, false, [&](int k) { return lds_of(k, reach) <= RES_LDS && !(s_nu == 0 && k > 8); });
+  return s < 0 ? 0 : std::min(s, 8); // (16 rows per lane: two blocks of 8 each)
+}
+
+// one workgroup's rows after the other, instance by instance; false when the lanes that add the partials of an
+// instance of one workgroup do not hold them all
+static bool list_tasks(const Operator& op, int slots, std::vector<ResidentTask>& tasks)
+{
+  const SolverFormat& F = op.fmt;
+  const std::vector<int64_t>& row0 = op.space->inst_dof;
+  const int64_t R = int64_t(slots) * RES_LANES, va = int64_t(F.A.block) * F.A.items, vv = int64_t(F.V.block) * F.V.items;
+  for (size_t in = 0; in + 1 < row0.size(); ++in) {
     const int64_t ni = row0[in + 1] - row0[in];
     const int team = int((ni + R - 1) / R);
     for (int k = 0; k < team; ++k) {
       ResidentTask K{};
       K.row0 = row0[in] + k * R;
       K.rows = int32_t(std::min(R, ni - k * R));
-      K.inst = in, K.team = team, K.rank = k;
+      K.inst = int32_t(in), K.team = team, K.rank = k;
       K.a0 = F.A.inst_block0[in], K.na = F.A.inst_block0[in + 1] - K.a0;
       K.v0 = F.V.inst_block0[in], K.nv = F.V.inst_block0[in + 1] - K.v0;
-      K.own_a = K.a0 + int32_t(k * R / ba), K.own_v = K.v0 + int32_t(k * R / (int64_t(bv) * iv));
-      if (team == 1 && (K.na > bv || K.nv > bv)) // the lanes that add the partials do not hold them
-        return;
-      start.push_back(int32_t(tasks.size()));
+      K.own_a = K.a0 + int32_t(k * R / va), K.own_v = K.v0 + int32_t(k * R / vv);
+      K.mask = int32_t(tasks.size());
+      if (ni == 0 || (team == 1 && (K.na > F.V.block || K.nv > F.V.block)))
+        return false;
       tasks.push_back(K);
     }
   }
-  start.push_back(int32_t(tasks.size()));
-  plan.slots = slots, plan.nu = s_nu, plan.workgroups = int(start.size()) - 1, plan.lds = lds;
-  plan.tasks.upload(tasks);
+  return true;
+}
+
+// the tasks (instance by instance) in the order in which the workgroups take them
+static void finish_plan(ResidentPlan& plan, const Operator& op, const std::vector<ResidentTask>& tasks, int64_t lds)
+{
+  std::vector<int> order;
+  std::vector<std::vector<int>> groups;
+  if (schedule(op.space->inst_dof, plan.slots, device_cus(), &order, &groups) < 0.)
+    return;
+  std::vector<int64_t> first(groups.size(), 0); // first task of every instance
+  for (size_t k = tasks.size(); k-- > 0;)
+    first[tasks[k].inst] = int64_t(k);
+  std::vector<std::vector<ResidentTask>> of;
+  for (int i : order)
+    for (size_t k = 0; k < groups[i].size(); ++k) {
+      if (groups[i][k] >= int(of.size()))
+        of.resize(groups[i][k] + 1);
+      of[groups[i][k]].push_back(tasks[first[i] + int64_t(k)]);
+    }
+  std::vector<ResidentTask> list;
+  std::vector<int32_t> start{0};
+  for (auto& w : of) {
+    list.insert(list.end(), w.begin(), w.end());
+    start.push_back(int32_t(list.size()));
+  }
+  plan.workgroups = int(of.size()), plan.lds = lds;
+  plan.tasks.upload(list);
   plan.task_start.upload(start);
-  plan.exchange.allocate(size_t(2 * F.A.nblocks + 4 * F.V.nblocks));
+  plan.exchange.allocate(size_t(3 * op.fmt.A.nblocks + 4 * op.fmt.V.nblocks));
   plan.gave_up.allocate(1);
   if (!plan.host_gave_up)
     HGDT_HIP(hipHostMalloc((void**)&plan.host_gave_up, sizeof(int)));
   plan.usable = true;
 }
 
+void resident_plan_dia(ResidentPlan& plan, const Operator& op, const std::vector<std::vector<int64_t>>& s_offs,
+                       int s_nu)
+{
+  plan.usable = false;
+  const SolverFormat& F = op.fmt;
+  const int bv = F.V.block, iv = F.V.items, ba = F.A.block * F.A.items;
+  const bool same = bv == RES_LANES && F.A.block == bv && F.A.items == iv;
+  if (s_nu < 0 || s_nu > 4 || RES_LANES % bv != 0 || !(same || (F.A.items == 1 && ba <= 1024 && (ba & (ba - 1)) == 0)))
+    return;
+  const std::vector<int64_t>& row0 = op.space->inst_dof;
+  int lg = 0;
+  while ((1 << lg) < iv)
+    ++lg;
+  if (lg > 0 && bv != RES_LANES)
+    return;
+  const int64_t reach = reach_of(row0, s_offs);
+  const int slots = choose_slots(row0, false, [&](int k) {
+    // (a diagonal matrix holds no slot to stream)
+    return (int64_t(k) * RES_LANES) % ba == 0 && kernel_of(k, lg, same, s_nu) && lds_of(k, reach) <= RES_LDS &&
+           !(s_nu == 0 && k > 8);
+  });
+  if (slots < 0)
+    return;
+  std::vector<ResidentTask> tasks;
+  if (!list_tasks(op, slots, tasks))
+    return;
+  plan.sell = false;
+  plan.slots = slots, plan.lg_items = lg, plan.same_blocks = same, plan.nu = s_nu;
+  finish_plan(plan, op, tasks, lds_of(slots, reach));
+}
+
+// columns of the rows [r0, r1) that lie outside them, ascending
+static void halo_of(const Operator& op, int64_t r0, int64_t r1, std::vector<int32_t>& halo)
+{
+  halo.clear();
+  for (int64_t k = op.row_ptr[r0]; k < op.row_ptr[r1]; ++k)
+    if (op.cols[k] < r0 || op.cols[k] >= r1)
+      halo.push_back(op.cols[k]);
+  std::sort(halo.begin(), halo.end());
+  halo.erase(std::unique(halo.begin(), halo.end()), halo.end());
+}
+
+int resident_items_sell(const Operator& op)
+{
+  const std::vector<int64_t>& row0 = op.space->inst_dof;
+  const int s = choose_slots(row0, true, [&](int k) {
+    if (k > 8)
+      return false;
+    // p of the own rows and the halo in LDS
+    const int64_t R = int64_t(k) * RES_LANES;
+    std::vector<int64_t> first;
+    for (size_t in = 0; in + 1 < row0.size(); ++in)
+      for (int64_t r = row0[in]; r < row0[in + 1]; r += R)
+        first.push_back(r);
+    first.push_back(row0.back());
+    std::atomic<int64_t> most{0};
+    parallel_for(int64_t(first.size()) - 1, [&](int64_t b0, int64_t b1) {
+      std::vector<int32_t> halo;
+      for (int64_t b = b0; b < b1; ++b) {
+        halo_of(op, first[b], first[b + 1], halo);
+        int64_t m = most;
+        while (m < int64_t(halo.size()) && !most.compare_exchange_weak(m, int64_t(halo.size())))
+          ;
+      }
+    });
+    return (R + most) * int64_t(sizeof(double)) <= RES_LDS;
+  });
+  return std::max(s, 0);
+}
+
+void resident_plan_sell(ResidentPlan& plan, const Operator& op)
+{
+  plan.usable = false;
+  const SolverFormat& F = op.fmt;
+  const int slots = F.V.items;
+  if (F.V.block != RES_LANES || F.A.block != RES_LANES || F.A.items != slots || slots > RES_MAX_SLOTS)
+    return;
+  int lg = 0;
+  while ((1 << lg) < slots)
+    ++lg;
+  if (!kernel_of(slots, lg, true, -1))
+    return;
+  std::vector<ResidentTask> tasks;
+  if (!list_tasks(op, slots, tasks))
+    return;
+  const int64_t R = int64_t(slots) * RES_LANES, nt = int64_t(tasks.size());
+  std::vector<std::vector<int32_t>> halo(nt);
+  parallel_for(nt, [&](int64_t b0, int64_t b1) {
+    for (int64_t b = b0; b < b1; ++b)
+      halo_of(op, tasks[b].row0, tasks[b].row0 + tasks[b].rows, halo[b]);
+  });
+  // the rows that other workgroups read
+  std::vector<uint8_t> read(std::max<int64_t>(op.n, 1), 0);
+  std::vector<int32_t> rows;
+  int64_t most = 0, slices = 0;
+  for (int64_t b = 0; b < nt; ++b) {
+    tasks[b].halo0 = int32_t(rows.size()), tasks[b].nhalo = int32_t(halo[b].size());
+    tasks[b].slice0 = int32_t(slices);
+    slices += (tasks[b].rows + 63) / 64;
+    most = std::max<int64_t>(most, tasks[b].nhalo);
+    for (int32_t c : halo[b])
+      read[c] = 1;
+    rows.insert(rows.end(), halo[b].begin(), halo[b].end());
+  }
+  if (slices != F.nslices || (R + most) * int64_t(sizeof(double)) > RES_LDS)
+    return;
+  std::vector<uint32_t> pub(nt * RES_LANES, 0u);
+  std::vector<uint16_t> local(std::max<size_t>(F.d_sell_vals.count, 1), 0);
+  std::vector<int64_t> slice_ptr(F.nslices + 1);
+  F.d_slice_ptr.download(slice_ptr.data());
+  parallel_for(nt, [&](int64_t b0, int64_t b1) {
+    for (int64_t b = b0; b < b1; ++b) {
+      const ResidentTask& K = tasks[b];
+      const std::vector<int32_t>& h = halo[b];
+      for (int o = 0; o < K.rows; ++o) {
+        const int64_t i = K.row0 + o;
+        if (read[i])
+          pub[b * RES_LANES + o % RES_LANES] |= 1u << (o / RES_LANES);
+        const int64_t sl = K.slice0 + o / 64;
+        const int64_t w = (slice_ptr[sl + 1] - slice_ptr[sl]) / 64, len = op.row_ptr[i + 1] - op.row_ptr[i];
+        for (int64_t k = 0; k < w; ++k) {
+          int64_t at = o; // padding: the own row, as the columns of the storage
+          if (k < len) {
+            const int32_t c = op.cols[op.row_ptr[i] + k];
+            at = (c >= K.row0 && c < K.row0 + K.rows) ? c - K.row0
+                                                      : R + (std::lower_bound(h.begin(), h.end(), c) - h.begin());
+          }
+          local[slice_ptr[sl] + k * 64 + o % 64] = uint16_t(at);
+        }
+      }
+    }
+  });
+  plan.sell_local.upload(local);
+  if (rows.empty())
+    rows.push_back(0);
+  plan.halo_rows.upload(rows);
+  plan.publish.upload(pub);
+  plan.sell = true;
+  int64_t widest = 1;
+  for (int64_t k = 0; k < F.nslices; ++k)
+    widest = std::max(widest, (slice_ptr[k + 1] - slice_ptr[k]) / 64);
+  plan.slots = slots, plan.lg_items = lg, plan.same_blocks = true, plan.nu = -int(std::min<int64_t>(widest, 1 << 20));
+  finish_plan(plan, op, tasks, (R + most) * int64_t(sizeof(double)));
+}
+
 bool resident_run(ResidentPlan& plan, ResidentParams P, hipStream_t stream, PcgScalars* host_records)
 {
   P.g1 = plan.exchange.ptr;
-  P.g2 = plan.exchange.ptr + 2 * P.n_a;
+  P.g2 = plan.exchange.ptr + 3 * P.n_a;
+  P.sell_local = plan.sell_local.ptr, P.halo_rows = plan.halo_rows.ptr, P.publish = plan.publish.ptr;
   P.tasks = plan.tasks.ptr, P.task_start = plan.task_start.ptr, P.gave_up = plan.gave_up.ptr;
   P.wait_ticks = int64_t(4) * 100000000; // 4 s
   const int64_t nx = int64_t(plan.exchange.count);
-  hipLaunchKernelGGL(k_resident_clear, dim3(unsigned((nx + 255) / 256)), dim3(256), 0, stream, nx, plan.exchange.ptr,
-                     plan.gave_up.ptr);
-  const Kernel k = kernel_of(plan.slots, plan.nu);
+  hipLaunchKernelGGL(k_resident_clear, dim3(xcd_grid(std::max(P.n, nx), 256)), dim3(256), 0, stream, P, nx);
+  const Kernel k = kernel_of(plan.slots, plan.lg_items, P.same_blocks, plan.nu);
   HGDT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
                                int(RES_LDS)));
   int dev = 0;

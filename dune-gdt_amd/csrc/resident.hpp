@@ -16,26 +16,35 @@ struct ResidentTask {
   int32_t a0, na;        // first block of the instance and their number, operator partition
   int32_t v0, nv;        // the same, vector partition
   int32_t own_a, own_v;  // first own block of either partition
+  // SELL: first own slice, and the rows of other workgroups that the own rows meet (entries of halo_rows)
+  int32_t slice0, halo0, nhalo;
+  int32_t mask; // its block of `publish`
 };
 
 struct ResidentParams {
   int64_t n;
   int ninst;
   const int64_t* inst_row0;
-  // launch shapes whose block partials (and therefore bits) the solve reproduces: operator blocks of a_block
-  // rows, vector blocks of v_block lanes and 1 << v_lg_items rows per lane
-  int a_block, v_block, v_lg_items;
+  // launch shapes whose block partials (and therefore bits) the solve reproduces: vector blocks of v_block lanes and
+  // 1 << v_lg_items rows per lane, operator blocks the same or of a_rows lanes with one row each
+  int a_rows, v_block, same_blocks;
   // scaled symmetric DIA: strict upper slots
   int s_nu;
   const int64_t* s_off;
   const double* scaled;
+  // scaled SELL-64 values in `scaled`; per entry its position in the workgroup's p (own rows, then its halo)
+  const int64_t* slice_ptr;
+  const uint16_t* sell_local;
+  const int32_t* halo_rows;
+  const uint32_t* publish; // per workgroup and lane: the slots whose rows other workgroups read
   const double* dsq;
   const double* r;     // r of the initial residual (not written: a solve that gives up leaves it to the caller)
   double* x;           // scaled iterate: read at the start, written by the instances that end
-  double* r_pub;       // rows of r that other workgroups of the team read
+  double* x_work;      // the iterate of workgroups that do not hold it in registers
+  double* r_pub[2];    // rows of r that other workgroups of the team read, by parity of the step
   const double* part2; // partials of the initial residual, 2 per vector block
-  double* g1;          // 2 x (operator blocks): partials of p.q, by parity of the step
-  double* g2;          // 2 x 2 x (vector blocks): partials of the two residual norms
+  double* g1;          // 3 x (operator blocks): partials of p.q, by step
+  double* g2;          // behind it, 2 x 2 x (vector blocks): partials of the two residual norms, by parity
   int64_t n_a, n_v;    // operator / vector blocks of all instances
   PcgScalars* S;       // record of every instance: tolerance read, result written
   int64_t max_iter;
@@ -50,9 +59,15 @@ struct ResidentPlan {
   int64_t version = -1; // SolverCache::version the plan was made for
   bool usable = false;
   int slots = 0;        // rows per lane
+  int lg_items = 0;     // log2 of the vector blocks' rows per lane
+  bool same_blocks = false; // operator blocks = vector blocks
   int nu = 0;           // strict upper slots the kernel is compiled for
   int workgroups = 0;
   int64_t lds = 0;
+  bool sell = false;
+  DeviceArray<uint16_t> sell_local;
+  DeviceArray<int32_t> halo_rows;
+  DeviceArray<uint32_t> publish;
   DeviceArray<ResidentTask> tasks;
   DeviceArray<int32_t> task_start;
   DeviceArray<double> exchange; // g1, g2
@@ -65,9 +80,16 @@ struct ResidentPlan {
   }
 };
 
+constexpr int RES_BLOCK = 512; // lanes of a workgroup, and of the row blocks that suit it
+// rows per lane of row blocks for a solve in one launch of symmetric DIA storage with these strict upper offsets;
+// 0: it does not fit on the chip
+int resident_items(const std::vector<int64_t>& inst_row0, const std::vector<std::vector<int64_t>>& s_offs, int s_nu);
 // s_offs: the strict upper offsets of every instance's scaled matrix
 void resident_plan_dia(ResidentPlan& plan, const Operator& op, const std::vector<std::vector<int64_t>>& s_offs,
                        int s_nu);
+// the same for SELL storage (general meshes): rows per lane, and the plan
+int resident_items_sell(const Operator& op);
+void resident_plan_sell(ResidentPlan& plan, const Operator& op);
 // runs the solve; false when it gave up (then nothing but r_pub and the exchange buffers was written for the
 // instances without a result: the caller goes on with one launch per kernel).  Waits for the kernel.
 bool resident_run(ResidentPlan& plan, ResidentParams P, hipStream_t stream, PcgScalars* host_records);

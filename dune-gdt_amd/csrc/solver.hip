@@ -306,25 +306,23 @@ __device__ __forceinline__ void apply_rows(const PcgParams& P, const double* __r
   }
 }
 
-template <int FMT, int ITEMS>
-__global__ void __launch_bounds__(1024) k_apply(PcgParams P, const double* __restrict__ x, double* __restrict__ y)
+// y = A x, one row per lane: a row block of `items` rows per lane is handled by `items` workgroups
+template <int FMT>
+__global__ void __launch_bounds__(1024) k_apply(PcgParams P, int items, const double* __restrict__ x, double* __restrict__ y)
 {
-  const int b = logical_block(P.a_nb);
-  if (b < 0)
+  const int w = logical_block(P.a_nb * items);
+  if (w < 0)
     return;
+  const int b = w / items;
   const int inst = P.a_inst[b];
-  const int64_t rb = P.a_row0[b], r1 = P.a_row0[b + 1];
+  const int64_t rb = P.a_row0[b], r1 = P.a_row0[b + 1], r0 = rb + int64_t(w - b * items) * blockDim.x;
+  if (r0 >= r1)
+    return;
   const double* vals = (FMT == FMT_SELL) ? P.sell_vals : P.dia;
-  for (int64_t r0 = rb; r0 < r1; r0 += int64_t(blockDim.x) * ITEMS) {
-    double acc[ITEMS];
-    apply_rows<FMT, ITEMS, false>(P, vals, b, inst, rb, r0, r1, [&](int64_t c) { return x[c]; }, acc);
-#pragma unroll
-    for (int j = 0; j < ITEMS; ++j) {
-      const int64_t i = r0 + threadIdx.x + int64_t(j) * blockDim.x;
-      if (i < r1)
-        y[i] = acc[j];
-    }
-  }
+  double acc[1];
+  apply_rows<FMT, 1, false>(P, vals, b, inst, rb, r0, r1, [&](int64_t c) { return x[c]; }, acc);
+  if (r0 + threadIdx.x < r1)
+    y[r0 + threadIdx.x] = acc[0];
 }
 
 // 4 x 4 element blocks: y = A x over the 4 rows of element E (lane per element).  Each row sums its
@@ -1384,6 +1382,8 @@ struct SolverCache {
   int64_t graph_version = -1;
   int64_t version = 0;
   ResidentPlan resident;
+  int shaped_for = 0; // resident_shape of the row partitions
+  int sell_items = 0; // SELL: rows per lane that suit a solve in one launch (0: none)
   ~SolverCache()
   {
     for (auto& h : host_scalars)
@@ -1471,6 +1471,22 @@ void RowPartition::build_counts(const std::vector<int64_t>& inst_dof, const std:
 }
 
 static bool blk_wanted(const Operator& op);
+static int kernel_format(const Operator& op);
+
+// rows per lane of the row blocks that suit a solve in one launch (resident.hip: blocks of RES_BLOCK lanes, the
+// operator's and the vector kernels' alike); 0: the caller chose shapes, or the storage (once it is known) or size
+// does not fit
+static int resident_shape(const Operator& op)
+{
+  const SolverCache& C = *op.solver_cache;
+  if (op.launch[3].user || op.launch[4].user || !op.square())
+    return 0;
+  if (op.fmt.format == HGDT_FORMAT_SELL && op.fmt.structure_ready)
+    return C.sell_items;
+  if (!op.fmt.valid || op.fmt.format != HGDT_FORMAT_DIA || kernel_format(op) != FMT_DIAS)
+    return 0;
+  return resident_items(op.space->inst_dof, C.s_offs, C.s_nu);
+}
 
 // row-block partitions of the operator (host set-up, O(number of blocks))
 static void build_partitions(Operator& op)
@@ -1483,6 +1499,9 @@ static void build_partitions(Operator& op)
   // instance's partials stays small
   if (!op.launch[3].user)
     op.launch[3].block = 256, op.launch[3].items = 1;
+  const int resident = resident_shape(op); // rows per lane of a solve in one launch
+  if (resident)
+    op.launch[3].block = RES_BLOCK, op.launch[3].items = resident;
   // the matrix-free kernels give every lane one row (continuous spaces, at most 256 lanes per block) or one
   // element of a tile of elements (discontinuous spaces: 256 lanes, 4 rows each)
   const bool mf = op.requested_format == HGDT_FORMAT_MATRIX_FREE;
@@ -1495,7 +1514,10 @@ static void build_partitions(Operator& op)
     op.launch[4].block = 256;
     const int64_t want = (op.n + 256 * 1024 - 1) / (256 * 1024);
     op.launch[4].items = want <= 1 ? 1 : want <= 2 ? 2 : want <= 4 ? 4 : 8;
+    if (resident)
+      op.launch[4].block = RES_BLOCK, op.launch[4].items = resident;
   }
+  C.shaped_for = resident;
   const std::vector<int64_t> tiles = mf_tiles ? mf_tile_counts(op) : std::vector<int64_t>{};
   if (!tiles.empty())
     F.A.build_counts(s.inst_dof, tiles, block3, items3);
@@ -1888,6 +1910,10 @@ static void build_structure(Operator& op)
     F.d_dia.allocate(std::max<int64_t>(int64_t(nd) * op.n, 1));
   } else {
     F.format = HGDT_FORMAT_SELL;
+    C.sell_items = op.square() ? resident_items_sell(op) : 0;
+    F.structure_ready = true;
+    if (resident_shape(op) != C.shaped_for)
+      build_partitions(op); // (the slices follow the row blocks)
     std::vector<int64_t> slice_ptr{0}, bslice0;
     for (int64_t b = 0; b < F.A.nblocks; ++b) {
       bslice0.push_back(int64_t(slice_ptr.size()) - 1);
@@ -2134,6 +2160,8 @@ void Operator::materialize_values(hipStream_t stream)
 void Operator::prepare_solver(hipStream_t stream)
 {
   prepare_storage(stream);
+  if (resident_shape(*this) != cache_of(*this).shaped_for) // default shapes follow the storage
+    build_partitions(*this);
   // column windows for the current row blocks, on the device once the staged application is chosen
   // (set-up, never captured)
   SolverCache& C = cache_of(*this);
@@ -2283,7 +2311,7 @@ void Operator::apply(const double* x, double* y, hipStream_t stream)
   }
   PcgParams P = make_params(*this);
   const int block = fmt.A.block;
-  const unsigned grid = hw_blocks(fmt.A.nblocks);
+  const unsigned grid = hw_blocks(fmt.A.nblocks * fmt.A.items);
   const int kf = kernel_format(*this);
   if (kf == FMT_BLK) {
     const unsigned g1 = xcd_grid(fmt.blk_ne, 256);
@@ -2294,15 +2322,12 @@ void Operator::apply(const double* x, double* y, hipStream_t stream)
     HGDT_HIP(hipGetLastError());
     return;
   }
-  dispatch_items(apply_lane_rows(fmt.A.items), [&](auto IT) {
-    constexpr int I = decltype(IT)::value;
-    if (kf == FMT_DIA)
-      hipLaunchKernelGGL((k_apply<FMT_DIA, I>), dim3(grid), dim3(block), 0, stream, P, x, y);
-    else if (kf == FMT_DIAS)
-      hipLaunchKernelGGL((k_apply<FMT_DIAS, I>), dim3(grid), dim3(block), 0, stream, P, x, y);
-    else
-      hipLaunchKernelGGL((k_apply<FMT_SELL, I>), dim3(grid), dim3(block), 0, stream, P, x, y);
-  });
+  if (kf == FMT_DIA)
+    hipLaunchKernelGGL(k_apply<FMT_DIA>, dim3(grid), dim3(block), 0, stream, P, fmt.A.items, x, y);
+  else if (kf == FMT_DIAS)
+    hipLaunchKernelGGL(k_apply<FMT_DIAS>, dim3(grid), dim3(block), 0, stream, P, fmt.A.items, x, y);
+  else
+    hipLaunchKernelGGL(k_apply<FMT_SELL>, dim3(grid), dim3(block), 0, stream, P, fmt.A.items, x, y);
   HGDT_HIP(hipGetLastError());
 }
 
@@ -2393,6 +2418,8 @@ static ResidentPlan& resident_plan(Operator& op)
     plan.usable = false;
     if (kernel_format(op) == FMT_DIAS && op.fmt.format == HGDT_FORMAT_DIA)
       resident_plan_dia(plan, op, C.s_offs, C.s_nu);
+    else if (op.fmt.format == HGDT_FORMAT_SELL)
+      resident_plan_sell(plan, op);
     plan.version = C.version;
   }
   return plan;
@@ -2404,11 +2431,10 @@ static bool resident_solve(Operator& op, const PcgParams& P, hipStream_t stream)
   SolverCache& C = cache_of(op);
   ResidentParams R{};
   R.n = op.n, R.ninst = P.ninst, R.inst_row0 = P.inst_row0;
-  R.a_block = F.A.block, R.v_block = F.V.block;
-  while ((1 << R.v_lg_items) < F.V.items)
-    ++R.v_lg_items;
-  R.s_nu = P.s_nu, R.s_off = P.s_off, R.scaled = P.scaled, R.dsq = P.dsq;
-  R.r = P.r, R.x = P.x, R.r_pub = P.p, R.part2 = P.part2;
+  R.a_rows = F.A.block * F.A.items, R.v_block = F.V.block;
+  R.same_blocks = C.resident.same_blocks;
+  R.s_nu = P.s_nu, R.s_off = P.s_off, R.scaled = P.scaled, R.dsq = P.dsq, R.slice_ptr = P.slice_ptr;
+  R.r = P.r, R.x = P.x, R.x_work = P.q, R.r_pub[0] = P.p, R.r_pub[1] = P.p2, R.part2 = P.part2;
   R.n_a = F.A.nblocks, R.n_v = F.V.nblocks;
   R.S = P.S, R.max_iter = P.max_iter;
   return resident_run(C.resident, R, stream, C.host_scalars[0]);
