@@ -10,8 +10,8 @@
 // Exchange: every block partial has a slot in global memory that holds a sentinel until its workgroup has
 // stored it; every workgroup of the instance reads all slots, again until none holds the sentinel, and adds
 // them in block order.  So the values are their own flags: one store and one load between the slowest
-// workgroup and all others (2.4-3.5 us with 256 workgroups, 1-1.3 us with 16).  The sets of slots rotate,
-// three for p.q and two for the norms: a workgroup empties its slots of the set that comes up next but one (norms:
+// workgroup and all others (2.4-3.5 us with 256 workgroups, 1-1.3 us with 16).  The sets of slots
+// rotate, three for p.q and two for the norms: a workgroup empties its slots of the set that comes up next but one (norms:
 // next) when it stores to one.  By then every workgroup has read what they held (it has stored to an exchange since),
 // and none polls them again before this workgroup has stored to the p.q exchange in between, which it does after
 // waiting for its earlier stores (vmcnt 0).  The rows of r that other workgroups read go the same way, through two
@@ -22,11 +22,13 @@
 // the operator's and the vector partition, sums over the partials), so a solve gives the same bits on either path,
 // alone or in a batch.
 //
-// Measured (us per iteration, three kernels -> one launch, before and after the default row blocks became those of a
-// workgroup's lanes): Q1 128^2 14 -> 4.5, 701x523 18 -> 8.6, 1023^2 33 -> 10.7, P1 48^3 x 6 19 -> 7.3, eight of these in a
-// batch 33 -> 9.4; SELL: P1 triangles of a mesh with 160 401 vertices 18 -> 7.5, P2 triangles with 90 201 DoFs 18 -> 8.2.
-// What is left of an iteration: two exchanges of 1-2.5 us, the barriers and sums around them, and for 4096 rows per
-// workgroup LDS (13 reads of 8 bytes per row at 128 B per clock: 1.4 us).
+// Measured (us per iteration, three kernels -> one launch): Q1 32^2 15 -> 2.7, 128^2 14 -> 4.5, 701x523 18 -> 7.8, 1023^2
+// 33 -> 11.8, P1 48^3 x 6 18 -> 7.0, eight of these in a batch 33 -> 9.4, 100^3 x 6 34 -> 19, 128^3 x 6 54 -> 27; SELL: P1
+// triangles of a mesh with 160 401 vertices 18 -> 7.0, P2 triangles with 90 201 DoFs 18 -> 7.5.
+// What bounds an iteration now: small problems two exchanges of 1-2.5 us, the barriers and sums around them; 4096 rows
+// per workgroup LDS (13 reads of 8 bytes per row at 128 B per clock: 1.4 us) and registers (a variant that spilled 46 took
+// 19 us instead of 11.8 at 1023^2: the scratch of 256 workgroups evicts L2); 128^3 x 6 the published p (17 MB of
+// write-through stores at about 2.5 TB/s) and the matrix (68 MB read past L2).
 //
 // All workgroups of a team must be on the chip together: the host launches at most one per CU and counts the
 // CUs of all running launches of the process.  A wait that outlasts its limit (another process holds the
@@ -46,11 +48,16 @@
 namespace hgdt {
 namespace {
 
-constexpr int RES_LANES = RES_BLOCK, RES_WAVES = RES_LANES / 64;
+constexpr int RES_LANES = RES_BLOCK;  // lanes of a workgroup (FAR: RES_FAR_BLOCK)
 constexpr int RES_MAX_SLOTS = 16;
-constexpr int RES_HALO = 3; // halo rows a lane asks for while the residual norms are exchanged
-constexpr int RES_GROUPS = RES_WAVES * RES_MAX_SLOTS; // 64-row groups of a workgroup
+constexpr int RES_HALO = 4; // halo rows a lane asks for while the residual norms are exchanged
+constexpr int RES_WAVES = 12;              // of a workgroup, at most
+constexpr int RES_GROUPS = 144;            // 64-row groups of a workgroup, at most
+constexpr int RES_MAX_GROUPS = 1024;                  // workgroups of an instance, at most (flags)
 constexpr int64_t RES_LDS = 150 * 1024;               // dynamic LDS of a workgroup, of 160 KB
+
+// doubles from one workgroup block's slot to the next: packed slots share lines that all poll while they are written
+constexpr int RES_PAD = 2;
 
 // sentinel of the exchange slots: a NaN no sum produces (a NaN sum is stored as the default NaN)
 constexpr unsigned long long RES_EMPTY = 0x7ff8dead00000001ull;
@@ -108,7 +115,7 @@ __device__ __forceinline__ T* at(T* base, unsigned i)
 // t + block, ...; then the waves' butterflies; then the waves in order), in every lane.  Partials come from the
 // exchange slots, or (one workgroup, at most `block` partials: own) from the lane that computed them.  false:
 // gave up.  One barrier; red is not written again before a later barrier.
-template <int NV>
+template <int NV, int NW>
 __device__ __forceinline__ bool exchange_sum(const double* slots, const double (&own)[NV], bool alone, int count,
                                              int block, double (*red)[RES_WAVES], int* failed, int* gave_up,
                                              int64_t ticks, double (&tot)[NV])
@@ -130,7 +137,7 @@ __device__ __forceinline__ bool exchange_sum(const double* slots, const double (
         bool empty = false;
 #pragma unroll
         for (int k = 0; k < NV; ++k)
-          u[k] = slot_load(at(slots, unsigned(b) * NV + k));
+          u[k] = slot_load(at(slots, unsigned(b) * RES_PAD + k));
 #pragma unroll
         for (int k = 0; k < NV; ++k)
           empty = empty || u[k] == RES_EMPTY;
@@ -161,11 +168,16 @@ __device__ __forceinline__ bool exchange_sum(const double* slots, const double (
   for (int k = 0; k < NV; ++k) {
     double s = 0.;
 #pragma unroll
-    for (int w = 0; w < RES_WAVES; ++w)
+    for (int w = 0; w < NW; ++w)
       s += red[k][w];
     tot[k] = s;
   }
   return true;
+}
+
+constexpr bool q_in_lds(int slots, int nu, bool far)
+{
+  return far || slots > 8 || (slots == 8 && nu == 4);
 }
 
 // g consecutive LDS values added in order (g a power of two up to 16), four loads at a time
@@ -183,24 +195,28 @@ __device__ __forceinline__ double add_run(const double* v, int g)
   return s;
 }
 
-// PCG of the tasks of one workgroup, one after the other.  Lane t holds rows t, t + RES_LANES, ... of the workgroup,
-// one per slot.  Vector blocks have 1 << LG rows per lane: RES_LANES lanes, or (LG = 0) any number that divides it.  So
+// PCG of the tasks of one workgroup, one after the other.  Lane t holds rows t, t + T, ... of the workgroup,
+// one per slot.  Vector blocks have 1 << LG rows per lane: T lanes, or (LG = 0) any number that divides it.  So
 // a slot's rows are a constant away from slot 0's and LDS is read at constant offsets.  Rows past the end of the instance
 // hold zeros and take part like others.  NU: strict upper slots compiled for (missing ones have zero values).
 // KEEP != 0: the matrix rows stay in registers, else they are read every iteration.
 // SAME: the operator blocks are the vector blocks; else they have one row per lane (64-row sums combined by threads).
 // NU = 0: SELL-64 storage; p of the own rows is followed by the halo, a list of rows, and the entries hold positions
 // in that; KEEP: entries of a row that registers hold (at least the widest slice's).
-template <int S, int LG, bool SAME, int NU, int KEEP>
-__global__ void __launch_bounds__(RES_LANES) k_pcg_resident(ResidentParams P)
+// FAR: the outermost of the NU offsets reaches further than LDS does (planes of a 3-d lattice): its columns, and the
+// halo, are read as p from the other workgroups in every step.
+template <int T, int S, int LG, bool SAME, int NU, int KEEP, bool FAR = false>
+__global__ void __launch_bounds__(T) k_pcg_resident(ResidentParams P)
 {
   extern __shared__ double pl[]; // p of the own rows and `reach` rows to either side (0 outside the instance)
   __shared__ double ga[RES_GROUPS], gv[2][RES_GROUPS];
   __shared__ double red1[1][RES_WAVES], red2[2][RES_WAVES];
   __shared__ int failed;
-  constexpr int ITEMS = 1 << LG, R = S * RES_LANES;
+  constexpr int NW = T / 64, ITEMS = 1 << LG, R = S * T;
   constexpr bool SELL = NU == 0;
-  constexpr bool LEAN = S > 8; // registers hold r only: q lies in LDS, x and D^{1/2} are read (x written) in every step
+  // what registers do not hold: q (in LDS), D^{1/2} (read in every step), x (read and written in every step)
+  constexpr bool QLDS = q_in_lds(S, NU, FAR), SQMEM = FAR || S > 8 || (S == 8 && !SELL), XMEM = S > 12;
+  constexpr int NN = FAR ? NU - 1 : NU; // upper slots whose columns lie in LDS
   constexpr int MU = SELL ? 1 : NU;
   const int t = threadIdx.x, wave = t >> 6;
   const int vwaves = P.v_block >> 6;
@@ -221,7 +237,8 @@ __global__ void __launch_bounds__(RES_LANES) k_pcg_resident(ResidentParams P)
     for (int u = 0; u < NU; ++u) {
       const int64_t o = u < ku ? so[u] : 0; // padding slots: values 0, offset 0
       off[u] = o < hi - lo ? int(o) : 0;
-      reach = max(reach, off[u]);
+      if (u < NN)
+        reach = max(reach, off[u]);
     }
     const int below = int(min(K.row0 - lo, int64_t(reach)));        // rows of the instance below the own ones
     const int above = int(min(hi - K.row0 - rows, int64_t(reach))); // and above, at most `reach`
@@ -230,41 +247,40 @@ __global__ void __launch_bounds__(RES_LANES) k_pcg_resident(ResidentParams P)
     const int32_t* const hrow = P.halo_rows + (SELL ? K.halo0 : 0);
     auto halo_row = [&](int e) { return SELL ? int64_t(hrow[e]) : K.row0 - below + (e < below ? e : rows + e); };
     auto halo_place = [&](int e) { return SELL ? R + e : reach - below + (e < below ? e : rows + e); };
-    double r[S], x[LEAN ? 1 : S], sq[LEAN ? 1 : S];
+    double r[S], x[XMEM ? 1 : S], sq[SQMEM ? 1 : S];
     double au[!SELL && KEEP ? S : 1][MU], al[!SELL && KEEP ? S : 1][MU];
     constexpr int KW = SELL && KEEP ? KEEP : 2; // (even)
     double mv[SELL && KEEP ? S : 1][KW];
     uint32_t mi[SELL && KEEP ? S : 1][KW / 2];
     int width[SELL ? S : 1];
     __syncthreads(); // the previous task's last reads of LDS
-    for (int e = t; e < R + 2 * reach; e += RES_LANES) {
+    for (int e = t; e < R + 2 * reach; e += T) {
       const int o = e - reach;
       pl[e] = (o >= -below && o < rows + above) ? P.r[K.row0 + o] : 0.;
     }
     if constexpr (SELL)
-      for (int e = t; e < nhalo; e += RES_LANES)
+      for (int e = t; e < nhalo; e += T)
         pl[R + e] = P.r[halo_row(e)];
 #pragma unroll
     for (int s = 0; s < S; ++s) {
-      const int o = t + s * RES_LANES;
+      const int o = t + s * T;
       const int64_t i = K.row0 + o;
       const bool in = o < rows;
       r[s] = in ? P.r[i] : 0.;
-      if constexpr (LEAN) {
-        if (in)
-          P.x_work[i] = P.x[i];
-      } else {
-        x[s] = in ? P.x[i] : 0.;
+      if constexpr (!SQMEM)
         sq[s] = in ? P.dsq[i] : 0.;
-      }
+      if constexpr (!XMEM)
+        x[s] = in ? P.x[i] : 0.;
+      else if (in)
+        P.x_work[i] = P.x[i];
       if constexpr (SELL) {
         width[s] = 0;
         if constexpr (KEEP != 0)
 #pragma unroll
           for (int k = 0; k < KW; ++k)
             mv[s][k] = 0., mi[s][k / 2] = 0u;
-        if (uniform((s * RES_WAVES + wave) * 64) < rows) {
-          const int64_t* sp = P.slice_ptr + K.slice0 + s * RES_WAVES + uniform(wave);
+        if (uniform((s * NW + wave) * 64) < rows) {
+          const int64_t* sp = P.slice_ptr + K.slice0 + s * NW + uniform(wave);
           const int64_t first = sp[0];
           width[s] = int((sp[1] - first) >> 6);
           if constexpr (KEEP != 0)
@@ -285,11 +301,17 @@ __global__ void __launch_bounds__(RES_LANES) k_pcg_resident(ResidentParams P)
         }
     }
     const double tol2 = P.S[K.inst].tol2;
+    const bool whole = rows == R;
+    // FAR: workgroups that hold columns of the own rows
+    const int64_t far_reach = FAR ? int64_t(off[NU - 1 > 0 ? NU - 1 : 0]) : 0;
+    const int far_first = FAR ? int((max(K.row0 - far_reach, lo) - lo) / R) : 0;
+    const int far_last = FAR ? int((min(K.row0 + rows + far_reach, hi) - 1 - lo) / R) : 0;
+    const bool single = alone && K.na == 1 && K.nv == 1; // one partial: the sum itself, in every lane
     const int own_na = (rows + P.a_rows - 1) / P.a_rows;
     const int own_nv = (rows + P.v_block * ITEMS - 1) / (P.v_block * ITEMS);
     // own rows [0, pub_lo) and [pub_hi, ...) are read by other workgroups of the team
     // (SELL: the slots in `pub`)
-    const uint32_t pub = SELL ? P.publish[int64_t(K.mask) * RES_LANES + t] : 0u;
+    const uint32_t pub = SELL ? P.publish[int64_t(K.mask) * T + t] : 0u;
     const int pub_lo = K.rank > 0 ? min(reach, rows) : 0, pub_hi = K.rank + 1 < K.team ? rows - reach : R;
     double rn[2], rho_prev = 0., beta = 0.;
     {
@@ -309,19 +331,19 @@ __global__ void __launch_bounds__(RES_LANES) k_pcg_resident(ResidentParams P)
       for (int k = 0; k < 2; ++k) {
         rn[k] = 0.;
 #pragma unroll
-        for (int w = 0; w < RES_WAVES; ++w)
+        for (int w = 0; w < NW; ++w)
           rn[k] += red2[k][w];
       }
     }
     int it = 0, begun = 0;
     int state = 0;
     double alpha = 0., pq = 0.;
-    unsigned long long halo[RES_HALO]; // rows of r of the halo, entries t, t + RES_LANES, ...
+    unsigned long long halo[RES_HALO]; // rows of r of the halo, entries t, t + T, ...
     int hr[RES_HALO];                  // SELL: which rows these are
     if constexpr (SELL)
 #pragma unroll
       for (int k = 0; k < RES_HALO; ++k)
-        hr[k] = t + k * RES_LANES < nhalo ? hrow[t + k * RES_LANES] : 0;
+        hr[k] = t + k * T < nhalo ? hrow[t + k * T] : 0;
     const int max_iter = int(min(P.max_iter, int64_t(0x7ffffff0)));
     for (;; ++it) {
       // the lane, opaque in every step: the addresses made from it are not kept in registers across steps
@@ -334,20 +356,50 @@ __global__ void __launch_bounds__(RES_LANES) k_pcg_resident(ResidentParams P)
       if (state)
         break;
       double* const pt = pl + reach + l; // p of the lane's row in slot 0
-      if (it > 0) {
+      if (it > 0)
         beta = rho / rho_prev;
+      if constexpr (FAR) {
+        // p itself goes to the other workgroups: the rows, then (all have arrived) the step's number as this workgroup's
+        // flag; the first wave waits for the flags of the workgroups within reach and fetches the halo
+        double* const to = P.r_pub[0] + K.row0;
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+          const double p = it > 0 ? fma(beta, pt[s * T], r[s]) : r[s];
+          pt[s * T] = p;
+          if (l + s * T < rows)
+            __hip_atomic_store(at(to + s * T, unsigned(l)), p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (uniform(wave) == 0) {
+          if (l == 0)
+            __hip_atomic_store(P.flags + K.rank, it + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          for (int k = far_first + l; k <= far_last; k += 64) {
+            Patience wait;
+            while (__hip_atomic_load(P.flags + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < it + 1)
+              if (wait.over(P.gave_up, P.wait_ticks)) {
+                failed = 1;
+                break;
+              }
+          }
+          const double* from = to - below;
+          for (int e = l; e < nhalo; e += 64)
+            pl[halo_place(e)] = __hip_atomic_load(at(from, unsigned(e < below ? e : rows + e)), __ATOMIC_RELAXED,
+                                                  __HIP_MEMORY_SCOPE_AGENT);
+        }
+      } else if (it > 0) {
 #pragma unroll
         for (int s = 0; s < S; ++s)
-          pt[s * RES_LANES] = fma(beta, pt[s * RES_LANES], r[s]);
+          pt[s * T] = fma(beta, pt[s * T], r[s]);
         if (!alone) {
           const double* from = P.r_pub[(it & 1) ^ 1] + (SELL ? 0 : K.row0 - below);
-          for (int e0 = l; e0 < nhalo; e0 += RES_HALO * RES_LANES) {
+          for (int e0 = l; e0 < nhalo; e0 += RES_HALO * T) {
             Patience wait;
-            const bool later = e0 >= RES_HALO * RES_LANES; // entries not asked for yet
+            const bool later = e0 >= RES_HALO * T; // entries not asked for yet
             unsigned src[RES_HALO];
 #pragma unroll
             for (int k = 0; k < RES_HALO; ++k) {
-              const int e = e0 + k * RES_LANES;
+              const int e = e0 + k * T;
               if (later)
                 halo[k] = RES_EMPTY;
               if constexpr (SELL)
@@ -360,11 +412,11 @@ __global__ void __launch_bounds__(RES_LANES) k_pcg_resident(ResidentParams P)
               empty = false;
 #pragma unroll
               for (int k = 0; k < RES_HALO; ++k)
-                if (e0 + k * RES_LANES < nhalo && halo[k] == RES_EMPTY)
+                if (e0 + k * T < nhalo && halo[k] == RES_EMPTY)
                   halo[k] = slot_load(at(from, src[k]));
 #pragma unroll
               for (int k = 0; k < RES_HALO; ++k)
-                empty = empty || (e0 + k * RES_LANES < nhalo && halo[k] == RES_EMPTY);
+                empty = empty || (e0 + k * T < nhalo && halo[k] == RES_EMPTY);
               if (empty && wait.over(P.gave_up, P.wait_ticks)) {
                 failed = 1;
                 break;
@@ -372,7 +424,7 @@ __global__ void __launch_bounds__(RES_LANES) k_pcg_resident(ResidentParams P)
             } while (empty);
 #pragma unroll
             for (int k = 0; k < RES_HALO; ++k) {
-              const int e = e0 + k * RES_LANES;
+              const int e = e0 + k * T;
               if (e < nhalo) {
                 double& pe = pl[halo_place(e)];
                 pe = fma(beta, pe, __longlong_as_double((long long)halo[k]));
@@ -386,18 +438,18 @@ __global__ void __launch_bounds__(RES_LANES) k_pcg_resident(ResidentParams P)
       if (uniform(failed))
         return;
       // q = Ah p, and p.q of the operator blocks: per 64 rows of one slot, or as the vector blocks
-      double q[LEAN ? 1 : S], dot = 0.;
+      double q[QLDS ? 1 : S], dot = 0.;
       double* const ql = pl + R + 2 * reach + l;
       auto take = [&](int s, double p, double a) { // the product's row of slot s
-        if constexpr (LEAN)
-          ql[s * RES_LANES] = a;
+        if constexpr (QLDS)
+          ql[s * T] = a;
         else
           q[s] = a;
         dot = fma(p, a, dot);
         if (!SAME || s % ITEMS == ITEMS - 1) {
           const double w = wave_sum(dot);
           if ((l & 63) == 0)
-            ga[(SAME ? s >> LG : s) * RES_WAVES + wave] = w;
+            ga[(SAME ? s >> LG : s) * NW + wave] = w;
           dot = 0.;
         }
       };
@@ -417,7 +469,7 @@ __global__ void __launch_bounds__(RES_LANES) k_pcg_resident(ResidentParams P)
               for (int k = 0; k < W; ++k)
                 a = fma(mv[s][k0 + k], x[k], a);
             }
-          take(s, pt[s * RES_LANES], a);
+          take(s, pt[s * T], a);
         }
       } else if constexpr (SELL) {
         // a wave's rows of a slot are one slice; the first entries of the next slice are asked for ahead of the sums
@@ -427,7 +479,7 @@ __global__ void __launch_bounds__(RES_LANES) k_pcg_resident(ResidentParams P)
         int64_t first[2];
         auto ask = [&](int s) {
           if (width[s] > 0) {
-            first[s & 1] = P.slice_ptr[K.slice0 + s * RES_WAVES + uniform(wave)];
+            first[s & 1] = P.slice_ptr[K.slice0 + s * NW + uniform(wave)];
 #pragma unroll
             for (int k = 0; k < W; ++k) {
               const unsigned e = unsigned(min(k, width[s] - 1) * 64 + (l & 63));
@@ -456,33 +508,77 @@ __global__ void __launch_bounds__(RES_LANES) k_pcg_resident(ResidentParams P)
               a = fma(*at(P.scaled + first[s & 1], e), pl[*at(P.sell_local + first[s & 1], e)], a);
             }
           }
-          take(s, pt[s * RES_LANES], a);
+          take(s, pt[s * T], a);
         }
       } else {
       const double *pd[MU], *pu[MU];
 #pragma unroll
-      for (int u = 0; u < NU; ++u)
+      for (int u = 0; u < NN; ++u)
         pd[u] = pt - off[u], pu[u] = pt + off[u];
-      constexpr int G = S < 2 ? S : 2; // slots whose loads are in flight together
+      // FAR: the outermost columns, asked for two slots at a time ahead of the sums
+      const double* const pf = P.r_pub[0] + K.row0;
+      const int fo = FAR ? off[NU - 1] : 0;
+      const int fl = FAR ? int(max(int64_t(fo) - (K.row0 - lo), int64_t(0))) : 0;  // first row with a column below
+      const int fu = FAR ? int(min(hi - fo - K.row0, int64_t(rows))) : 0;          // end of the rows with one above
+      double xf[2][2][2]; // [pair of slots][slot][below, above]
+      auto far_ask = [&](int s0, int b) {
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+          const int o = l + (s0 + g) * T;
+          xf[b][g][0] = xf[b][g][1] = 0.;
+          if (o >= fl && o < rows)
+            xf[b][g][0] = __hip_atomic_load(at(pf - fo, unsigned(o)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          if (o < fu)
+            xf[b][g][1] = __hip_atomic_load(at(pf + fo, unsigned(o)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+      };
+      if constexpr (FAR)
+        far_ask(0, 0);
+      constexpr int G = S < 2 || (KEEP && S == 8 && NU == 4) ? 1 : 2; // slots whose loads are in flight together
 #pragma unroll
       for (int s0 = 0; s0 < S; s0 += G) {
         double ml[G][MU], mu[G][MU], xl[G][MU], xu[G][MU], xc[G];
+        constexpr int FB = 2;
+        const int fb = (s0 / FB) & 1;
+        if constexpr (FAR)
+          if (s0 + G < S)
+            far_ask(s0 + G, fb ^ 1);
 #pragma unroll
         for (int g = 0; g < G; ++g) {
-          const int s = s0 + g, oc = KEEP ? 0 : min(l + s * RES_LANES, rows - 1);
+          const int s = s0 + g;
+          if constexpr (KEEP) {
 #pragma unroll
-          for (int u = 0; u < NU; ++u) {
-            if constexpr (KEEP) {
+            for (int u = 0; u < NU; ++u)
               ml[g][u] = al[s][u], mu[g][u] = au[s][u];
-            } else {
+          } else if constexpr (FAR) {
+            // (entries past either end of the instance are read from the storage's padding, times p = 0)
+#pragma unroll
+            for (int u = 0; u < NU; ++u) {
+              const double* col = P.scaled + int64_t(u) * n + K.row0 + s * T;
+              ml[g][u] = *at(col - off[u], unsigned(l));
+              mu[g][u] = *at(col, unsigned(l));
+            }
+          } else {
+            const int oc = min(l + s * T, rows - 1);
+#pragma unroll
+            for (int u = 0; u < NU; ++u) {
               // (rows whose partner lies below the instance read the first valid entry, times p = 0)
               const double* col = P.scaled + int64_t(u < ku ? u : 0) * n + K.row0;
               ml[g][u] = *at(col - min(off[u], below), unsigned(max(oc - max(off[u] - below, 0), 0)));
               mu[g][u] = *at(col, unsigned(oc));
+              if (off[u] <= 0)
+                ml[g][u] = mu[g][u] = 0.;
             }
-            xl[g][u] = pd[u][s * RES_LANES], xu[g][u] = pu[u][s * RES_LANES];
           }
-          xc[g] = pt[s * RES_LANES];
+#pragma unroll
+          for (int u = 0; u < NN; ++u)
+            xl[g][u] = pd[u][s * T], xu[g][u] = pu[u][s * T];
+          xc[g] = pt[s * T];
+        }
+        if constexpr (FAR) {
+#pragma unroll
+          for (int g = 0; g < G; ++g)
+            xl[g][NU - 1] = xf[fb][g][0], xu[g][NU - 1] = xf[fb][g][1];
         }
 #pragma unroll
         for (int g = 0; g < G; ++g) {
@@ -490,114 +586,131 @@ __global__ void __launch_bounds__(RES_LANES) k_pcg_resident(ResidentParams P)
           double a = 0.;
 #pragma unroll
           for (int u = NU - 1; u >= 0; --u)
-            a = fma((KEEP || off[u] > 0) ? ml[g][u] : 0., xl[g][u], a);
+            a = fma(ml[g][u], xl[g][u], a);
           a += xc[g];
 #pragma unroll
           for (int u = 0; u < NU; ++u)
-            a = fma((KEEP || off[u] > 0) ? mu[g][u] : 0., xu[g][u], a);
-          if constexpr (!KEEP)
-            a = l + s * RES_LANES < rows ? a : 0.;
+            a = fma(mu[g][u], xu[g][u], a);
+          if (!KEEP && !whole)
+            a = l + s * T < rows ? a : 0.;
           take(s, xc[g], a);
         }
         if constexpr (!KEEP)
           asm volatile("" ::: "memory"); // no more matrix loads in flight than there are registers for
       }
       }
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // the slots cleared by the last exchange are empty
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads();
-      double own1[1] = {0.};
       const int par = it & 1, set = it % 3;
-      if (l < own_na) {
-        const int g = SAME ? vwaves : P.a_rows >> 6;
-        own1[0] = add_run(ga + l * g, g);
-        if (!alone) {
-          slot_store(at(P.g1 + set * P.n_a + K.own_a, unsigned(l)), own1[0]);
-          slot_clear(at(P.g1 + (it + 2) % 3 * P.n_a + K.own_a, unsigned(l)));
-        }
-      }
-      double sv[LEAN ? S : 1];
-      if constexpr (LEAN)
+      double sv[SQMEM ? S : 1];
+      if constexpr (SQMEM)
 #pragma unroll
         for (int s = 0; s < S; ++s)
-          sv[s] = *at(P.dsq + K.row0, unsigned(min(l + s * RES_LANES, rows - 1)));
+          sv[s] = *at(P.dsq + K.row0, unsigned(min(l + s * T, rows - 1)));
       double tot1[1];
-      if (!exchange_sum<1>(P.g1 + set * P.n_a + K.a0, own1, alone, K.na, P.v_block, red1, &failed, P.gave_up,
-                           P.wait_ticks, tot1))
-        return;
+      if (single) {
+        tot1[0] = add_run(ga, SAME ? vwaves : P.a_rows >> 6);
+      } else {
+        double own1[1] = {0.};
+        if (l < own_na) {
+          const int g = SAME ? vwaves : P.a_rows >> 6;
+          own1[0] = add_run(ga + l * g, g);
+          if (!alone) {
+            slot_store(at(P.g1 + (set * P.n_a + K.own_a) * RES_PAD, unsigned(l) * RES_PAD), own1[0]);
+            slot_clear(at(P.g1 + ((it + 2) % 3 * P.n_a + K.own_a) * RES_PAD, unsigned(l) * RES_PAD));
+          }
+        }
+        if (!exchange_sum<1, NW>(P.g1 + (set * P.n_a + K.a0) * RES_PAD, own1, alone, K.na, P.v_block, red1, &failed,
+                                 P.gave_up, P.wait_ticks, tot1))
+          return;
+      }
       pq = tot1[0];
       if (!uniform(pq > 0.)) { // breakdown: the iterate holds every earlier step
         state = 3;
         break;
       }
-      // update of r, the partials of the residual norms, the rows other workgroups read
+      // update of r, the rows other workgroups read, the partials of the residual norms
       alpha = rho / pq;
       double v[2] = {0., 0.};
+      double* const to = P.r_pub[par] + K.row0;
 #pragma unroll
       for (int s = 0; s < S; ++s) {
-        const double ri = fma(-alpha, LEAN ? ql[s * RES_LANES] : q[LEAN ? 0 : s], r[s]);
+        const double ri = fma(-alpha, QLDS ? ql[s * T] : q[QLDS ? 0 : s], r[s]);
         r[s] = ri;
-        const double ru = (LEAN ? sv[LEAN ? s : 0] : sq[LEAN ? 0 : s]) * ri;
+        if (!FAR && !alone) {
+          const int o = l + s * T;
+          if (SELL ? (pub >> s) & 1u : o < pub_lo || o >= pub_hi)
+            slot_store(at(to, unsigned(o)), ri);
+        }
+        const double ru = (SQMEM ? sv[SQMEM ? s : 0] : sq[SQMEM ? 0 : s]) * ri;
         v[0] = fma(ri, ri, v[0]), v[1] = fma(ru, ru, v[1]);
         if (s % ITEMS == ITEMS - 1) {
           const double w0 = wave_sum(v[0]), w1 = wave_sum(v[1]);
           if ((l & 63) == 0)
-            gv[0][(s >> LG) * RES_WAVES + wave] = w0, gv[1][(s >> LG) * RES_WAVES + wave] = w1;
+            gv[0][(s >> LG) * NW + wave] = w0, gv[1][(s >> LG) * NW + wave] = w1;
           v[0] = v[1] = 0.;
         }
       }
       __syncthreads();
       double own2[2] = {0., 0.};
-      if (l < own_nv) {
+      if (single) {
+        rn[0] = add_run(gv[0], vwaves), rn[1] = add_run(gv[1], vwaves);
+      } else if (l < own_nv) {
         own2[0] = add_run(gv[0] + l * vwaves, vwaves), own2[1] = add_run(gv[1] + l * vwaves, vwaves);
         if (!alone) {
-          double* mine = at(P.g2 + 2 * (par * P.n_v + K.own_v), 2u * unsigned(l));
-          double* other = at(P.g2 + 2 * ((par ^ 1) * P.n_v + K.own_v), 2u * unsigned(l));
+          double* mine = at(P.g2 + (par * P.n_v + K.own_v) * RES_PAD, unsigned(l) * RES_PAD);
           slot_store(mine, own2[0]), slot_store(mine + 1, own2[1]);
-          slot_clear(other), slot_clear(other + 1);
         }
       }
-      if (!alone) {
-        double *to = P.r_pub[par] + K.row0, *old = P.r_pub[par ^ 1] + K.row0;
-#pragma unroll
-        for (int s = 0; s < S; ++s) {
-          const int o = l + s * RES_LANES;
-          if (SELL ? (pub >> s) & 1u : o < pub_lo || o >= pub_hi)
-            slot_store(at(to, unsigned(o)), r[s]), slot_clear(at(old, unsigned(o)));
-        }
-      }
-      // in the time the exchange takes: x, and the halo's rows of r (empty where their workgroup is not that far)
-      if constexpr (LEAN) {
+      // in the time the exchange takes: x, the next step's slots and rows emptied, and the halo's rows of r asked for
+      // (empty where their workgroup is not that far)
+      if constexpr (XMEM) {
         double xv[S];
 #pragma unroll
         for (int s = 0; s < S; ++s)
-          xv[s] = *at(P.x_work + K.row0, unsigned(min(l + s * RES_LANES, rows - 1)));
+          xv[s] = *at(P.x_work + K.row0, unsigned(min(l + s * T, rows - 1)));
 #pragma unroll
         for (int s = 0; s < S; ++s)
-          if (l + s * RES_LANES < rows)
-            *at(P.x_work + K.row0, unsigned(l + s * RES_LANES)) = fma(alpha, pt[s * RES_LANES], xv[s]);
+          if (l + s * T < rows)
+            *at(P.x_work + K.row0, unsigned(l + s * T)) = fma(alpha, pt[s * T], xv[s]);
       } else {
 #pragma unroll
         for (int s = 0; s < S; ++s)
-          x[s] = fma(alpha, pt[s * RES_LANES], x[s]);
+          x[s] = fma(alpha, pt[s * T], x[s]);
       }
       if (!alone) {
+        if (l < own_nv) {
+          double* next = at(P.g2 + ((par ^ 1) * P.n_v + K.own_v) * RES_PAD, unsigned(l) * RES_PAD);
+          slot_clear(next), slot_clear(next + 1);
+        }
+        if constexpr (!FAR) {
+          double* const next = P.r_pub[par ^ 1] + K.row0;
+#pragma unroll
+          for (int s = 0; s < S; ++s) {
+            const int o = l + s * T;
+            if (SELL ? (pub >> s) & 1u : o < pub_lo || o >= pub_hi)
+              slot_clear(at(next, unsigned(o)));
+          }
+        }
+      }
+      if (!alone && !FAR) {
         const double* from = P.r_pub[par] + (SELL ? 0 : K.row0 - below);
 #pragma unroll
         for (int k = 0; k < RES_HALO; ++k) {
-          const int e = l + k * RES_LANES;
+          const int e = l + k * T;
           if (e < nhalo)
             halo[k] = slot_load(at(from, unsigned(SELL ? hr[k] : e < below ? e : rows + e)));
         }
       }
-      if (!exchange_sum<2>(P.g2 + 2 * (par * P.n_v + K.v0), own2, alone, K.nv, P.v_block, red2, &failed, P.gave_up,
-                           P.wait_ticks, rn))
+      if (!single && !exchange_sum<2, NW>(P.g2 + (par * P.n_v + K.v0) * RES_PAD, own2, alone, K.nv, P.v_block, red2, &failed,
+                                          P.gave_up, P.wait_ticks, rn))
         return;
     }
 #pragma unroll
     for (int s = 0; s < S; ++s) {
-      const int o = t + s * RES_LANES;
+      const int o = t + s * T;
       if (o < rows)
-        P.x[K.row0 + o] = LEAN ? P.x_work[K.row0 + o] : x[LEAN ? 0 : s];
+        P.x[K.row0 + o] = XMEM ? P.x_work[K.row0 + o] : x[XMEM ? 0 : s];
     }
     if (K.rank == 0 && t == 0) {
       PcgScalars* D = P.S + K.inst;
@@ -613,11 +726,14 @@ __global__ void __launch_bounds__(RES_LANES) k_pcg_resident(ResidentParams P)
 __global__ void __launch_bounds__(256) k_resident_clear(ResidentParams P, int64_t slots)
 {
   const double empty = __longlong_as_double((long long)RES_EMPTY);
-  const int64_t i = xcd_index(max(P.n, slots));
+  constexpr int FLAGS = RES_MAX_GROUPS;
+  const int64_t i = xcd_index(max(max(P.n, slots), int64_t(FLAGS)));
   if (i < slots)
     P.g1[i] = empty;
   if (i < P.n)
     P.r_pub[0][i] = empty, P.r_pub[1][i] = empty;
+  if (i < FLAGS)
+    P.flags[i] = 0;
   if (i == 0)
     *P.gave_up = 0;
 }
@@ -632,28 +748,36 @@ Kernel kernel_for(int slots, int lg, bool same)
   if (same)
     switch (slots * 16 + lg) {
       case 16:
-        return k_pcg_resident<1, 0, true, NU, 1>;
+        return k_pcg_resident<RES_LANES, 1, 0, true, NU, 1>;
       case 33:
-        return k_pcg_resident<2, 1, true, NU, 1>;
+        return k_pcg_resident<RES_LANES, 2, 1, true, NU, 1>;
       case 66:
-        return k_pcg_resident<4, 2, true, NU, 1>;
+        return k_pcg_resident<RES_LANES, 4, 2, true, NU, 1>;
       case 131:
-        return k_pcg_resident<8, 3, true, NU, 1>;
+        return k_pcg_resident<RES_LANES, 8, 3, true, NU, 1>;
       case 259:
-        return k_pcg_resident<16, 3, true, NU, 0>;
+        return k_pcg_resident<RES_LANES, 16, 3, true, NU, 0>;
     }
   if (lg == 0)
     switch (slots) {
       case 1:
-        return k_pcg_resident<1, 0, false, NU, 1>;
+        return k_pcg_resident<RES_LANES, 1, 0, false, NU, 1>;
       case 2:
-        return k_pcg_resident<2, 0, false, NU, 1>;
+        return k_pcg_resident<RES_LANES, 2, 0, false, NU, 1>;
       case 4:
-        return k_pcg_resident<4, 0, false, NU, 1>;
+        return k_pcg_resident<RES_LANES, 4, 0, false, NU, 1>;
       case 8:
-        return k_pcg_resident<8, 0, false, NU, 1>;
+        return k_pcg_resident<RES_LANES, 8, 0, false, NU, 1>;
     }
   return nullptr;
+}
+
+// FAR: blocks of RES_FAR_BLOCK lanes and 4 rows per lane
+Kernel far_kernel(int slots)
+{
+  return slots == 4 ? k_pcg_resident<RES_FAR_BLOCK, 4, 2, true, 3, 1, true>
+         : slots == 8 ? k_pcg_resident<RES_FAR_BLOCK, 8, 2, true, 3, 0, true>
+                      : k_pcg_resident<RES_FAR_BLOCK, 12, 2, true, 3, 0, true>;
 }
 
 // nu < 0: SELL, slices of at most -nu entries per row
@@ -665,14 +789,14 @@ Kernel kernel_of(int slots, int lg, bool same, int nu)
     const int w = -nu;
     switch (slots) {
       case 1:
-        return w <= 28 ? k_pcg_resident<1, 0, true, 0, 28> : k_pcg_resident<1, 0, true, 0, 0>;
+        return w <= 28 ? k_pcg_resident<RES_LANES, 1, 0, true, 0, 28> : k_pcg_resident<RES_LANES, 1, 0, true, 0, 0>;
       case 2:
-        return w <= 12 ? k_pcg_resident<2, 1, true, 0, 12> : w <= 28 ? k_pcg_resident<2, 1, true, 0, 28>
-                                                                       : k_pcg_resident<2, 1, true, 0, 0>;
+        return w <= 12 ? k_pcg_resident<RES_LANES, 2, 1, true, 0, 12> : w <= 28 ? k_pcg_resident<RES_LANES, 2, 1, true, 0, 28>
+                                                                       : k_pcg_resident<RES_LANES, 2, 1, true, 0, 0>;
       case 4:
-        return w <= 12 ? k_pcg_resident<4, 2, true, 0, 12> : k_pcg_resident<4, 2, true, 0, 0>;
+        return w <= 12 ? k_pcg_resident<RES_LANES, 4, 2, true, 0, 12> : k_pcg_resident<RES_LANES, 4, 2, true, 0, 0>;
       case 8:
-        return k_pcg_resident<8, 3, true, 0, 0>;
+        return k_pcg_resident<RES_LANES, 8, 3, true, 0, 0>;
     }
     return nullptr;
   }
@@ -715,9 +839,9 @@ int device_cus()
 
 } // namespace
 
-static int64_t team_of(int64_t rows, int slots)
+static int64_t team_of(int64_t rows, int slots, int lanes = RES_LANES)
 {
-  const int64_t R = int64_t(slots) * RES_LANES;
+  const int64_t R = int64_t(slots) * lanes;
   return (rows + R - 1) / R;
 }
 
@@ -736,7 +860,7 @@ static bool enough_rows(int64_t rows, int slots, int cus, bool sell)
 // Instances of a batch in the order of their size, each on the workgroups that are free first: the estimated time until
 // the last one ends, and (order, groups) which instance is next and on which workgroups.  A workgroup takes its instances
 // in this order, so the first unfinished one always has all of its workgroups.  Negative: an instance does not fit.
-static double schedule(const std::vector<int64_t>& row0, int slots, int cus, std::vector<int>* order,
+static double schedule(const std::vector<int64_t>& row0, int slots, int lanes, int cus, std::vector<int>* order,
                        std::vector<std::vector<int>>* groups)
 {
   // us per iteration of one workgroup with 1, 2, 4, 8, 16 rows per lane (measured), and of the exchanges
@@ -754,8 +878,8 @@ static double schedule(const std::vector<int64_t>& row0, int slots, int cus, std
     groups->assign(ninst, {});
   double last = 0.;
   for (int i : by_size) {
-    const int64_t n = row0[i + 1] - row0[i], team = team_of(n, slots);
-    if (team > cus)
+    const int64_t n = row0[i + 1] - row0[i], team = team_of(n, slots, lanes);
+    if (team > cus || team > RES_MAX_GROUPS)
       return -1.;
     std::partial_sort(load.begin(), load.begin() + team, load.end());
     // iterations grow like the square root of the size (two dimensions)
@@ -785,7 +909,7 @@ static int choose_slots(const std::vector<int64_t>& row0, bool sell, F fits)
         return s;
       continue;
     }
-    const double t = schedule(row0, s, cus, nullptr, nullptr);
+    const double t = schedule(row0, s, RES_LANES, cus, nullptr, nullptr);
     if (t >= 0. && (best < 0 || t < time) && fits(s))
       best = s, time = t;
   }
@@ -803,27 +927,55 @@ static int64_t reach_of(const std::vector<int64_t>& row0, const std::vector<std:
   return reach;
 }
 
-static int64_t lds_of(int slots, int64_t reach)
+static int64_t lds_of(int slots, int64_t reach, int s_nu)
 {
-  return (int64_t(slots) * RES_LANES * (slots > 8 ? 2 : 1) + 2 * reach) * int64_t(sizeof(double)); // (LEAN: q)
+  return (int64_t(slots) * RES_LANES * (q_in_lds(slots, s_nu <= 3 ? 3 : 4, false) ? 2 : 1) + 2 * reach) *
+         int64_t(sizeof(double));
+}
+static int64_t far_lds(int slots, int64_t near)
+{
+  return (int64_t(slots) * RES_FAR_BLOCK * 2 + 2 * near) * int64_t(sizeof(double));
 }
 
-int resident_items(const std::vector<int64_t>& row0, const std::vector<std::vector<int64_t>>& s_offs, int s_nu)
+// FAR: one instance of three offsets, the outermost past what LDS holds; rows per lane (0: not this case)
+static int far_slots(const std::vector<int64_t>& row0, const std::vector<std::vector<int64_t>>& s_offs, int s_nu)
+{
+  if (row0.size() != 2 || s_nu != 3 || s_offs[0].size() != 3 || s_offs[0][2] >= row0[1] - row0[0])
+    return 0;
+  for (int s : {4, 8, 12})
+    if (team_of(row0[1], s, RES_FAR_BLOCK) <= device_cus() && far_lds(s, s_offs[0][1]) <= RES_LDS)
+      return s;
+  return 0;
+}
+
+int64_t resident_padding(const std::vector<int64_t>& row0, const std::vector<std::vector<int64_t>>& s_offs, int s_nu)
+{
+  if (!far_slots(row0, s_offs, s_nu))
+    return 0;
+  return std::max<int64_t>(s_offs[0].back(), int64_t(12) * RES_FAR_BLOCK);
+}
+
+ResidentShape resident_shape_dia(const std::vector<int64_t>& row0, const std::vector<std::vector<int64_t>>& s_offs,
+                                 int s_nu)
 {
   if (s_nu < 0 || s_nu > 4)
-    return 0;
+    return {};
   const int64_t reach = reach_of(row0, s_offs);
-  const int s = choose_slots(row0, false, [&](int k) { return lds_of(k, reach) <= RES_LDS && !(s_nu == 0 && k > 8); });
-  return s < 0 ? 0 : std::min(s, 8); // (16 rows per lane: two blocks of 8 each)
+  const int s = choose_slots(row0, false, [&](int k) { return lds_of(k, reach, s_nu) <= RES_LDS && !(s_nu == 0 && k > 8); });
+  if (s > 0)
+    return {RES_LANES, std::min(s, 8)}; // (16 rows per lane: two blocks of 8 each)
+  if (far_slots(row0, s_offs, s_nu))
+    return {RES_FAR_BLOCK, 4};
+  return {};
 }
 
 // one workgroup's rows after the other, instance by instance; false when the lanes that add the partials of an
 // instance of one workgroup do not hold them all
-static bool list_tasks(const Operator& op, int slots, std::vector<ResidentTask>& tasks)
+static bool list_tasks(const Operator& op, int slots, int lanes, std::vector<ResidentTask>& tasks)
 {
   const SolverFormat& F = op.fmt;
   const std::vector<int64_t>& row0 = op.space->inst_dof;
-  const int64_t R = int64_t(slots) * RES_LANES, va = int64_t(F.A.block) * F.A.items, vv = int64_t(F.V.block) * F.V.items;
+  const int64_t R = int64_t(slots) * lanes, va = int64_t(F.A.block) * F.A.items, vv = int64_t(F.V.block) * F.V.items;
   for (size_t in = 0; in + 1 < row0.size(); ++in) {
     const int64_t ni = row0[in + 1] - row0[in];
     const int team = int((ni + R - 1) / R);
@@ -849,7 +1001,7 @@ static void finish_plan(ResidentPlan& plan, const Operator& op, const std::vecto
 {
   std::vector<int> order;
   std::vector<std::vector<int>> groups;
-  if (schedule(op.space->inst_dof, plan.slots, device_cus(), &order, &groups) < 0.)
+  if (schedule(op.space->inst_dof, plan.slots, plan.lanes, device_cus(), &order, &groups) < 0.)
     return;
   std::vector<int64_t> first(groups.size(), 0); // first task of every instance
   for (size_t k = tasks.size(); k-- > 0;)
@@ -861,17 +1013,25 @@ static void finish_plan(ResidentPlan& plan, const Operator& op, const std::vecto
         of.resize(groups[i][k] + 1);
       of[groups[i][k]].push_back(tasks[first[i] + int64_t(k)]);
     }
+  // consecutive workgroups on one XCD (hardware deals them round-robin to 8), as neighbours exchange their halos
+  plan.workgroups = int(of.size());
+  const size_t q = (of.size() + 7) / 8;
+  of.resize(8 * q);
+  std::vector<std::vector<ResidentTask>> dealt(8 * q);
+  for (size_t w = 0; w < 8 * q; ++w)
+    dealt[(w % q) * 8 + w / q] = std::move(of[w]);
+  of = std::move(dealt);
   std::vector<ResidentTask> list;
   std::vector<int32_t> start{0};
   for (auto& w : of) {
     list.insert(list.end(), w.begin(), w.end());
     start.push_back(int32_t(list.size()));
   }
-  plan.workgroups = int(of.size()), plan.lds = lds;
+  plan.grid = int(of.size()), plan.lds = lds;
   plan.tasks.upload(list);
   plan.task_start.upload(start);
-  plan.exchange.allocate(size_t(3 * op.fmt.A.nblocks + 4 * op.fmt.V.nblocks));
-  plan.gave_up.allocate(1);
+  plan.exchange.allocate(size_t(RES_PAD * (3 * op.fmt.A.nblocks + 2 * op.fmt.V.nblocks)));
+  plan.gave_up.allocate(1 + RES_MAX_GROUPS);
   if (!plan.host_gave_up)
     HGDT_HIP(hipHostMalloc((void**)&plan.host_gave_up, sizeof(int)));
   plan.usable = true;
@@ -883,6 +1043,19 @@ void resident_plan_dia(ResidentPlan& plan, const Operator& op, const std::vector
   plan.usable = false;
   const SolverFormat& F = op.fmt;
   const int bv = F.V.block, iv = F.V.items, ba = F.A.block * F.A.items;
+  plan.sell = plan.far = false;
+  plan.lanes = RES_LANES;
+  if (bv == RES_FAR_BLOCK && iv == 4 && F.A.block == bv && F.A.items == iv) {
+    const int slots = far_slots(op.space->inst_dof, s_offs, s_nu);
+    std::vector<ResidentTask> tasks;
+    if (!slots || !list_tasks(op, slots, RES_FAR_BLOCK, tasks))
+      return;
+    plan.far = true;
+    plan.lanes = RES_FAR_BLOCK;
+    plan.slots = slots, plan.lg_items = 2, plan.same_blocks = true, plan.nu = s_nu;
+    finish_plan(plan, op, tasks, far_lds(slots, s_offs[0][1]));
+    return;
+  }
   const bool same = bv == RES_LANES && F.A.block == bv && F.A.items == iv;
   if (s_nu < 0 || s_nu > 4 || RES_LANES % bv != 0 || !(same || (F.A.items == 1 && ba <= 1024 && (ba & (ba - 1)) == 0)))
     return;
@@ -895,17 +1068,16 @@ void resident_plan_dia(ResidentPlan& plan, const Operator& op, const std::vector
   const int64_t reach = reach_of(row0, s_offs);
   const int slots = choose_slots(row0, false, [&](int k) {
     // (a diagonal matrix holds no slot to stream)
-    return (int64_t(k) * RES_LANES) % ba == 0 && kernel_of(k, lg, same, s_nu) && lds_of(k, reach) <= RES_LDS &&
+    return (int64_t(k) * RES_LANES) % ba == 0 && kernel_of(k, lg, same, s_nu) && lds_of(k, reach, s_nu) <= RES_LDS &&
            !(s_nu == 0 && k > 8);
   });
   if (slots < 0)
     return;
   std::vector<ResidentTask> tasks;
-  if (!list_tasks(op, slots, tasks))
+  if (!list_tasks(op, slots, RES_LANES, tasks))
     return;
-  plan.sell = false;
   plan.slots = slots, plan.lg_items = lg, plan.same_blocks = same, plan.nu = s_nu;
-  finish_plan(plan, op, tasks, lds_of(slots, reach));
+  finish_plan(plan, op, tasks, lds_of(slots, reach, s_nu));
 }
 
 // columns of the rows [r0, r1) that lie outside them, ascending
@@ -960,7 +1132,7 @@ void resident_plan_sell(ResidentPlan& plan, const Operator& op)
   if (!kernel_of(slots, lg, true, -1))
     return;
   std::vector<ResidentTask> tasks;
-  if (!list_tasks(op, slots, tasks))
+  if (!list_tasks(op, slots, RES_LANES, tasks))
     return;
   const int64_t R = int64_t(slots) * RES_LANES, nt = int64_t(tasks.size());
   std::vector<std::vector<int32_t>> halo(nt);
@@ -1014,7 +1186,8 @@ void resident_plan_sell(ResidentPlan& plan, const Operator& op)
     rows.push_back(0);
   plan.halo_rows.upload(rows);
   plan.publish.upload(pub);
-  plan.sell = true;
+  plan.sell = true, plan.far = false;
+  plan.lanes = RES_LANES;
   int64_t widest = 1;
   for (int64_t k = 0; k < F.nslices; ++k)
     widest = std::max(widest, (slice_ptr[k + 1] - slice_ptr[k]) / 64);
@@ -1025,13 +1198,13 @@ void resident_plan_sell(ResidentPlan& plan, const Operator& op)
 bool resident_run(ResidentPlan& plan, ResidentParams P, hipStream_t stream, PcgScalars* host_records)
 {
   P.g1 = plan.exchange.ptr;
-  P.g2 = plan.exchange.ptr + 3 * P.n_a;
+  P.g2 = plan.exchange.ptr + 3 * P.n_a * RES_PAD;
   P.sell_local = plan.sell_local.ptr, P.halo_rows = plan.halo_rows.ptr, P.publish = plan.publish.ptr;
-  P.tasks = plan.tasks.ptr, P.task_start = plan.task_start.ptr, P.gave_up = plan.gave_up.ptr;
+  P.tasks = plan.tasks.ptr, P.task_start = plan.task_start.ptr, P.gave_up = plan.gave_up.ptr, P.flags = plan.gave_up.ptr + 1;
   P.wait_ticks = int64_t(4) * 100000000; // 4 s
   const int64_t nx = int64_t(plan.exchange.count);
-  hipLaunchKernelGGL(k_resident_clear, dim3(xcd_grid(std::max(P.n, nx), 256)), dim3(256), 0, stream, P, nx);
-  const Kernel k = kernel_of(plan.slots, plan.lg_items, P.same_blocks, plan.nu);
+  hipLaunchKernelGGL(k_resident_clear, dim3(xcd_grid(std::max<int64_t>(std::max(P.n, nx), RES_MAX_GROUPS), 256)), dim3(256), 0, stream, P, nx);
+  const Kernel k = plan.far ? far_kernel(plan.slots) : kernel_of(plan.slots, plan.lg_items, P.same_blocks, plan.nu);
   HGDT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
                                int(RES_LDS)));
   int dev = 0;
@@ -1043,9 +1216,10 @@ bool resident_run(ResidentPlan& plan, ResidentParams P, hipStream_t stream, PcgS
       CuBudget::get().give(dev, count);
     }
   };
-  CuBudget::get().take(dev, plan.workgroups, device_cus());
-  Hold hold{dev, plan.workgroups};
-  hipLaunchKernelGGL(k, dim3(unsigned(plan.workgroups)), dim3(RES_LANES), size_t(plan.lds), stream, P);
+  const int cus = device_cus(), held = std::min(plan.grid, cus);
+  CuBudget::get().take(dev, held, cus);
+  Hold hold{dev, held};
+  hipLaunchKernelGGL(k, dim3(unsigned(plan.grid)), dim3(unsigned(plan.lanes)), size_t(plan.lds), stream, P);
   hipError_t e = hipGetLastError();
   if (e == hipSuccess)
     e = hipMemcpyAsync(plan.host_gave_up, plan.gave_up.ptr, sizeof(int), hipMemcpyDeviceToHost, stream);

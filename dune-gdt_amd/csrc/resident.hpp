@@ -7,6 +7,18 @@
 
 namespace hgdt {
 
+constexpr int RES_BLOCK = 512;     // lanes of a workgroup, and of the row blocks that suit it
+constexpr int RES_FAR_BLOCK = 768; // the same for 3-d lattices whose planes do not fit in LDS (12 rows per lane and 3
+                                   // waves per SIMD: 256 workgroups hold 2.36 million rows)
+// row blocks for a solve in one launch (block 0: it does not fit on the chip)
+struct ResidentShape {
+  int block = 0, items = 0;
+  bool operator!=(const ResidentShape& o) const
+  {
+    return block != o.block || items != o.items;
+  }
+};
+
 // one instance's share of a workgroup: consecutive rows of the instance, handled by `rank` of its team
 struct ResidentTask {
   int64_t row0;          // first own row
@@ -43,13 +55,14 @@ struct ResidentParams {
   double* x_work;      // the iterate of workgroups that do not hold it in registers
   double* r_pub[2];    // rows of r that other workgroups of the team read, by parity of the step
   const double* part2; // partials of the initial residual, 2 per vector block
-  double* g1;          // 3 x (operator blocks): partials of p.q, by step
-  double* g2;          // behind it, 2 x 2 x (vector blocks): partials of the two residual norms, by parity
+  double* g1;          // 2 x (operator blocks), padded: partials of p.q, by parity of the step
+  double* g2;          // behind it, 2 x (vector blocks), padded: partials of the two residual norms
   int64_t n_a, n_v;    // operator / vector blocks of all instances
   PcgScalars* S;       // record of every instance: tolerance read, result written
   int64_t max_iter;
   const ResidentTask* tasks;
   const int32_t* task_start; // per workgroup
+  int* flags;          // FAR: per workgroup, the step whose p it has published
   int* gave_up;        // set when a wait outlasts its limit: every workgroup then ends
   int64_t wait_ticks;  // limit of one wait, in ticks of the 100 MHz counter
 };
@@ -62,9 +75,11 @@ struct ResidentPlan {
   int lg_items = 0;     // log2 of the vector blocks' rows per lane
   bool same_blocks = false; // operator blocks = vector blocks
   int nu = 0;           // strict upper slots the kernel is compiled for
-  int workgroups = 0;
+  int workgroups = 0;   // with rows; the grid is rounded up to the 8 XCDs
+  int grid = 0;
   int64_t lds = 0;
-  bool sell = false;
+  bool sell = false, far = false;
+  int lanes = RES_BLOCK;
   DeviceArray<uint16_t> sell_local;
   DeviceArray<int32_t> halo_rows;
   DeviceArray<uint32_t> publish;
@@ -80,10 +95,11 @@ struct ResidentPlan {
   }
 };
 
-constexpr int RES_BLOCK = 512; // lanes of a workgroup, and of the row blocks that suit it
-// rows per lane of row blocks for a solve in one launch of symmetric DIA storage with these strict upper offsets;
-// 0: it does not fit on the chip
-int resident_items(const std::vector<int64_t>& inst_row0, const std::vector<std::vector<int64_t>>& s_offs, int s_nu);
+// symmetric DIA storage with these strict upper offsets
+ResidentShape resident_shape_dia(const std::vector<int64_t>& inst_row0, const std::vector<std::vector<int64_t>>& s_offs,
+                                 int s_nu);
+// doubles that the solve reads ahead of and past the scaled matrix's diagonals (those ahead must be finite)
+int64_t resident_padding(const std::vector<int64_t>& inst_row0, const std::vector<std::vector<int64_t>>& s_offs, int s_nu);
 // s_offs: the strict upper offsets of every instance's scaled matrix
 void resident_plan_dia(ResidentPlan& plan, const Operator& op, const std::vector<std::vector<int64_t>>& s_offs,
                        int s_nu);

@@ -306,16 +306,16 @@ __device__ __forceinline__ void apply_rows(const PcgParams& P, const double* __r
   }
 }
 
-// y = A x, one row per lane: a row block of `items` rows per lane is handled by `items` workgroups
+// y = A x, one row per lane: a row block of 1 << lg rows per lane is handled by as many workgroups
 template <int FMT>
-__global__ void __launch_bounds__(1024) k_apply(PcgParams P, int items, const double* __restrict__ x, double* __restrict__ y)
+__global__ void __launch_bounds__(1024) k_apply(PcgParams P, int lg, const double* __restrict__ x, double* __restrict__ y)
 {
-  const int w = logical_block(P.a_nb * items);
+  const int w = logical_block(P.a_nb << lg);
   if (w < 0)
     return;
-  const int b = w / items;
+  const int b = w >> lg;
   const int inst = P.a_inst[b];
-  const int64_t rb = P.a_row0[b], r1 = P.a_row0[b + 1], r0 = rb + int64_t(w - b * items) * blockDim.x;
+  const int64_t rb = P.a_row0[b], r1 = P.a_row0[b + 1], r0 = rb + int64_t(w - (b << lg)) * blockDim.x;
   if (r0 >= r1)
     return;
   const double* vals = (FMT == FMT_SELL) ? P.sell_vals : P.dia;
@@ -1382,7 +1382,8 @@ struct SolverCache {
   int64_t graph_version = -1;
   int64_t version = 0;
   ResidentPlan resident;
-  int shaped_for = 0; // resident_shape of the row partitions
+  int64_t scaled_pad = 0;   // doubles ahead of the scaled matrix in its storage (and past it)
+  ResidentShape shaped_for; // resident_shape of the row partitions
   int sell_items = 0; // SELL: rows per lane that suit a solve in one launch (0: none)
   ~SolverCache()
   {
@@ -1473,19 +1474,18 @@ void RowPartition::build_counts(const std::vector<int64_t>& inst_dof, const std:
 static bool blk_wanted(const Operator& op);
 static int kernel_format(const Operator& op);
 
-// rows per lane of the row blocks that suit a solve in one launch (resident.hip: blocks of RES_BLOCK lanes, the
-// operator's and the vector kernels' alike); 0: the caller chose shapes, or the storage (once it is known) or size
-// does not fit
-static int resident_shape(const Operator& op)
+// row blocks that suit a solve in one launch (resident.hip; the operator's and the vector kernels' alike); none: the
+// caller chose shapes, or the storage (once it is known) or size does not fit
+static ResidentShape resident_shape(const Operator& op)
 {
   const SolverCache& C = *op.solver_cache;
   if (op.launch[3].user || op.launch[4].user || !op.square())
-    return 0;
+    return {};
   if (op.fmt.format == HGDT_FORMAT_SELL && op.fmt.structure_ready)
-    return C.sell_items;
+    return C.sell_items ? ResidentShape{RES_BLOCK, C.sell_items} : ResidentShape{};
   if (!op.fmt.valid || op.fmt.format != HGDT_FORMAT_DIA || kernel_format(op) != FMT_DIAS)
-    return 0;
-  return resident_items(op.space->inst_dof, C.s_offs, C.s_nu);
+    return {};
+  return resident_shape_dia(op.space->inst_dof, C.s_offs, C.s_nu);
 }
 
 // row-block partitions of the operator (host set-up, O(number of blocks))
@@ -1499,9 +1499,9 @@ static void build_partitions(Operator& op)
   // instance's partials stays small
   if (!op.launch[3].user)
     op.launch[3].block = 256, op.launch[3].items = 1;
-  const int resident = resident_shape(op); // rows per lane of a solve in one launch
-  if (resident)
-    op.launch[3].block = RES_BLOCK, op.launch[3].items = resident;
+  const ResidentShape resident = resident_shape(op);
+  if (resident.block)
+    op.launch[3].block = resident.block, op.launch[3].items = resident.items;
   // the matrix-free kernels give every lane one row (continuous spaces, at most 256 lanes per block) or one
   // element of a tile of elements (discontinuous spaces: 256 lanes, 4 rows each)
   const bool mf = op.requested_format == HGDT_FORMAT_MATRIX_FREE;
@@ -1514,8 +1514,8 @@ static void build_partitions(Operator& op)
     op.launch[4].block = 256;
     const int64_t want = (op.n + 256 * 1024 - 1) / (256 * 1024);
     op.launch[4].items = want <= 1 ? 1 : want <= 2 ? 2 : want <= 4 ? 4 : 8;
-    if (resident)
-      op.launch[4].block = RES_BLOCK, op.launch[4].items = resident;
+    if (resident.block)
+      op.launch[4].block = resident.block, op.launch[4].items = resident.items;
   }
   C.shaped_for = resident;
   const std::vector<int64_t> tiles = mf_tiles ? mf_tile_counts(op) : std::vector<int64_t>{};
@@ -2022,7 +2022,7 @@ static PcgParams make_params(Operator& op)
   P.blk_nb = F.d_blk_nb.ptr;
   P.blk_mir = F.d_blk_mir.ptr;
   P.blk = F.d_blk.ptr;
-  P.scaled = F.d_scaled.ptr;
+  P.scaled = F.d_scaled.ptr + C.scaled_pad;
   P.dh = F.d_dh.ptr;
   P.dsq = F.d_dsq.ptr;
   P.ninst = int(op.space->inst_dof.size()) - 1;
@@ -2220,6 +2220,7 @@ void Operator::prepare_storage(hipStream_t stream)
     HGDT_HIP(hipStreamSynchronize(stream));
     F.diag_positive = (C.host_flags[0] == 0);
     const bool sym = C.host_flags[1] == 0 && allow_symmetric;
+    C.scaled_pad = 0;
     F.d_scaled.allocate(std::max<int64_t>(total, 1));
     hipLaunchKernelGGL(k_blk_scale, dim3(blocks_for(F.blk_ne, B)), dim3(B), 0, stream, P, F.d_dh.ptr,
                        F.d_scaled.ptr);
@@ -2277,15 +2278,22 @@ void Operator::prepare_storage(hipStream_t stream)
   // otherwise in the layout of the storage
   if (dia && sym) {
     compact_upper(*this, C.host_flags + 2);
-    F.d_scaled.allocate(std::max<int64_t>(int64_t(C.s_nu) * n, 1));
+    const int64_t pad = resident_padding(space->inst_dof, C.s_offs, C.s_nu);
+    const bool fresh = F.d_scaled.count != size_t(std::max<int64_t>(int64_t(C.s_nu) * n, 1) + 2 * pad);
+    F.d_scaled.allocate(size_t(std::max<int64_t>(int64_t(C.s_nu) * n, 1) + 2 * pad));
+    if (pad > 0 && (fresh || C.scaled_pad != pad))
+      hipLaunchKernelGGL(k_fill, dim3(blocks_for(pad, B)), dim3(B), 0, stream, pad, F.d_scaled.ptr, 0.);
+    C.scaled_pad = pad;
     hipLaunchKernelGGL(k_scale_upper, dim3(blocks_for(n, B)), dim3(B), 0, stream, n, C.s_nu, C.s_off.ptr,
-                       C.s_kidx.ptr, C.row_inst.ptr, F.d_inst_row0.ptr, F.d_dia.ptr, F.d_dh.ptr, F.d_scaled.ptr);
+                       C.s_kidx.ptr, C.row_inst.ptr, F.d_inst_row0.ptr, F.d_dia.ptr, F.d_dh.ptr, F.d_scaled.ptr + pad);
   } else if (dia) {
+    C.scaled_pad = 0;
     F.d_scaled.allocate(std::max<int64_t>(total, 1));
     hipLaunchKernelGGL(k_scale_dia, dim3(blocks_for(n, B), unsigned(F.ndiag)), dim3(B), 0, stream, n, F.ndiag,
                        F.d_dia_offsets.ptr, C.dia_k0.ptr, 1, C.row_inst.ptr, F.d_inst_row0.ptr, F.d_dia.ptr,
                        F.d_dh.ptr, F.d_scaled.ptr);
   } else {
+    C.scaled_pad = 0;
     F.d_scaled.allocate(std::max<int64_t>(total, 1));
     hipLaunchKernelGGL(k_fill, dim3(blocks_for(total, B)), dim3(B), 0, stream, total, F.d_scaled.ptr, 0.);
     hipLaunchKernelGGL(k_scale_values, dim3(blocks_for(n, B)), dim3(B), 0, stream, n, d_row_ptr.ptr, d_cols.ptr,
@@ -2311,7 +2319,10 @@ void Operator::apply(const double* x, double* y, hipStream_t stream)
   }
   PcgParams P = make_params(*this);
   const int block = fmt.A.block;
-  const unsigned grid = hw_blocks(fmt.A.nblocks * fmt.A.items);
+  int lg = 0; // (items is a power of two)
+  while ((1 << lg) < fmt.A.items)
+    ++lg;
+  const unsigned grid = hw_blocks(fmt.A.nblocks << lg);
   const int kf = kernel_format(*this);
   if (kf == FMT_BLK) {
     const unsigned g1 = xcd_grid(fmt.blk_ne, 256);
@@ -2323,11 +2334,11 @@ void Operator::apply(const double* x, double* y, hipStream_t stream)
     return;
   }
   if (kf == FMT_DIA)
-    hipLaunchKernelGGL(k_apply<FMT_DIA>, dim3(grid), dim3(block), 0, stream, P, fmt.A.items, x, y);
+    hipLaunchKernelGGL(k_apply<FMT_DIA>, dim3(grid), dim3(block), 0, stream, P, lg, x, y);
   else if (kf == FMT_DIAS)
-    hipLaunchKernelGGL(k_apply<FMT_DIAS>, dim3(grid), dim3(block), 0, stream, P, fmt.A.items, x, y);
+    hipLaunchKernelGGL(k_apply<FMT_DIAS>, dim3(grid), dim3(block), 0, stream, P, lg, x, y);
   else
-    hipLaunchKernelGGL(k_apply<FMT_SELL>, dim3(grid), dim3(block), 0, stream, P, fmt.A.items, x, y);
+    hipLaunchKernelGGL(k_apply<FMT_SELL>, dim3(grid), dim3(block), 0, stream, P, lg, x, y);
   HGDT_HIP(hipGetLastError());
 }
 

@@ -29,7 +29,8 @@ def _both(hgdt, op, **kw):
     ("heat_q1", [31, 15], 1), ("heat_q1", [63, 63], None), ("heat_q1", [90, 91], None), ("heat_q1", [700, 37], None),
     ("heat_q1", [3, 2000], None), ("heat_q1", [361, 362], None), ("heat_q1", [515, 509], None),
     ("p1_tets", [3, 2, 4], 1), ("p1_tets", [20, 17, 13], None), ("p1_tets", [9, 40, 31], None),
-    ("p1_tets", [47, 48, 49], None)])
+    ("p1_tets", [47, 48, 49], None), ("p1_tets", [86, 87, 88], 222), ("p1_tets", [120, 125, 60], 152),
+    ("p1_tets", [127, 128, 127], None)])
 def test_one_launch_equals_three_kernels(hgdt_mod, kind, cells, workgroups):
     print(f"case {kind} {cells}", flush=True)
     ne = int(np.prod(cells)) * (6 if kind == "p1_tets" else 1)
