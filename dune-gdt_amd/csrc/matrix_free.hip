@@ -41,51 +41,12 @@
 #include <hip/hip_ext.h>
 
 #include "block_reduce.hpp"
-#include "hgdt_internal.hpp"
+#include "mf_params.hpp"
 
 namespace hgdt {
 namespace {
 
-constexpr int MF_MAXF = 8;
 constexpr int TX = 32, TY = 8; // tile of the discontinuous kernel (elements): halo rows 1.3x the tile
-enum { MFK_CG_QUAD = 0, MFK_CG_HEX = 1, MFK_DG_QUAD = 2 };
-
-// the parameters of an appended form, in one record (a kernel's few forms then span few lines of its argument
-// block, which the kernel reads before anything else)
-struct MfElementForm {
-  const double* coef;
-  double value, scale;
-  int kind;
-};
-struct MfFaceForm {
-  const double* kappa;
-  const double* omega;
-  double kv, ov, param, scale;
-  int kind;
-};
-
-struct MfParams {
-  int ninst;
-  // per row block: first DoF and first element of the instance, cells n0 n1 n2, instance, first and last
-  // row of the block relative to the instance's first DoF
-  const int64_t* blk;
-  int64_t ref_stride; // doubles per instance of the reference data: h0 h1 1/h1 1/h0, element, face, boundary matrices
-  int64_t eoff; // offset of the element matrices inside an instance's block (continuous spaces)
-  int dirichlet;
-  int nef, ncf, nbf;
-  int nb; // row blocks (the solver's operator partition): one row or element per lane
-  const double* single; // the one coefficient field of every form (kernels that prefetch it), or NULL
-  MfVectors v;
-  // the forms last: a kernel reads the first nef / ncf / nbf records of each array
-  MfElementForm ef[MF_MAXF];
-  MfFaceForm ff[2][MF_MAXF]; // [0] inner, [1] boundary forms
-};
-
-// coefficient of a form at element e: the field's value, or the constant
-__device__ __forceinline__ double cf(const double* __restrict__ f, double value, int64_t e)
-{
-  return f ? f[e] : value;
-}
 
 // y += s (M v) for the N x N row-major matrix M (T: s (M^T v)); DIAG: y_i += s M_ii
 template <int N, bool T, bool DIAG>
@@ -1026,7 +987,7 @@ bool mf_fused_direction(const Operator& op)
   return op.fmt.format == HGDT_FORMAT_MATRIX_FREE && op.fmt.mf_kind == MFK_DG_QUAD;
 }
 
-void mf_launch(const Operator& op, int mode, const MfVectors& v, hipStream_t stream, hipEvent_t ev0, hipEvent_t ev1)
+MfParams mf_params(const Operator& op)
 {
   const SolverFormat& F = op.fmt;
   MfParams P{};
@@ -1050,6 +1011,13 @@ void mf_launch(const Operator& op, int mode, const MfVectors& v, hipStream_t str
       P.ff[grp][f].omega = Fm.omega, P.ff[grp][f].ov = Fm.omega_value;
     }
   }
+  return P;
+}
+
+void mf_launch(const Operator& op, int mode, const MfVectors& v, hipStream_t stream, hipEvent_t ev0, hipEvent_t ev1)
+{
+  const SolverFormat& F = op.fmt;
+  MfParams P = mf_params(op);
   P.nb = v.nb >= 0 ? v.nb : int(F.A.nblocks);
   P.v = v;
   // the coefficient field shared by every form, if there is one (every other coefficient a constant)

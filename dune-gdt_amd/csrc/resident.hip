@@ -42,157 +42,14 @@
 #include <map>
 #include <mutex>
 
-#include "block_reduce.hpp"
-#include "resident.hpp"
+#include "resident_device.hpp"
 
 namespace hgdt {
 namespace {
 
-constexpr int RES_LANES = RES_BLOCK;  // lanes of a workgroup (FAR: RES_FAR_BLOCK)
-constexpr int RES_MAX_SLOTS = 16;
-constexpr int RES_HALO = 4; // halo rows a lane asks for while the residual norms are exchanged
-constexpr int RES_WAVES = 12;              // of a workgroup, at most
-constexpr int RES_GROUPS = 144;            // 64-row groups of a workgroup, at most
-constexpr int RES_MAX_GROUPS = 1024;                  // workgroups of an instance, at most (flags)
-constexpr int64_t RES_LDS = 150 * 1024;               // dynamic LDS of a workgroup, of 160 KB
-
-// doubles from one workgroup block's slot to the next: packed slots share lines that all poll while they are written
-constexpr int RES_PAD = 2;
-
-// sentinel of the exchange slots: a NaN no sum produces (a NaN sum is stored as the default NaN)
-constexpr unsigned long long RES_EMPTY = 0x7ff8dead00000001ull;
-
-__device__ __forceinline__ void slot_store(double* p, double v)
-{
-  unsigned long long u = (unsigned long long)__double_as_longlong(v);
-  if (v != v)
-    u = 0x7ff8000000000000ull;
-  __hip_atomic_store(reinterpret_cast<unsigned long long*>(p), u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void slot_clear(double* p)
-{
-  __hip_atomic_store(reinterpret_cast<unsigned long long*>(p), RES_EMPTY, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ unsigned long long slot_load(const double* p)
-{
-  return __hip_atomic_load(reinterpret_cast<const unsigned long long*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-// limit of a wait: over() after each failed look, true when the wait is to end (its limit is reached, or another
-// workgroup gave up).  The first looks follow each other at once; later ones sleep and watch the clock.
-struct Patience {
-  int looks = 0;
-  long long since = 0;
-  __device__ __forceinline__ bool over(int* gave_up, int64_t ticks)
-  {
-    if (++looks < 256)
-      return false;
-    __builtin_amdgcn_s_sleep(2);
-    if (looks == 256)
-      since = wall_clock64();
-    if (looks & 255)
-      return false;
-    if (!__hip_atomic_load(gave_up, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) && wall_clock64() - since <= ticks)
-      return false;
-    __hip_atomic_store(gave_up, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    return true;
-  }
-};
-
-// a value that is the same in all lanes, as a scalar
-__device__ __forceinline__ int uniform(int v)
-{
-  return __builtin_amdgcn_readfirstlane(v);
-}
-
-// element `i` of an array whose base is the same for the whole wave: a 32-bit byte offset per lane
-template <class T>
-__device__ __forceinline__ T* at(T* base, unsigned i)
-{
-  return reinterpret_cast<T*>(reinterpret_cast<char*>(const_cast<std::remove_const_t<T>*>(base)) + i * unsigned(sizeof(T)));
-}
-
-// sums of `count` partials of NV values as Partials::sum adds them (lane t of `block` lanes adds the partials t,
-// t + block, ...; then the waves' butterflies; then the waves in order), in every lane.  Partials come from the
-// exchange slots, or (one workgroup, at most `block` partials: own) from the lane that computed them.  false:
-// gave up.  One barrier; red is not written again before a later barrier.
-template <int NV, int NW>
-__device__ __forceinline__ bool exchange_sum(const double* slots, const double (&own)[NV], bool alone, int count,
-                                             int block, double (*red)[RES_WAVES], int* failed, int* gave_up,
-                                             int64_t ticks, double (&tot)[NV])
-{
-  const int t = threadIdx.x;
-#pragma unroll
-  for (int k = 0; k < NV; ++k)
-    tot[k] = 0.;
-  if (alone) {
-    if (t < count)
-#pragma unroll
-      for (int k = 0; k < NV; ++k)
-        tot[k] += own[k];
-  } else if (t < block) {
-    for (int b = t; b < count; b += block) {
-      unsigned long long u[NV];
-      Patience wait;
-      while (true) {
-        bool empty = false;
-#pragma unroll
-        for (int k = 0; k < NV; ++k)
-          u[k] = slot_load(at(slots, unsigned(b) * RES_PAD + k));
-#pragma unroll
-        for (int k = 0; k < NV; ++k)
-          empty = empty || u[k] == RES_EMPTY;
-        if (!empty)
-          break;
-        if (wait.over(gave_up, ticks)) {
-          *failed = 1;
-          break;
-        }
-      }
-      if (*failed)
-        break;
-#pragma unroll
-      for (int k = 0; k < NV; ++k)
-        tot[k] += __longlong_as_double((long long)u[k]);
-    }
-  }
-#pragma unroll
-  for (int k = 0; k < NV; ++k) {
-    const double w = wave_sum(tot[k]); // (0 in the waves past `block`: added below without a change)
-    if ((t & 63) == 0)
-      red[k][t >> 6] = w;
-  }
-  __syncthreads();
-  if (uniform(*failed))
-    return false;
-#pragma unroll
-  for (int k = 0; k < NV; ++k) {
-    double s = 0.;
-#pragma unroll
-    for (int w = 0; w < NW; ++w)
-      s += red[k][w];
-    tot[k] = s;
-  }
-  return true;
-}
-
 constexpr bool q_in_lds(int slots, int nu, bool far)
 {
   return far || slots > 8 || (slots == 8 && nu == 4);
-}
-
-// g consecutive LDS values added in order (g a power of two up to 16), four loads at a time
-__device__ __forceinline__ double add_run(const double* v, int g)
-{
-  double s = 0.;
-  if (g == 1)
-    return s + v[0];
-  if (g == 2)
-    return s + v[0] + v[1];
-  for (int w = 0; w < g; w += 4) {
-    const double a = v[w], b = v[w + 1], c = v[w + 2], d = v[w + 3];
-    s += a, s += b, s += c, s += d;
-  }
-  return s;
 }
 
 // PCG of the tasks of one workgroup, one after the other.  Lane t holds rows t, t + T, ... of the workgroup,
@@ -272,7 +129,7 @@ __global__ void __launch_bounds__(T) k_pcg_resident(ResidentParams P)
       if constexpr (!XMEM)
         x[s] = in ? P.x[i] : 0.;
       else if (in)
-        P.x_work[i] = P.x[i];
+        P.x_out[i] = P.x[i];
       if constexpr (SELL) {
         width[s] = 0;
         if constexpr (KEEP != 0)
@@ -668,11 +525,11 @@ __global__ void __launch_bounds__(T) k_pcg_resident(ResidentParams P)
         double xv[S];
 #pragma unroll
         for (int s = 0; s < S; ++s)
-          xv[s] = *at(P.x_work + K.row0, unsigned(min(l + s * T, rows - 1)));
+          xv[s] = *at(P.x_out + K.row0, unsigned(min(l + s * T, rows - 1)));
 #pragma unroll
         for (int s = 0; s < S; ++s)
           if (l + s * T < rows)
-            *at(P.x_work + K.row0, unsigned(l + s * T)) = fma(alpha, pt[s * T], xv[s]);
+            *at(P.x_out + K.row0, unsigned(l + s * T)) = fma(alpha, pt[s * T], xv[s]);
       } else {
 #pragma unroll
         for (int s = 0; s < S; ++s)
@@ -709,15 +566,16 @@ __global__ void __launch_bounds__(T) k_pcg_resident(ResidentParams P)
 #pragma unroll
     for (int s = 0; s < S; ++s) {
       const int o = t + s * T;
-      if (o < rows)
-        P.x[K.row0 + o] = XMEM ? P.x_work[K.row0 + o] : x[XMEM ? 0 : s];
+      if (!XMEM && o < rows)
+        P.x_out[K.row0 + o] = x[XMEM ? 0 : s];
     }
     if (K.rank == 0 && t == 0) {
-      PcgScalars* D = P.S + K.inst;
-      D->rz = rn[0], D->rr = rn[1], D->beta = beta, D->alpha = alpha, D->alpha_prev = alpha, D->pq = pq;
-      D->iters = begun;
-      D->done = state;
-      D->brk = 0;
+      PcgScalars D = P.S[K.inst];
+      D.rz = rn[0], D.rr = rn[1], D.beta = beta, D.alpha = alpha, D.alpha_prev = alpha, D.pq = pq;
+      D.iters = begun;
+      D.done = state;
+      D.brk = 0;
+      P.S[P.ninst + K.inst] = D;
     }
   }
 }
@@ -857,15 +715,10 @@ static bool enough_rows(int64_t rows, int slots, int cus, bool sell)
   return slots == 1 ? w <= 1 : slots == 2 ? w <= (rows <= 4 * RES_LANES ? 1 : cus / 8) : slots == 4 ? w <= cus / 4 : w <= cus;
 }
 
-// Instances of a batch in the order of their size, each on the workgroups that are free first: the estimated time until
-// the last one ends, and (order, groups) which instance is next and on which workgroups.  A workgroup takes its instances
-// in this order, so the first unfinished one always has all of its workgroups.  Negative: an instance does not fit.
-static double schedule(const std::vector<int64_t>& row0, int slots, int lanes, int cus, std::vector<int>* order,
-                       std::vector<std::vector<int>>* groups)
+double resident_schedule(const std::vector<int64_t>& row0, const std::vector<int>& teams, double step,
+                         std::vector<int>* order, std::vector<std::vector<int>>* groups)
 {
-  // us per iteration of one workgroup with 1, 2, 4, 8, 16 rows per lane (measured), and of the exchanges
-  const double step = slots == 1 ? 1.8 : slots == 2 ? 2.1 : slots == 4 ? 2.7 : slots == 8 ? 4.3 : 10.;
-  const int ninst = int(row0.size()) - 1;
+  const int cus = device_cus(), ninst = int(teams.size());
   std::vector<int> by_size(ninst);
   for (int i = 0; i < ninst; ++i)
     by_size[i] = i;
@@ -878,13 +731,14 @@ static double schedule(const std::vector<int64_t>& row0, int slots, int lanes, i
     groups->assign(ninst, {});
   double last = 0.;
   for (int i : by_size) {
-    const int64_t n = row0[i + 1] - row0[i], team = team_of(n, slots, lanes);
+    const int team = teams[i];
     if (team > cus || team > RES_MAX_GROUPS)
       return -1.;
     std::partial_sort(load.begin(), load.begin() + team, load.end());
     // iterations grow like the square root of the size (two dimensions)
-    const double end = load[team - 1].first + std::sqrt(double(n)) * (step + (team > 1 ? 2.6 + 0.01 * double(team) : 0.));
-    for (int64_t k = 0; k < team; ++k) {
+    const double end = load[team - 1].first +
+                       std::sqrt(double(row0[i + 1] - row0[i])) * (step + (team > 1 ? 2.6 + 0.01 * double(team) : 0.));
+    for (int k = 0; k < team; ++k) {
       load[k].first = end;
       if (groups)
         (*groups)[i].push_back(load[k].second);
@@ -894,6 +748,12 @@ static double schedule(const std::vector<int64_t>& row0, int slots, int lanes, i
   if (order)
     *order = by_size;
   return last;
+}
+
+// us per iteration of one workgroup with 1, 2, 4, 8, 16 rows per lane (measured)
+static double step_of(int slots)
+{
+  return slots == 1 ? 1.8 : slots == 2 ? 2.1 : slots == 4 ? 2.7 : slots == 8 ? 4.3 : 10.;
 }
 
 // rows per lane: -1 when no choice of `fits` (LDS, compiled variant) takes all instances
@@ -909,7 +769,10 @@ static int choose_slots(const std::vector<int64_t>& row0, bool sell, F fits)
         return s;
       continue;
     }
-    const double t = schedule(row0, s, RES_LANES, cus, nullptr, nullptr);
+    std::vector<int> teams;
+    for (size_t i = 0; i + 1 < row0.size(); ++i)
+      teams.push_back(int(std::min<int64_t>(team_of(row0[i + 1] - row0[i], s), 1 << 20)));
+    const double t = resident_schedule(row0, teams, step_of(s), nullptr, nullptr);
     if (t >= 0. && (best < 0 || t < time) && fits(s))
       best = s, time = t;
   }
@@ -996,12 +859,14 @@ static bool list_tasks(const Operator& op, int slots, int lanes, std::vector<Res
   return true;
 }
 
-// the tasks (instance by instance) in the order in which the workgroups take them
-static void finish_plan(ResidentPlan& plan, const Operator& op, const std::vector<ResidentTask>& tasks, int64_t lds)
+void resident_finish(ResidentPlan& plan, const Operator& op, const std::vector<ResidentTask>& tasks, int64_t lds,
+                     int64_t n_a, int64_t n_v)
 {
-  std::vector<int> order;
+  std::vector<int> order, teams(op.space->inst_dof.size() - 1, 0);
   std::vector<std::vector<int>> groups;
-  if (schedule(op.space->inst_dof, plan.slots, plan.lanes, device_cus(), &order, &groups) < 0.)
+  for (const auto& K : tasks)
+    teams[K.inst] = K.team;
+  if (resident_schedule(op.space->inst_dof, teams, plan.step, &order, &groups) < 0.)
     return;
   std::vector<int64_t> first(groups.size(), 0); // first task of every instance
   for (size_t k = tasks.size(); k-- > 0;)
@@ -1030,7 +895,8 @@ static void finish_plan(ResidentPlan& plan, const Operator& op, const std::vecto
   plan.grid = int(of.size()), plan.lds = lds;
   plan.tasks.upload(list);
   plan.task_start.upload(start);
-  plan.exchange.allocate(size_t(RES_PAD * (3 * op.fmt.A.nblocks + 2 * op.fmt.V.nblocks)));
+  plan.n_a = n_a, plan.n_v = n_v;
+  plan.exchange.allocate(size_t(RES_PAD * (3 * n_a + 2 * n_v)));
   plan.gave_up.allocate(1 + RES_MAX_GROUPS);
   if (!plan.host_gave_up)
     HGDT_HIP(hipHostMalloc((void**)&plan.host_gave_up, sizeof(int)));
@@ -1043,7 +909,7 @@ void resident_plan_dia(ResidentPlan& plan, const Operator& op, const std::vector
   plan.usable = false;
   const SolverFormat& F = op.fmt;
   const int bv = F.V.block, iv = F.V.items, ba = F.A.block * F.A.items;
-  plan.sell = plan.far = false;
+  plan.sell = plan.far = plan.dg = false;
   plan.lanes = RES_LANES;
   if (bv == RES_FAR_BLOCK && iv == 4 && F.A.block == bv && F.A.items == iv) {
     const int slots = far_slots(op.space->inst_dof, s_offs, s_nu);
@@ -1053,7 +919,8 @@ void resident_plan_dia(ResidentPlan& plan, const Operator& op, const std::vector
     plan.far = true;
     plan.lanes = RES_FAR_BLOCK;
     plan.slots = slots, plan.lg_items = 2, plan.same_blocks = true, plan.nu = s_nu;
-    finish_plan(plan, op, tasks, far_lds(slots, s_offs[0][1]));
+    plan.step = step_of(plan.slots);
+    resident_finish(plan, op, tasks, far_lds(slots, s_offs[0][1]), F.A.nblocks, F.V.nblocks);
     return;
   }
   const bool same = bv == RES_LANES && F.A.block == bv && F.A.items == iv;
@@ -1077,7 +944,8 @@ void resident_plan_dia(ResidentPlan& plan, const Operator& op, const std::vector
   if (!list_tasks(op, slots, RES_LANES, tasks))
     return;
   plan.slots = slots, plan.lg_items = lg, plan.same_blocks = same, plan.nu = s_nu;
-  finish_plan(plan, op, tasks, lds_of(slots, reach, s_nu));
+  plan.step = step_of(plan.slots);
+  resident_finish(plan, op, tasks, lds_of(slots, reach, s_nu), F.A.nblocks, F.V.nblocks);
 }
 
 // columns of the rows [r0, r1) that lie outside them, ascending
@@ -1186,17 +1054,20 @@ void resident_plan_sell(ResidentPlan& plan, const Operator& op)
     rows.push_back(0);
   plan.halo_rows.upload(rows);
   plan.publish.upload(pub);
-  plan.sell = true, plan.far = false;
+  plan.sell = true, plan.far = plan.dg = false;
   plan.lanes = RES_LANES;
   int64_t widest = 1;
   for (int64_t k = 0; k < F.nslices; ++k)
     widest = std::max(widest, (slice_ptr[k + 1] - slice_ptr[k]) / 64);
   plan.slots = slots, plan.lg_items = lg, plan.same_blocks = true, plan.nu = -int(std::min<int64_t>(widest, 1 << 20));
-  finish_plan(plan, op, tasks, (R + most) * int64_t(sizeof(double)));
+  plan.step = step_of(plan.slots);
+  resident_finish(plan, op, tasks, (R + most) * int64_t(sizeof(double)), F.A.nblocks, F.V.nblocks);
 }
 
-bool resident_run(ResidentPlan& plan, ResidentParams P, hipStream_t stream, PcgScalars* host_records)
+bool resident_run(ResidentPlan& plan, ResidentParams P, const MfParams& M, hipStream_t stream, PcgScalars* host_records)
 {
+  P.n_a = plan.n_a, P.n_v = plan.n_v;
+  P.dg_elements = plan.elements.ptr, P.zero_place = plan.zero_place;
   P.g1 = plan.exchange.ptr;
   P.g2 = plan.exchange.ptr + 3 * P.n_a * RES_PAD;
   P.sell_local = plan.sell_local.ptr, P.halo_rows = plan.halo_rows.ptr, P.publish = plan.publish.ptr;
@@ -1204,9 +1075,11 @@ bool resident_run(ResidentPlan& plan, ResidentParams P, hipStream_t stream, PcgS
   P.wait_ticks = int64_t(4) * 100000000; // 4 s
   const int64_t nx = int64_t(plan.exchange.count);
   hipLaunchKernelGGL(k_resident_clear, dim3(xcd_grid(std::max<int64_t>(std::max(P.n, nx), RES_MAX_GROUPS), 256)), dim3(256), 0, stream, P, nx);
-  const Kernel k = plan.far ? far_kernel(plan.slots) : kernel_of(plan.slots, plan.lg_items, P.same_blocks, plan.nu);
-  HGDT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
-                               int(RES_LDS)));
+  const void* const k = plan.dg ? resident_dg_kernel(plan)
+                                : reinterpret_cast<const void*>(plan.far ? far_kernel(plan.slots)
+                                                                         : kernel_of(plan.slots, plan.lg_items,
+                                                                                     P.same_blocks, plan.nu));
+  HGDT_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, int(RES_LDS)));
   int dev = 0;
   HGDT_HIP(hipGetDevice(&dev));
   struct Hold {
@@ -1219,12 +1092,13 @@ bool resident_run(ResidentPlan& plan, ResidentParams P, hipStream_t stream, PcgS
   const int cus = device_cus(), held = std::min(plan.grid, cus);
   CuBudget::get().take(dev, held, cus);
   Hold hold{dev, held};
-  hipLaunchKernelGGL(k, dim3(unsigned(plan.grid)), dim3(unsigned(plan.lanes)), size_t(plan.lds), stream, P);
-  hipError_t e = hipGetLastError();
+  MfParams Mk = M;
+  void* args[2] = {&P, &Mk}; // (the second: discontinuous spaces)
+  hipError_t e = hipLaunchKernel(k, dim3(unsigned(plan.grid)), dim3(unsigned(plan.lanes)), args, size_t(plan.lds), stream);
   if (e == hipSuccess)
     e = hipMemcpyAsync(plan.host_gave_up, plan.gave_up.ptr, sizeof(int), hipMemcpyDeviceToHost, stream);
   if (e == hipSuccess)
-    e = hipMemcpyAsync(host_records, P.S, sizeof(PcgScalars) * P.ninst, hipMemcpyDeviceToHost, stream);
+    e = hipMemcpyAsync(host_records, P.S + P.ninst, sizeof(PcgScalars) * P.ninst, hipMemcpyDeviceToHost, stream);
   const hipError_t e2 = hipStreamSynchronize(stream); // also after an error: the CUs are given back with none running
   HGDT_HIP(e);
   HGDT_HIP(e2);

@@ -1,9 +1,10 @@
-// resident.hpp -- PCG solves whose vectors stay on the chip (resident.hip).
+// resident.hpp -- PCG solves whose vectors stay on the chip (resident.hip; discontinuous spaces: resident_dg.hip).
 #pragma once
 
 #include <memory>
 
 #include "hgdt_internal.hpp"
+#include "mf_params.hpp"
 
 namespace hgdt {
 
@@ -49,16 +50,26 @@ struct ResidentParams {
   const uint16_t* sell_local;
   const int32_t* halo_rows;
   const uint32_t* publish; // per workgroup and lane: the slots whose rows other workgroups read
+  // discontinuous spaces: elements of a workgroup, in order (-1: none; bit 30: read by other workgroups), place of the zeros
+  // in p; the scaled element blocks as the storage has them; reference data of the matrix-free operator
+  const int32_t* dg_elements;
+  int zero_place;
+  int blk_mn, blk_sym;
+  int64_t blk_ne;
+  const int32_t* blk_nb;
+  const int32_t* blk_mir;
+  const double* dg_ref;
+  const double* dh;
   const double* dsq;
   const double* r;     // r of the initial residual (not written: a solve that gives up leaves it to the caller)
-  double* x;           // scaled iterate: read at the start, written by the instances that end
-  double* x_work;      // the iterate of workgroups that do not hold it in registers
+  const double* x;     // scaled iterate at the start
+  double* x_out;       // and at the end (until then the iterate of workgroups that do not hold it in registers)
   double* r_pub[2];    // rows of r that other workgroups of the team read, by parity of the step
   const double* part2; // partials of the initial residual, 2 per vector block
   double* g1;          // 2 x (operator blocks), padded: partials of p.q, by parity of the step
   double* g2;          // behind it, 2 x (vector blocks), padded: partials of the two residual norms
   int64_t n_a, n_v;    // operator / vector blocks of all instances
-  PcgScalars* S;       // record of every instance: tolerance read, result written
+  PcgScalars* S;       // records of the instances: tolerances read; the results go to the ninst records behind these
   int64_t max_iter;
   const ResidentTask* tasks;
   const int32_t* task_start; // per workgroup
@@ -78,8 +89,12 @@ struct ResidentPlan {
   int workgroups = 0;   // with rows; the grid is rounded up to the 8 XCDs
   int grid = 0;
   int64_t lds = 0;
-  bool sell = false, far = false;
+  bool sell = false, far = false, dg = false, matrix_free = false; // (dg: slots are elements per lane)
   int lanes = RES_BLOCK;
+  double step = 0.;         // estimate of one iteration of a workgroup
+  int zero_place = 0;
+  int64_t n_a = 0, n_v = 0; // partials of the two exchanges
+  DeviceArray<int32_t> elements;
   DeviceArray<uint16_t> sell_local;
   DeviceArray<int32_t> halo_rows;
   DeviceArray<uint32_t> publish;
@@ -106,8 +121,20 @@ void resident_plan_dia(ResidentPlan& plan, const Operator& op, const std::vector
 // the same for SELL storage (general meshes): rows per lane, and the plan
 int resident_items_sell(const Operator& op);
 void resident_plan_sell(ResidentPlan& plan, const Operator& op);
-// runs the solve; false when it gave up (then nothing but r_pub and the exchange buffers was written for the
-// instances without a result: the caller goes on with one launch per kernel).  Waits for the kernel.
-bool resident_run(ResidentPlan& plan, ResidentParams P, hipStream_t stream, PcgScalars* host_records);
+// discontinuous spaces of 4 DoFs per element: element blocks, or matrix-free (whatever the launch shapes are)
+void resident_plan_dg(ResidentPlan& plan, const Operator& op);
+const void* resident_dg_kernel(const ResidentPlan& plan);
+// Instances of a batch in the order of their size, each on the workgroups that are free first, `teams[i]` of them: the
+// estimated time until the last one ends, and (order, groups) which instance is next and on which workgroups.  A workgroup
+// takes its instances in this order, so the first unfinished one always has all of its workgroups.  step: us per iteration
+// of one workgroup.  Negative: an instance does not fit.
+double resident_schedule(const std::vector<int64_t>& row0, const std::vector<int>& teams, double step,
+                         std::vector<int>* order, std::vector<std::vector<int>>* groups);
+// the tasks (instance by instance) in the order in which the workgroups take them; buffers of the exchanges
+void resident_finish(ResidentPlan& plan, const Operator& op, const std::vector<ResidentTask>& tasks, int64_t lds,
+                     int64_t n_a, int64_t n_v);
+// runs the solve; false when it gave up (then nothing but r_pub, x_out, the results' records and the exchange buffers was
+// written: the caller goes on with one launch per kernel).  Waits for the kernel.  M: the matrix-free operator.
+bool resident_run(ResidentPlan& plan, ResidentParams P, const MfParams& M, hipStream_t stream, PcgScalars* host_records);
 
 } // namespace hgdt

@@ -950,11 +950,11 @@ __global__ void __launch_bounds__(1024) k_cg_update(PcgParams P, int par)
 }
 
 // x = D^{-1/2} xh after the last step
-__global__ void k_cg_finish(int64_t n, const double* __restrict__ dh, double* __restrict__ x)
+__global__ void k_cg_finish(int64_t n, const double* __restrict__ dh, const double* xh, double* x)
 {
   const int64_t i = xcd_index(n);
   if (i < n)
-    x[i] = dh[i] * x[i];
+    x[i] = dh[i] * xh[i];
 }
 
 // true residual at exit, on the vector row partition: block partials of |b - A x|^2 with ax = A x computed
@@ -1384,6 +1384,10 @@ struct SolverCache {
   ResidentPlan resident;
   int64_t scaled_pad = 0;   // doubles ahead of the scaled matrix in its storage (and past it)
   ResidentShape shaped_for; // resident_shape of the row partitions
+  // resident_shape_dia of these offsets
+  ResidentShape shape_dia;
+  std::vector<std::vector<int64_t>> shape_offs;
+  int shape_nu = -1;
   int sell_items = 0; // SELL: rows per lane that suit a solve in one launch (0: none)
   ~SolverCache()
   {
@@ -1478,14 +1482,16 @@ static int kernel_format(const Operator& op);
 // caller chose shapes, or the storage (once it is known) or size does not fit
 static ResidentShape resident_shape(const Operator& op)
 {
-  const SolverCache& C = *op.solver_cache;
+  SolverCache& C = *op.solver_cache;
   if (op.launch[3].user || op.launch[4].user || !op.square())
     return {};
   if (op.fmt.format == HGDT_FORMAT_SELL && op.fmt.structure_ready)
     return C.sell_items ? ResidentShape{RES_BLOCK, C.sell_items} : ResidentShape{};
   if (!op.fmt.valid || op.fmt.format != HGDT_FORMAT_DIA || kernel_format(op) != FMT_DIAS)
     return {};
-  return resident_shape_dia(op.space->inst_dof, C.s_offs, C.s_nu);
+  if (C.s_nu != C.shape_nu || C.s_offs != C.shape_offs) // (a batch's shape is a search over its instances)
+    C.shape_dia = resident_shape_dia(op.space->inst_dof, C.s_offs, C.s_nu), C.shape_offs = C.s_offs, C.shape_nu = C.s_nu;
+  return C.shape_dia;
 }
 
 // row-block partitions of the operator (host set-up, O(number of blocks))
@@ -2431,6 +2437,8 @@ static ResidentPlan& resident_plan(Operator& op)
       resident_plan_dia(plan, op, C.s_offs, C.s_nu);
     else if (op.fmt.format == HGDT_FORMAT_SELL)
       resident_plan_sell(plan, op);
+    else if (kernel_format(op) == FMT_BLK || (op.fmt.format == HGDT_FORMAT_MATRIX_FREE && op.fmt.mf_kind == MFK_DG_QUAD))
+      resident_plan_dg(plan, op);
     plan.version = C.version;
   }
   return plan;
@@ -2445,10 +2453,12 @@ static bool resident_solve(Operator& op, const PcgParams& P, hipStream_t stream)
   R.a_rows = F.A.block * F.A.items, R.v_block = F.V.block;
   R.same_blocks = C.resident.same_blocks;
   R.s_nu = P.s_nu, R.s_off = P.s_off, R.scaled = P.scaled, R.dsq = P.dsq, R.slice_ptr = P.slice_ptr;
-  R.r = P.r, R.x = P.x, R.x_work = P.q, R.r_pub[0] = P.p, R.r_pub[1] = P.p2, R.part2 = P.part2;
-  R.n_a = F.A.nblocks, R.n_v = F.V.nblocks;
+  R.blk_ne = P.blk_ne, R.blk_mn = P.blk_mn, R.blk_sym = F.symmetric, R.blk_nb = P.blk_nb, R.blk_mir = P.blk_mir;
+  R.dg_ref = F.d_mf_ref.ptr, R.dh = P.dh;
+  R.r = P.r, R.x = P.x, R.x_out = P.q, R.r_pub[0] = P.p, R.r_pub[1] = P.p2, R.part2 = P.part2;
   R.S = P.S, R.max_iter = P.max_iter;
-  return resident_run(C.resident, R, stream, C.host_scalars[0]);
+  return resident_run(C.resident, R, F.format == HGDT_FORMAT_MATRIX_FREE ? mf_params(op) : MfParams{}, stream,
+                      C.host_scalars[0]);
 }
 
 void Operator::apply_inverse(const double* b, double* x, const hgdt_solver_options& opt, hgdt_solver_stats& st,
@@ -2674,7 +2684,8 @@ void Operator::apply_inverse(const double* b, double* x, const hgdt_solver_optio
     for (int i = 0; i < ninst; ++i)
       compactions += C.host_scalars[0][i].iters < most;
   }
-  hipLaunchKernelGGL(k_cg_finish, dim3(blocks_for(n, 256)), dim3(256), 0, stream, n, fmt.d_dh.ptr, x);
+  hipLaunchKernelGGL(k_cg_finish, dim3(blocks_for(n, 256)), dim3(256), 0, stream, n, fmt.d_dh.ptr,
+                     solved ? d_q.ptr : x, x);
   HGDT_HIP(hipGetLastError());
   // true residual |b - A x| / |b| of every instance at exit, with the unscaled operator (one application and
   // one pass over b and A x, over all blocks whatever the narrowed launches held)

@@ -197,3 +197,106 @@ def test_batch_of_several_rounds(hgdt_mod):
     wg = _both(H, op)
     print(f"  {space.num_DoFs} DoFs, {wg} workgroups")
     assert 0 < wg <= 256 and space.num_DoFs > 8192 * 200
+
+
+def _swipdg(H, grid, kappa, omega=None, mass=0.0, faces=True, fmt="auto"):
+    omega = kappa if omega is None else omega
+    space = H.DiscontinuousLagrangeSpace(grid, 1)
+    op = H.make_matrix_operator(space, H.Stencil.element_and_intersection if faces else H.Stencil.element)
+    op.append(H.LocalElementIntegralBilinearForm(H.LocalLaplaceIntegrand(kappa)))
+    if mass:
+        op.append(H.LocalElementIntegralBilinearForm(H.LocalProductIntegrand(mass)))
+    if faces:
+        op.append(H.LocalCouplingIntersectionIntegralBilinearForm(
+            H.LocalLaplaceIPDGInnerCoupling(1.0, kappa, omega) + H.LocalIPDGInnerPenalty(16.0, omega)), {},
+            H.ApplyOn.InnerIntersectionsOnce())
+        op.append(H.LocalIntersectionIntegralBilinearForm(
+            H.LocalIPDGBoundaryPenalty(16.0, omega) + H.LocalLaplaceIPDGDirichletCoupling(1.0, kappa)), {},
+            H.ApplyOn.CustomBoundaryIntersections(H.AllDirichletBoundaryInfo()))
+    rhs = H.make_vector_functional(space)
+    rhs.append(H.LocalElementIntegralFunctional(H.LocalProductIntegrand().with_ansatz(1.0)))
+    op.append(rhs)
+    op.set_format(fmt)
+    op.assemble()
+    return space, op
+
+
+def _same_steps(H, space, op, limits=(1, 2, 3, 8)):
+    """the iterates of both ways after a few steps: the same sums in another order, so that alpha and beta differ by the
+    round-off of sums of up to a million terms (1e-13) and the iterate by a small multiple: bound 1e-11"""
+    wg = None
+    for limit in limits:
+        xs = []
+        for spmv in (0, 8):
+            x = torch.zeros(space.num_DoFs, dtype=torch.float64, device="cuda")
+            try:
+                op.apply_inverse("rhs", x, opts={"max_iter": limit}, time_spmv=spmv)
+            except H.linear_solver_failed:
+                assert op.last_solve["iterations"] == limit
+            wg = op.solve_workgroups() if spmv == 0 else wg
+            xs.append(x)
+        assert float((xs[0] - xs[1]).norm()) <= 1e-11 * float(xs[1].norm()), limit
+    return wg
+
+
+@pytest.mark.parametrize("cells,blocks,matrix_free", [
+    ([1, 1], 1, 1), ([2, 3], 1, 1), ([32, 16], 1, 1), ([23, 23], 2, 2), ([1, 700], 2, 2), ([700, 1], 2, 2),
+    ([33, 65], 5, 5), ([131, 97], None, None), ([256, 192], 96, 96), ([362, 361], 0, None), ([512, 512], 0, 256),
+    ([513, 512], 0, 0)])
+@pytest.mark.parametrize("fmt", ["auto", "matrix_free"])
+def test_discontinuous_spaces(hgdt_mod, cells, blocks, matrix_free, fmt):
+    print(f"case swipdg {fmt} {cells}", flush=True)
+    H = hgdt_mod
+    grid = H.Grid.structured("quad", [0, 0], [cells[0] / 100, 0.7 * cells[1] / 100], cells)
+    kappa = torch.from_numpy(H.fields.lognormal(21, grid.num_elements)).cuda()
+    omega = kappa * (1.0 + torch.from_numpy(H.fields.uniform(22, grid.num_elements)).cuda())  # (coercive: a penalty >= kappa's)
+    space, op = _swipdg(H, grid, kappa, omega, mass=3.0 if cells[0] % 2 else 0.0, fmt=fmt)
+    wg = _same_steps(H, space, op)
+    print(f"  {space.num_DoFs} DoFs, {wg} workgroups")
+    want = blocks if fmt == "auto" else matrix_free
+    assert (wg > 0) if want is None else wg == want
+    if space.num_DoFs < 20000:
+        x = op.apply_inverse("rhs")
+        assert op.last_solve["true_relres"] <= 2e-10
+        again = op.apply_inverse("rhs", use_graph=True)
+        assert torch.equal(x, again)
+
+
+@pytest.mark.parametrize("fmt", ["auto", "matrix_free"])
+def test_discontinuous_batch(hgdt_mod, fmt):
+    """instances of one workgroup and of several, more than fit at once: each with the bits of its own solve (whose first
+    residual is summed over the same row blocks)"""
+    print(f"case swipdg batch {fmt}", flush=True)
+    H = hgdt_mod
+    sizes = [3, 40, 1, 150, 64, 23] + [100] * 14
+    parts = [H.Grid.structured("quad", [0, 0], [1, 1 + 0.1 * (i % 3)], [m, m + 1]) for i, m in enumerate(sizes)]
+    union = H.Grid.union(parts)
+    kappa = torch.from_numpy(H.fields.lognormal(23, union.num_elements)).cuda()
+    space, op = _swipdg(H, union, kappa, fmt=fmt)
+    x = op.apply_inverse("rhs", opts={"precision": 1e-6})
+    assert op.solve_workgroups() > 0
+    its = op.instance_stats()[0]
+    first = np.cumsum([0] + [m * (m + 1) for m in sizes])
+    for i in (0, 1, 2, 3, 5, 19):
+        s1, op1 = _swipdg(H, parts[i], kappa[int(first[i]):int(first[i + 1])].contiguous(), fmt=fmt)
+        for k in (3, 4):
+            op1.set_launch(k, *op.get_launch(k))
+        x1 = op1.apply_inverse("rhs", opts={"precision": 1e-6})
+        assert op1.solve_workgroups() > 0 and op1.last_solve["iterations"] == its[i]
+        assert torch.equal(x1, x[4 * int(first[i]):4 * int(first[i + 1])])
+
+
+def test_element_blocks_of_other_elements(hgdt_mod):
+    """simplices (4 neighbours anywhere), an operator without neighbours, and a start from a given iterate"""
+    print("case blocks of tets", flush=True)
+    H = hgdt_mod
+    # (without neighbours the solution is 1: the Laplace part of the product is nothing but round-off, which every step
+    # multiplies by its ratio to the mass, so only the first iterate is compared)
+    for geometry, cells, faces, limits in (("tet", [7, 6, 5], True, (1, 2, 5)), ("quad", [30, 31], False, (1,))):
+        grid = H.Grid.structured(geometry, [0.] * len(cells), [1.] * len(cells), cells)
+        kappa = torch.from_numpy(H.fields.lognormal(24, grid.num_elements)).cuda()
+        space, op = _swipdg(H, grid, kappa, mass=1.0, faces=faces)
+        assert _same_steps(H, space, op, limits) > 0
+        guess = torch.from_numpy(H.fields.uniform(8, space.num_DoFs)).cuda()
+        got = [op.apply_inverse("rhs", guess.clone(), opts={"initial_guess": True}, time_spmv=spmv) for spmv in (0, 8)]
+        assert float((got[0] - got[1]).norm()) <= 1e-8 * float(got[1].norm())
