@@ -942,6 +942,222 @@ __global__ void __launch_bounds__(256) k_inner_local(FaceParams P)
   }
 }
 
+// rows of a discontinuous operator with symmetric forms and at most 4 DoFs and faces per element, from its intersections
+// straight to the CSR values: one lane per (element, face), the 4 lanes of an element side by side.  A lane evaluates its
+// intersection's own block (upper triangle) and its block with the neighbour; the own blocks are added to the staged
+// element and boundary blocks across the 4 lanes.  Both elements of an intersection evaluate it, in the same way (the
+// inside's frame, the in_out block, stored transposed by the outside): the matrix is symmetric bit for bit.
+// Against k_inner_local and k_gather_values this evaluates every intersection twice, but needs 52 registers for
+// accumulators instead of 128 (2 waves per SIMD instead of 1) and neither writes and reads back the blocks of the
+// intersections (512 bytes each) nor reads a list of contributions (4 bytes each).  P1 on 82 944 tetrahedra (6.4 million
+// entries): 77 + 58 us -> 54 us.  Bound by the arithmetic and by chains of loads that two waves per SIMD do not hide.
+struct DgRows {
+  int64_t ne;
+  const int32_t* code;
+  const int64_t* row0;
+  const double* staging;
+  int64_t bnd_base;
+  int has_element, has_boundary; // staged element / boundary blocks
+  double* values;
+};
+
+// value of lane K of the 4 lanes of an element, in all of them
+template <int K>
+__device__ __forceinline__ int lane_of_4(int v)
+{
+  return __builtin_amdgcn_update_dpp(0, v, K * 0x55, 0xf, 0xf, true);
+}
+template <int K>
+__device__ __forceinline__ double lane_of_4(double v)
+{
+  return __hiloint2double(lane_of_4<K>(__double2hiint(v)), lane_of_4<K>(__double2loint(v)));
+}
+
+template <int GEOM>
+__global__ void __launch_bounds__(256) k_dg_rows(FaceParams P, DgRows R)
+{
+  using T = Traits<GEOM>;
+  constexpr int D = T::D, ND = Basis<GEOM, 1>::ND, NF = T::SIMPLEX ? D + 1 : 2 * D;
+  constexpr int NU = ND * (ND + 1) / 2;
+  static_assert(ND <= 4 && NF <= 4, "one lane per face, 4 lanes per element");
+  const int64_t t = xcd_index(4 * R.ne);
+  if (t >= 4 * R.ne) // (whole elements)
+    return;
+  const int64_t E = t >> 2;
+  const int f = int(t & 3);
+  const int32_t code = f < NF ? R.code[E * NF + f] : ScatterMaps::NO_FACE;
+  const bool outside = code & 1;
+  double own[NU], C[ND][ND]; // own block; in_out block (rows of the inside)
+#pragma unroll
+  for (int k = 0; k < NU; ++k)
+    own[k] = 0.;
+#pragma unroll
+  for (int i = 0; i < ND; ++i)
+#pragma unroll
+    for (int j = 0; j < ND; ++j)
+      C[i][j] = 0.;
+  int nbr = -1;
+  if (code >= 0) {
+    const int64_t fi = code >> 1;
+    const int64_t e = P.faces[4 * fi + 0], o = P.faces[4 * fi + 2];
+    nbr = int(outside ? e : o);
+    Geo<D> gin, gout;
+    load_geometry<GEOM>(P.coords, P.conn, e, gin);
+    load_geometry<GEOM>(P.coords, P.conn, o, gout);
+    FaceFrame<D> F;
+    face_frame<GEOM>(P.coords, P.conn, e, P.faces[4 * fi + 1], F);
+    const double* n = F.n;
+    // simplices: the basis functions at a point of the face are the point's barycentric coordinates; which of them belongs
+    // to a vertex of the elements (3: none, the vertex is opposite to the face)
+    int win_at[ND], wout_at[ND];
+    if constexpr (T::SIMPLEX) {
+      const int fe = P.faces[4 * fi + 1];
+      int32_t v[3] = {-1, -1, -1};
+#pragma unroll
+      for (int k = 0; k < D; ++k)
+        v[k] = P.conn[e * T::NV + face_vertex<GEOM>(fe, k)];
+#pragma unroll
+      for (int i = 0; i < ND; ++i) {
+        const int32_t a = P.conn[e * T::NV + i], b = P.conn[o * T::NV + i];
+        win_at[i] = a == v[0] ? 0 : a == v[1] ? 1 : a == v[2] ? 2 : 3;
+        wout_at[i] = b == v[0] ? 0 : b == v[1] ? 1 : b == v[2] ? 2 : 3;
+      }
+    }
+    for (int fm = 0; fm < P.nforms; ++fm) {
+      const double kin = P.kappa[fm] ? P.kappa[fm][e] : P.kappa_value[fm];
+      const double kout = P.kappa[fm] ? P.kappa[fm][o] : P.kappa_value[fm];
+      const double win = P.omega[fm] ? P.omega[fm][e] : P.omega_value[fm];
+      const double wout = P.omega[fm] ? P.omega[fm][o] : P.omega_value[fm];
+      const double *Kin = tblock<D>(P.kappa_t[fm], e), *Kout = tblock<D>(P.kappa_t[fm], o);
+      const double *Win = tblock<D>(P.omega_t[fm], e), *Wout = tblock<D>(P.omega_t[fm], o);
+      const double sc = P.scaling[fm], prm = P.param[fm];
+      const QRule Q = P.rule[fm];
+      const double delta_plus = n_w_n<D>(n, wout, Wout);
+      const double delta_minus = n_w_n<D>(n, win, Win);
+      const bool coupling = P.kind[fm] == FF_INNER_COUPLING;
+      double fin[ND], fout[ND]; // (kappa grad phi) . n
+      double wm = 0., wp = 0., pen = 0.;
+      if (coupling) {
+        wm = delta_plus / (delta_plus + delta_minus);
+        wp = delta_minus / (delta_plus + delta_minus);
+        if constexpr (T::SIMPLEX) { // constant: gradient 1 + a is row a of the inverse Jacobian, and they add up to 0
+          fin[0] = fout[0] = 0.;
+#pragma unroll
+          for (int a = 0; a < D; ++a) {
+            fin[1 + a] = flux<D>(kin, gin.Ji[a], n, Kin);
+            fout[1 + a] = flux<D>(kout, gout.Ji[a], n, Kout);
+            fin[0] -= fin[1 + a], fout[0] -= fout[1 + a];
+          }
+        }
+      } else {
+        pen = (prm * ((delta_plus * delta_minus) / (delta_plus + delta_minus))) / F.h;
+      }
+      const double wo = outside ? wp : -1.0 * wm; // of the own block
+      for (int q = 0; q < Q.npts; ++q) {
+        double s, tt, wq;
+        face_qp<D - 1>(P.qtab, Q, q, s, tt, wq);
+        double pin[ND], pout[ND];
+        if constexpr (T::SIMPLEX) {
+          const double lam[3] = {D == 2 ? 1. - s : 1. - s - tt, s, tt};
+#pragma unroll
+          for (int i = 0; i < ND; ++i) {
+            pin[i] = win_at[i] == 0 ? lam[0] : win_at[i] == 1 ? lam[1] : win_at[i] == 2 ? lam[2] : 0.;
+            pout[i] = wout_at[i] == 0 ? lam[0] : wout_at[i] == 1 ? lam[1] : wout_at[i] == 2 ? lam[2] : 0.;
+          }
+        } else {
+          double X[D], Gin[ND][D], Gout[ND][D];
+          F.point(s, tt, X);
+          eval_at<GEOM, 1>(gin, X, pin, Gin);
+          eval_at<GEOM, 1>(gout, X, pout, Gout);
+#pragma unroll
+          for (int i = 0; i < ND; ++i) {
+            fin[i] = flux<D>(kin, Gin[i], n, Kin);
+            fout[i] = flux<D>(kout, Gout[i], n, Kout);
+          }
+        }
+        const double factor = F.ie * wq;
+        double ps[ND];
+#pragma unroll
+        for (int i = 0; i < ND; ++i)
+          ps[i] = outside ? pout[i] : pin[i];
+        if (coupling) {
+          double fs[ND];
+#pragma unroll
+          for (int i = 0; i < ND; ++i)
+            fs[i] = outside ? fout[i] : fin[i];
+#pragma unroll
+          for (int i = 0, k = 0; i < ND; ++i)
+#pragma unroll
+            for (int j = i; j < ND; ++j, ++k)
+              own[k] += sc * ((wo * fs[j] * ps[i] + prm * wo * ps[j] * fs[i]) * factor);
+#pragma unroll
+          for (int i = 0; i < ND; ++i)
+#pragma unroll
+            for (int j = 0; j < ND; ++j)
+              C[i][j] += sc * ((-1.0 * wp * fout[j] * pin[i] + prm * wm * pout[j] * fin[i]) * factor);
+        } else {
+#pragma unroll
+          for (int i = 0, k = 0; i < ND; ++i)
+#pragma unroll
+            for (int j = i; j < ND; ++j, ++k)
+              own[k] += sc * ((pen * ps[j] * ps[i]) * factor);
+#pragma unroll
+          for (int i = 0; i < ND; ++i)
+#pragma unroll
+            for (int j = 0; j < ND; ++j)
+              C[i][j] += sc * ((-1.0 * pen * pout[j] * pin[i]) * factor);
+        }
+      }
+    }
+  } else if (code != ScatterMaps::NO_FACE && R.has_boundary) {
+    const double* __restrict__ b = R.staging + R.bnd_base + int64_t(-1 - code) * (ND * ND);
+#pragma unroll
+    for (int i = 0, k = 0; i < ND; ++i)
+#pragma unroll
+      for (int j = i; j < ND; ++j, ++k)
+        own[k] = b[i * ND + j];
+  }
+  // ranks of the blocks in the rows
+  const int id[4] = {lane_of_4<0>(nbr), lane_of_4<1>(nbr), lane_of_4<2>(nbr), lane_of_4<3>(nbr)};
+  int blocks = 1, rank_own = 0, rank = int(E) < nbr ? 1 : 0;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    blocks += id[k] >= 0;
+    rank_own += id[k] >= 0 && id[k] < int(E);
+    rank += id[k] >= 0 && id[k] < nbr;
+  }
+  double* __restrict__ out = R.values + R.row0[E];
+  const int L = blocks * ND;
+#pragma unroll
+  for (int i = 0, k = 0; i < ND; ++i)
+#pragma unroll
+    for (int j = i; j < ND; ++j, ++k) {
+      double v = R.has_element ? R.staging[int64_t(k) * R.ne + E] : 0.;
+      v += lane_of_4<0>(own[k]);
+      v += lane_of_4<1>(own[k]);
+      v += lane_of_4<2>(own[k]);
+      v += lane_of_4<3>(own[k]);
+      own[k] = v;
+    }
+  // lane i stores row i of the own block
+#pragma unroll
+  for (int i = 0; i < ND; ++i)
+    if (f == i) {
+#pragma unroll
+      for (int j = 0; j < ND; ++j) {
+        const int a = i < j ? i : j, b = i < j ? j : i;
+        out[i * L + rank_own * ND + j] = own[a * ND - a * (a - 1) / 2 + b - a];
+      }
+    }
+  if (nbr >= 0) {
+#pragma unroll
+    for (int i = 0; i < ND; ++i)
+#pragma unroll
+      for (int j = 0; j < ND; ++j)
+        out[i * L + rank * ND + j] = outside ? C[j][i] : C[i][j];
+  }
+}
+
 // block K of the four blocks of an inner intersection between elements of types GIN (inside) and GOUT
 // (outside) on a mixed grid: 0 in_in [NI][NI], 1 in_out [NI][NO], 2 out_in [NO][NI], 3 out_out [NO][NO]; every
 // entry is the expression of k_inner_local for the same rows and columns, accumulated in the same order
@@ -1986,10 +2202,15 @@ void launch_assembly(Operator& op, hipStream_t stream, bool matrix)
   auto part_geom = [&](int p) { return g.mixed ? g.parts[p].ref.geom : g.ref.geom; };
   for (FaceParams* F : {&C, &B})
     F->etype = g.mixed ? g.d_etype.ptr : nullptr, F->ls = op.space->local_size, F->cstride = g.ref.nverts;
+  // element, boundary and intersection blocks straight to the values
+  const bool rows = matrix && M.dg_rows && !op.cforms.empty() && C.symmetric && !op.borrowed && !op.dirichlet &&
+                    op.space->order == 1 && g.ref.geom != HGDT_HEX;
   if (matrix && !op.cforms.empty() && nin > 0) {
     C.nfaces = nin, C.faces = M.d_inner.ptr, C.coords = g.d_coords.ptr, C.conn = g.d_conn.ptr;
     C.qtab = op.d_qtab_line.ptr, C.staging = op.d_staging.ptr, C.base = M.inner_base;
-    if (q2hex) // 27 basis functions per side: one lane per (face, row)
+    if (rows)
+      ; // (with the values, below)
+    else if (q2hex) // 27 basis functions per side: one lane per (face, row)
       hipLaunchKernelGGL(k_inner_rows_q2hex, dim3(grid_for(nin * 54, fb)), dim3(fb), 0, stream, C);
     else if (!g.mixed)
       dispatch_faces(g.ref.geom, op.space->order, [&](auto G, auto O) {
@@ -2020,7 +2241,23 @@ void launch_assembly(Operator& op, hipStream_t stream, bool matrix)
       }
     HGDT_HIP(hipGetLastError());
   }
-  if (matrix && (!op.eforms.empty() || !op.cforms.empty() || !op.bforms.empty())) {
+  if (rows) {
+    C.faces = M.d_inner.ptr, C.coords = g.d_coords.ptr, C.conn = g.d_conn.ptr, C.qtab = op.d_qtab_line.ptr;
+    DgRows R{g.ne, M.d_face_code.ptr, M.d_elem_row.ptr, op.d_staging.ptr, M.bnd_base, !op.eforms.empty(),
+             !op.bforms.empty() && nbd > 0, op.d_values.ptr};
+    const dim3 grid(xcd_grid(4 * g.ne, 256));
+    switch (g.ref.geom) {
+      case HGDT_QUAD:
+        hipLaunchKernelGGL(k_dg_rows<HGDT_QUAD>, grid, dim3(256), 0, stream, C, R);
+        break;
+      case HGDT_TRI:
+        hipLaunchKernelGGL(k_dg_rows<HGDT_TRI>, grid, dim3(256), 0, stream, C, R);
+        break;
+      default:
+        hipLaunchKernelGGL(k_dg_rows<HGDT_TET>, grid, dim3(256), 0, stream, C, R);
+    }
+    HGDT_HIP(hipGetLastError());
+  } else if (matrix && (!op.eforms.empty() || !op.cforms.empty() || !op.bforms.empty())) {
     hipLaunchKernelGGL(k_gather_values, dim3(xcd_grid(op.nnz, gb)), dim3(gb), 0, stream, op.nnz, M.d_slot_ptr.ptr,
                        M.d_contrib.ptr, op.d_staging.ptr, op.dirichlet ? op.d_slot_flag.ptr : nullptr,
                        op.d_values.ptr, op.borrowed ? 1 : 0);

@@ -710,6 +710,45 @@ void Operator::build_scatter_maps()
     bnd_packed[2 * f + 0] = M.bnd_e[f], bnd_packed[2 * f + 1] = M.bnd_f[f];
   M.d_inner.upload(inner_packed);
   M.d_bnd.upload(bnd_packed);
+  // rows of blocks: element e's rows are ls e, ..., each with the ascending blocks of e and its neighbours
+  std::atomic<bool> rows_of_blocks{s.kind == HGDT_DISCONTINUOUS_LAGRANGE && !g.mixed && square() && !borrowed && ls <= 4 &&
+                                   nf <= 4 && has_c && nin < (int64_t(1) << 29) && n == ls * ne};
+  if (rows_of_blocks) {
+    std::vector<int32_t> code(size_t(ne) * nf, ScatterMaps::NO_FACE);
+    std::vector<int64_t> first(ne);
+    parallel_for(ne, [&](int64_t e0, int64_t e1) {
+      for (int64_t e = e0; e < e1 && rows_of_blocks; ++e) {
+        int64_t col[5] = {e}, cnt = 1;
+        bool ok = true;
+        for (int f = 0; f < nf; ++f) {
+          const int64_t o = g.nb[e * nf + f];
+          if (o >= 0) {
+            const int32_t fi = o > e ? inner_index[e * nf + f] : inner_index[o * nf + g.nbface[e * nf + f]];
+            ok = ok && fi >= 0 && (o > e ? M.inner_out[fi] == o : M.inner_in[fi] == o && M.inner_out[fi] == e);
+            code[e * nf + f] = 2 * fi + (o > e ? 0 : 1);
+            col[cnt++] = o;
+          } else if (bnd_index[e * nf + f] >= 0) {
+            code[e * nf + f] = -1 - bnd_index[e * nf + f];
+          }
+        }
+        std::sort(col, col + cnt);
+        for (int i = 0; i < ls; ++i) {
+          const int64_t r = ls * e + i;
+          ok = ok && s.dofs[r] == r && row_ptr[r + 1] - row_ptr[r] == ls * cnt;
+          for (int64_t k = 0; ok && k < ls * cnt; ++k)
+            ok = cols[row_ptr[r] + k] == ls * col[k / ls] + k % ls;
+        }
+        first[e] = row_ptr[ls * e];
+        if (!ok)
+          rows_of_blocks = false;
+      }
+    });
+    if (rows_of_blocks) {
+      M.d_face_code.upload(code);
+      M.d_elem_row.upload(first);
+    }
+  }
+  M.dg_rows = rows_of_blocks;
   d_staging.allocate(std::max<int64_t>(M.staging_size, 1));
   M.built = true;
   M.signature = signature;
