@@ -230,6 +230,8 @@ __global__ void __launch_bounds__(T) k_pcg_resident_dg(ResidentParams P, MfParam
   // (element blocks: registers hold the matrix, LDS also the iterate and D^{1/2}, behind p)
   double* const xl = pl + 4 * (P.zero_place + 1);
   double* const sl = xl + 4 * EL;
+  // published values lie by DoF, then by element: lanes of neighbouring elements store and read whole lines
+  const unsigned ne = unsigned(P.n / 4);
   const int t = threadIdx.x, wave = t >> 6;
   if (t == 0)
     failed = 0;
@@ -344,7 +346,7 @@ __global__ void __launch_bounds__(T) k_pcg_resident_dg(ResidentParams P, MfParam
 #pragma unroll
               for (int j = 0; j < 4; ++j)
                 if (halo[j] == RES_EMPTY)
-                  halo[j] = slot_load(at(from, unsigned(4 * src + j)));
+                  halo[j] = slot_load(at(from, unsigned(j) * ne + unsigned(src)));
 #pragma unroll
               for (int j = 0; j < 4; ++j)
                 empty = empty || halo[j] == RES_EMPTY;
@@ -425,9 +427,11 @@ __global__ void __launch_bounds__(T) k_pcg_resident_dg(ResidentParams P, MfParam
         }
         if (elem[k] >> 30 == 1u) {
           double* const to = P.r_pub[par];
+          unsigned id = elem[k] & 0x3fffffffu;
+          asm volatile("" : "+v"(id));
 #pragma unroll
           for (int j = 0; j < 4; ++j)
-            slot_store(at(to, 4u * (elem[k] & 0x3fffffffu) + unsigned(j)), z[j]);
+            slot_store(at(to, unsigned(j) * ne + id), z[j]);
         }
       }
 #pragma unroll
@@ -471,14 +475,19 @@ __global__ void __launch_bounds__(T) k_pcg_resident_dg(ResidentParams P, MfParam
         for (int k = 0; k < E; ++k)
           if (elem[k] >> 30 == 1u) {
             double* const next = P.r_pub[par ^ 1];
+            unsigned id = elem[k] & 0x3fffffffu;
+            asm volatile("" : "+v"(id));
 #pragma unroll
             for (int j = 0; j < 4; ++j)
-              slot_clear(at(next, 4u * (elem[k] & 0x3fffffffu) + unsigned(j)));
+              slot_clear(at(next, unsigned(j) * ne + id));
           }
-        if (l < nhalo)
+        if (l < nhalo) {
+          unsigned id = unsigned(h0);
+          asm volatile("" : "+v"(id));
 #pragma unroll
           for (int j = 0; j < 4; ++j)
-            halo[j] = slot_load(at(P.r_pub[par], unsigned(4 * h0 + j)));
+            halo[j] = slot_load(at(P.r_pub[par], unsigned(j) * ne + id));
+        }
         if (!exchange_sum<2, NW>(P.g2 + (par * P.n_v + K.a0) * RES_PAD, own2, false, K.na, T, red2, &failed, P.gave_up,
                                  P.wait_ticks, rn))
           return;
