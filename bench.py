@@ -219,13 +219,32 @@ def spmv_kernel_name(op, config):
 
 def traffic_record(config, mf):
     """HBM bytes per launch of the dominant kernel from the committed rocprofv3 counter summary"""
-    tfile = os.path.join(ROOT, "profiles", f"pmc_{'mf' if mf else 'cg_spmv'}_{config}.json")
+    return pmc_record(f"pmc_{'mf' if mf else 'cg_spmv'}_{config}.json")
+
+
+def pmc_record(name):
+    tfile = os.path.join(ROOT, "profiles", name)
     if not os.path.exists(tfile):
         return None, None
     with open(tfile) as f:
         d = json.load(f)
     src = f"profiles/{os.path.basename(tfile)} (rocprofv3 --pmc FETCH_SIZE, WRITE_SIZE; {d.get('date', 'undated')})"
     return d.get("hbm_bytes_per_launch"), src
+
+
+def one_launch_record(config, mf, stats, workgroups, step_bytes):
+    """the solves in one launch: their time against the bytes of an application per iteration (the matrix, p read and
+    the product written: what a solve that keeps nothing on the chip between two steps would have to move at least; with
+    the matrix in registers none of it is moved and the exchanges between the workgroups bound the step)"""
+    iters = sum(s["iterations"] for s in stats)
+    us = sum(s["solve_ms"] for s in stats) * 1e3
+    traffic, src = pmc_record(f"pmc_resident{'_mf' if mf else ''}_{config}.json")
+    rate = iters * step_bytes / (us * 1e-6) / 1e9
+    return {"kernel": "k_pcg_resident_dg" if config == "c3" else "k_pcg_resident", "workgroups": workgroups,
+            "avg_launch_us": us / len(stats), "us_per_iteration": us / iters, "achieved": rate, "peak": HBM_PEAK_GBS,
+            "unit": "GB/s", "frac": rate / HBM_PEAK_GBS, "bytes_per_launch": iters // len(stats) * step_bytes,
+            "traffic": traffic, "traffic_source": src,
+            "timing": "HIP events around the timed steps' solves (initial residual, the launch, exit passes)"}
 
 
 # ---------------------------------------------------------------------------------------------------------
@@ -328,6 +347,7 @@ def run_single(hgdt, torch, args, config, fmt, steps, warmup, spmv_sample):
         stats.append(dict(op.last_solve))
     torch.cuda.synchronize()
     elapsed = time.perf_counter() - t0
+    workgroups = op.solve_workgroups()  # of the last solve's one launch (0: three kernels per iteration)
     # the application's roofline comes from one more step with events bound to the sampled dispatches, outside
     # the timed region (the events' own cost stays out of ms_per_step)
     step(time_spmv=spmv_sample)
@@ -375,6 +395,10 @@ def run_single(hgdt, torch, args, config, fmt, steps, warmup, spmv_sample):
                               "ms_per_step; the solve's set-up and exit passes (initial residual, the solver's scaled "
                               "copy, true residual) are not counted"},
     }
+    if workgroups:
+        # the timed steps' dominant kernel; the application of the three-kernel iteration beside it
+        res["roofline_application"] = res["roofline"]
+        res["roofline"] = {"bound": "hbm", **one_launch_record(config, mf, stats, workgroups, step_bytes)}
     return res, (grid, space, op, kappa, x)
 
 

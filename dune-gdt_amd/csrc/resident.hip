@@ -758,7 +758,7 @@ static double step_of(int slots)
 
 // rows per lane: -1 when no choice of `fits` (LDS, compiled variant) takes all instances
 template <class F>
-static int choose_slots(const std::vector<int64_t>& row0, bool sell, F fits)
+static int choose_slots(const std::vector<int64_t>& row0, bool sell, bool given, F fits)
 {
   const int cus = device_cus();
   int best = -1;
@@ -776,6 +776,10 @@ static int choose_slots(const std::vector<int64_t>& row0, bool sell, F fits)
     if (t >= 0. && (best < 0 || t < time) && fits(s))
       best = s, time = t;
   }
+  // row blocks that the caller chose: any number of workgroups that fits
+  for (int s : {1, 2, 4, 8, 16})
+    if (given && best < 0 && row0.size() == 2 && team_of(row0[1] - row0[0], s) <= cus && fits(s))
+      best = s;
   return best;
 }
 
@@ -824,7 +828,7 @@ ResidentShape resident_shape_dia(const std::vector<int64_t>& row0, const std::ve
   if (s_nu < 0 || s_nu > 4)
     return {};
   const int64_t reach = reach_of(row0, s_offs);
-  const int s = choose_slots(row0, false, [&](int k) { return lds_of(k, reach, s_nu) <= RES_LDS && !(s_nu == 0 && k > 8); });
+  const int s = choose_slots(row0, false, false, [&](int k) { return lds_of(k, reach, s_nu) <= RES_LDS && !(s_nu == 0 && k > 8); });
   if (s > 0)
     return {RES_LANES, std::min(s, 8)}; // (16 rows per lane: two blocks of 8 each)
   if (far_slots(row0, s_offs, s_nu))
@@ -933,7 +937,7 @@ void resident_plan_dia(ResidentPlan& plan, const Operator& op, const std::vector
   if (lg > 0 && bv != RES_LANES)
     return;
   const int64_t reach = reach_of(row0, s_offs);
-  const int slots = choose_slots(row0, false, [&](int k) {
+  const int slots = choose_slots(row0, false, true, [&](int k) {
     // (a diagonal matrix holds no slot to stream)
     return (int64_t(k) * RES_LANES) % ba == 0 && kernel_of(k, lg, same, s_nu) && lds_of(k, reach, s_nu) <= RES_LDS &&
            !(s_nu == 0 && k > 8);
@@ -962,7 +966,7 @@ static void halo_of(const Operator& op, int64_t r0, int64_t r1, std::vector<int3
 int resident_items_sell(const Operator& op)
 {
   const std::vector<int64_t>& row0 = op.space->inst_dof;
-  const int s = choose_slots(row0, true, [&](int k) {
+  const int s = choose_slots(row0, true, false, [&](int k) {
     if (k > 8)
       return false;
     // p of the own rows and the halo in LDS

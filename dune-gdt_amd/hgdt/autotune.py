@@ -4,7 +4,8 @@ A candidate launch shape is timed on the operator itself: for the solver, a fixe
 iterations (relative tolerance 0, so exactly `iterations` iterations run) measured with HIP events
 inside libhgdt; for assembly, MatrixOperator.assemble() bracketed by torch events.  The operator
 application (kernel 3) and the vector kernels (kernel 4) have separate row partitions and are tuned
-one after the other; with symmetric DIA storage the tuner then times the application with and without
+one after the other, and the pair that the operator has by itself (which often lets the whole solve run in one
+launch, where one shape at a time is never seen to be better) is kept where it is as fast; with symmetric DIA storage the tuner then times the application with and without
 column staging (p entries of a row block read from LDS) at the chosen shapes and keeps the faster.
 Results are cached per problem signature in memory and optionally in a JSON file.
 """
@@ -16,9 +17,9 @@ import torch
 from . import _lib as L
 
 APPLY_CANDIDATES = [(64, 1), (128, 1), (256, 1), (512, 1), (1024, 1), (256, 2), (512, 2), (128, 2), (256, 4),
-                    (512, 4), (256, 8), (512, 8), (1024, 4), (256, 16)]
+                    (512, 4), (256, 8), (512, 8), (1024, 4), (256, 16), (768, 4)]
 VECTOR_CANDIDATES = [(256, 1), (256, 2), (256, 4), (256, 8), (512, 1), (512, 2), (512, 4), (512, 8),
-                     (1024, 1), (1024, 2), (1024, 4), (128, 4), (128, 8)]
+                     (1024, 1), (1024, 2), (1024, 4), (128, 4), (128, 8), (768, 4)]
 ASSEMBLY_CANDIDATES = [64, 128, 256]
 
 _memory = {}
@@ -44,7 +45,7 @@ def _solver_us_per_iteration(op, iterations):
     """time per PCG iteration from two run lengths (fixed set-up and drain costs cancel)"""
     t1, i1 = _solve_ms(op, iterations)
     t2, i2 = _solve_ms(op, 2 * iterations)
-    if i2 <= i1:  # converged early: fall back to the plain ratio
+    if i2 <= i1 or t2 <= t1:  # converged early, or lost in the set-up's own noise: fall back to the plain ratio
         return t2 * 1e3 / max(1, i2)
     return (t2 - t1) * 1e3 / (i2 - i1)
 
@@ -82,14 +83,21 @@ def tune_solver(op, iterations=40, repeats=2, cache_file=None, verbose=False):
                 print(f"  kernel {kernel} block {cand[0]:4d} items {cand[1]}: {t:8.2f} us/iteration", flush=True)
         return min(results, key=results.get), results
 
-    vec0 = op.get_launch(L.KERNEL_VECTOR)
+    own = (op.get_launch(L.KERNEL_APPLY), op.get_launch(L.KERNEL_VECTOR))
+    own_us = min(_solver_us_per_iteration(op, iterations) for _ in range(repeats))
+    if verbose:
+        print(f"  own shapes {own}: {own_us:8.2f} us/iteration", flush=True)
+    vec0 = own[1]
     best_a, ra = best_of(L.KERNEL_APPLY, APPLY_CANDIDATES, (L.KERNEL_VECTOR, *vec0))
     best_v, rv = best_of(L.KERNEL_VECTOR, VECTOR_CANDIDATES, (L.KERNEL_APPLY, *best_a))
+    best_us = rv[best_v]
+    if own_us <= best_us and own[0] in APPLY_CANDIDATES and own[1] in VECTOR_CANDIDATES:
+        (best_a, best_v), best_us = own, own_us
     op.set_launch(L.KERNEL_APPLY, *best_a)
     op.set_launch(L.KERNEL_VECTOR, *best_v)
     timings = {"apply": {f"{b}x{i}": t for (b, i), t in ra.items()},
                "vector": {f"{b}x{i}": t for (b, i), t in rv.items()}}
-    choice = {"apply": list(best_a), "vector": list(best_v), "us_per_iteration": rv[best_v]}
+    choice = {"apply": list(best_a), "vector": list(best_v), "us_per_iteration": best_us}
     if op.format_info()["format"] == "dia_symmetric" and best_a[1] == 1 and _staging_applies(op):
         # column staging off / on at the chosen shapes (only where the staged kernel applies: one row per
         # lane and a stencil whose windows fit; elsewhere both settings would time the same kernel and the
