@@ -327,6 +327,7 @@ struct SolverFormat {
   bool partitions_ready = false; // row partitions A and V built for the current launch shapes
   bool structure_ready = false;  // storage layout (DIA offsets / SELL slices) built
   bool valid = false;  // values converted since the last assemble
+  bool cleared = false, scaled_cleared = false; // the storage (SELL: the scaled copy) holds zeros outside the pattern
   bool diag_positive = false;
   bool symmetric = false; // DIA read through its upper diagonals only (exactly symmetric matrix)
   int nup = 0;            // diagonals with offset >= 0

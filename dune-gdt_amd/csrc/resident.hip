@@ -575,7 +575,7 @@ __global__ void __launch_bounds__(T) k_pcg_resident(ResidentParams P)
       D.iters = begun;
       D.done = state;
       D.brk = 0;
-      P.S[P.ninst + K.inst] = D;
+      P.result[K.inst] = D;
     }
   }
 }
@@ -593,7 +593,7 @@ __global__ void __launch_bounds__(256) k_resident_clear(ResidentParams P, int64_
   if (i < FLAGS)
     P.flags[i] = 0;
   if (i == 0)
-    *P.gave_up = 0;
+    *P.gave_up.device = 0;
 }
 
 using Kernel = void (*)(ResidentParams);
@@ -900,8 +900,15 @@ void resident_finish(ResidentPlan& plan, const Operator& op, const std::vector<R
   plan.tasks.upload(list);
   plan.task_start.upload(start);
   plan.n_a = n_a, plan.n_v = n_v;
+  plan.exchanges = std::any_of(teams.begin(), teams.end(), [](int t) { return t > 1; });
+  plan.cus = device_cus();
+  plan.kernel = plan.dg ? resident_dg_kernel(plan)
+                        : reinterpret_cast<const void*>(plan.far ? far_kernel(plan.slots)
+                                                                 : kernel_of(plan.slots, plan.lg_items, plan.same_blocks,
+                                                                             plan.nu));
+  HGDT_HIP(hipFuncSetAttribute(plan.kernel, hipFuncAttributeMaxDynamicSharedMemorySize, int(RES_LDS)));
   plan.exchange.allocate(size_t(RES_PAD * (3 * n_a + 2 * n_v)));
-  plan.gave_up.allocate(1 + RES_MAX_GROUPS);
+  plan.gave_up.upload(std::vector<int>(1 + RES_MAX_GROUPS, 0));
   if (!plan.host_gave_up)
     HGDT_HIP(hipHostMalloc((void**)&plan.host_gave_up, sizeof(int)));
   plan.usable = true;
@@ -1068,45 +1075,47 @@ void resident_plan_sell(ResidentPlan& plan, const Operator& op)
   resident_finish(plan, op, tasks, (R + most) * int64_t(sizeof(double)), F.A.nblocks, F.V.nblocks);
 }
 
-bool resident_run(ResidentPlan& plan, ResidentParams P, const MfParams& M, hipStream_t stream, PcgScalars* host_records)
+ResidentLaunch::ResidentLaunch(ResidentPlan& plan, ResidentParams P, const MfParams& M, hipStream_t stream)
+  : stream_(stream)
 {
   P.n_a = plan.n_a, P.n_v = plan.n_v;
   P.dg_elements = plan.elements.ptr, P.zero_place = plan.zero_place;
   P.g1 = plan.exchange.ptr;
   P.g2 = plan.exchange.ptr + 3 * P.n_a * RES_PAD;
   P.sell_local = plan.sell_local.ptr, P.halo_rows = plan.halo_rows.ptr, P.publish = plan.publish.ptr;
-  P.tasks = plan.tasks.ptr, P.task_start = plan.task_start.ptr, P.gave_up = plan.gave_up.ptr, P.flags = plan.gave_up.ptr + 1;
+  P.tasks = plan.tasks.ptr, P.task_start = plan.task_start.ptr;
+  P.gave_up = {plan.gave_up.ptr, plan.host_gave_up}, P.flags = plan.gave_up.ptr + 1;
   P.wait_ticks = int64_t(4) * 100000000; // 4 s
+  *plan.host_gave_up = 0;
   const int64_t nx = int64_t(plan.exchange.count);
-  hipLaunchKernelGGL(k_resident_clear, dim3(xcd_grid(std::max<int64_t>(std::max(P.n, nx), RES_MAX_GROUPS), 256)), dim3(256), 0, stream, P, nx);
-  const void* const k = plan.dg ? resident_dg_kernel(plan)
-                                : reinterpret_cast<const void*>(plan.far ? far_kernel(plan.slots)
-                                                                         : kernel_of(plan.slots, plan.lg_items,
-                                                                                     P.same_blocks, plan.nu));
-  HGDT_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, int(RES_LDS)));
-  int dev = 0;
-  HGDT_HIP(hipGetDevice(&dev));
-  struct Hold {
-    int dev, count;
-    ~Hold()
-    {
-      CuBudget::get().give(dev, count);
-    }
-  };
-  const int cus = device_cus(), held = std::min(plan.grid, cus);
-  CuBudget::get().take(dev, held, cus);
-  Hold hold{dev, held};
+  if (plan.exchanges)
+    hipLaunchKernelGGL(k_resident_clear, dim3(xcd_grid(std::max<int64_t>(std::max(P.n, nx), RES_MAX_GROUPS), 256)),
+                       dim3(256), 0, stream, P, nx);
+  HGDT_HIP(hipGetLastError());
+  HGDT_HIP(hipGetDevice(&device_));
+  held_ = std::min(plan.grid, plan.cus);
+  CuBudget::get().take(device_, held_, plan.cus);
   MfParams Mk = M;
   void* args[2] = {&P, &Mk}; // (the second: discontinuous spaces)
-  hipError_t e = hipLaunchKernel(k, dim3(unsigned(plan.grid)), dim3(unsigned(plan.lanes)), args, size_t(plan.lds), stream);
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(plan.host_gave_up, plan.gave_up.ptr, sizeof(int), hipMemcpyDeviceToHost, stream);
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(host_records, P.S + P.ninst, sizeof(PcgScalars) * P.ninst, hipMemcpyDeviceToHost, stream);
-  const hipError_t e2 = hipStreamSynchronize(stream); // also after an error: the CUs are given back with none running
+  const hipError_t e =
+      hipLaunchKernel(plan.kernel, dim3(unsigned(plan.grid)), dim3(unsigned(plan.lanes)), args, size_t(plan.lds), stream);
+  if (e != hipSuccess)
+    CuBudget::get().give(device_, held_);
   HGDT_HIP(e);
-  HGDT_HIP(e2);
-  return *plan.host_gave_up == 0;
+}
+
+ResidentLaunch::~ResidentLaunch()
+{
+  (void)hipStreamSynchronize(stream_); // the CUs are given back with none of its workgroups running
+  CuBudget::get().give(device_, held_);
+}
+
+bool resident_gave_up(ResidentPlan& plan)
+{
+  if (!__atomic_load_n(plan.host_gave_up, __ATOMIC_ACQUIRE))
+    return false;
+  plan.skip = 16; // (whoever holds the CUs may do so for a while, and a wait costs seconds)
+  return true;
 }
 
 } // namespace hgdt

@@ -34,6 +34,12 @@ struct ResidentTask {
   int32_t mask; // its block of `publish`
 };
 
+// set when a wait outlasts its limit, for the workgroups (every one then ends) and for the host (pinned memory)
+struct ResidentFlags {
+  int* device;
+  int* host;
+};
+
 struct ResidentParams {
   int64_t n;
   int ninst;
@@ -69,12 +75,13 @@ struct ResidentParams {
   double* g1;          // 2 x (operator blocks), padded: partials of p.q, by parity of the step
   double* g2;          // behind it, 2 x (vector blocks), padded: partials of the two residual norms
   int64_t n_a, n_v;    // operator / vector blocks of all instances
-  PcgScalars* S;       // records of the instances: tolerances read; the results go to the ninst records behind these
+  const PcgScalars* S; // records of the instances
+  PcgScalars* result;  // and their results (pinned host memory)
   int64_t max_iter;
   const ResidentTask* tasks;
   const int32_t* task_start; // per workgroup
   int* flags;          // FAR: per workgroup, the step whose p it has published
-  int* gave_up;        // set when a wait outlasts its limit: every workgroup then ends
+  ResidentFlags gave_up;
   int64_t wait_ticks;  // limit of one wait, in ticks of the 100 MHz counter
 };
 
@@ -101,8 +108,12 @@ struct ResidentPlan {
   DeviceArray<ResidentTask> tasks;
   DeviceArray<int32_t> task_start;
   DeviceArray<double> exchange; // g1, g2
-  DeviceArray<int> gave_up;
+  DeviceArray<int> gave_up;    // and the flags of the workgroups behind it
   int* host_gave_up = nullptr;
+  bool exchanges = false;      // some instance has more than one workgroup
+  const void* kernel = nullptr;
+  int cus = 0;
+  int skip = 0; // solves that go without the launch after one that gave up
   ~ResidentPlan()
   {
     if (host_gave_up)
@@ -133,8 +144,21 @@ double resident_schedule(const std::vector<int64_t>& row0, const std::vector<int
 // the tasks (instance by instance) in the order in which the workgroups take them; buffers of the exchanges
 void resident_finish(ResidentPlan& plan, const Operator& op, const std::vector<ResidentTask>& tasks, int64_t lds,
                      int64_t n_a, int64_t n_v);
-// runs the solve; false when it gave up (then nothing but r_pub, x_out, the results' records and the exchange buffers was
-// written: the caller goes on with one launch per kernel).  Waits for the kernel.  M: the matrix-free operator.
-bool resident_run(ResidentPlan& plan, ResidentParams P, const MfParams& M, hipStream_t stream, PcgScalars* host_records);
+// A launch of the solve.  Its CUs are the solve's until this object goes, which waits for the launch (and for what else the
+// stream holds by then).
+class ResidentLaunch {
+  int device_, held_;
+  hipStream_t stream_;
+
+public:
+  // results: pinned host memory.  What the launch writes besides these: r_pub, x_out and the exchange buffers; after
+  // one that gave up the caller goes on with one launch per kernel.  M: the matrix-free operator.
+  ResidentLaunch(ResidentPlan& plan, ResidentParams P, const MfParams& M, hipStream_t stream);
+  ~ResidentLaunch();
+  ResidentLaunch(const ResidentLaunch&) = delete;
+  ResidentLaunch& operator=(const ResidentLaunch&) = delete;
+};
+// the solve of a finished launch gave up
+bool resident_gave_up(ResidentPlan& plan);
 
 } // namespace hgdt

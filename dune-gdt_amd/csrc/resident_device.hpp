@@ -42,7 +42,7 @@ __device__ __forceinline__ unsigned long long slot_load(const double* p)
 struct Patience {
   int looks = 0;
   long long since = 0;
-  __device__ __forceinline__ bool over(int* gave_up, int64_t ticks)
+  __device__ __forceinline__ bool over(ResidentFlags gave_up, int64_t ticks)
   {
     if (++looks < 256)
       return false;
@@ -51,9 +51,10 @@ struct Patience {
       since = wall_clock64();
     if (looks & 255)
       return false;
-    if (!__hip_atomic_load(gave_up, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) && wall_clock64() - since <= ticks)
+    if (!__hip_atomic_load(gave_up.device, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) && wall_clock64() - since <= ticks)
       return false;
-    __hip_atomic_store(gave_up, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(gave_up.device, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(gave_up.host, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     return true;
   }
 };
@@ -77,7 +78,7 @@ __device__ __forceinline__ T* at(T* base, unsigned i)
 // gave up.  One barrier; red is not written again before a later barrier.
 template <int NV, int NW>
 __device__ __forceinline__ bool exchange_sum(const double* slots, const double (&own)[NV], bool alone, int count,
-                                             int block, double (*red)[RES_WAVES], int* failed, int* gave_up,
+                                             int block, double (*red)[RES_WAVES], int* failed, ResidentFlags gave_up,
                                              int64_t ticks, double (&tot)[NV])
 {
   const int t = threadIdx.x;

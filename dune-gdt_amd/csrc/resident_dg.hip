@@ -507,7 +507,7 @@ __global__ void __launch_bounds__(T) k_pcg_resident_dg(ResidentParams P, MfParam
       D.iters = begun;
       D.done = state;
       D.brk = 0;
-      P.S[P.ninst + K.inst] = D;
+      P.result[K.inst] = D;
     }
   }
 }

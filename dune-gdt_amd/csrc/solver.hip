@@ -949,11 +949,12 @@ __global__ void __launch_bounds__(1024) k_cg_update(PcgParams P, int par)
     P.part2[int64_t(b) * 2 + 0] = v[0], P.part2[int64_t(b) * 2 + 1] = v[1];
 }
 
-// x = D^{-1/2} xh after the last step
-__global__ void k_cg_finish(int64_t n, const double* __restrict__ dh, const double* xh, double* x)
+// x = D^{-1/2} xh after the last step (gave_up set: the launch that was to make xh ended without it, x stays)
+__global__ void k_cg_finish(int64_t n, const double* __restrict__ dh, const double* xh, double* x,
+                            const int* __restrict__ gave_up)
 {
   const int64_t i = xcd_index(n);
-  if (i < n)
+  if (i < n && !(gave_up && *gave_up))
     x[i] = dh[i] * xh[i];
 }
 
@@ -1366,7 +1367,6 @@ struct SolverCache {
   PcgScalars* host_scalars[2] = {nullptr, nullptr};
   int host_capacity = 0;
   // true relative residual per instance at the solver's exit (device and pinned host copy)
-  DeviceArray<double> true_relres;
   double* host_true = nullptr;
   int host_true_capacity = 0;
   hipEvent_t copied[2] = {nullptr, nullptr};
@@ -1804,6 +1804,7 @@ static void build_structure(Operator& op)
   C.win.release();
   F.d_dia.release(), F.d_dia_pos.release(), F.d_sell_vals.release(), F.d_sell_cols.release();
   F.d_sell_pos.release(), F.d_scaled.release();
+  F.cleared = F.scaled_cleared = false;
   F.d_mf_ref.release();
   F.mf_kind = -1;
   if (!op.square() && op.requested_format != HGDT_FORMAT_AUTO && op.requested_format != HGDT_FORMAT_SELL)
@@ -2137,6 +2138,7 @@ void Operator::assemble_direct(hipStream_t stream)
   hipLaunchKernelGGL(k_direct_p1_tets, dim3(blocks_for(n, B)), dim3(B), 0, stream, P);
   HGDT_HIP(hipGetLastError());
   F.valid = false;
+  F.cleared = false; // (wrote whole diagonals)
   direct_storage = true;
   values_stale = true;
 }
@@ -2212,9 +2214,15 @@ void Operator::prepare_storage(hipStream_t stream)
     HGDT_THROW(HGDT_ERR_OPERATOR,
                "the operator was assembled in matrix-free mode and holds no matrix: assemble again in this format");
   const int B = 256;
+  // entries outside the pattern are cleared with the first values: the later ones land on the same entries
+  auto clear_once = [&](bool& cleared, double* values, int64_t count) {
+    if (!cleared)
+      hipLaunchKernelGGL(k_fill, dim3(blocks_for(count, B)), dim3(B), 0, stream, count, values, 0.);
+    cleared = true;
+  };
   if (F.format == HGDT_FORMAT_BLOCK) {
     const int64_t total = int64_t(16 + 16 * F.blk_mn) * F.blk_ne;
-    hipLaunchKernelGGL(k_fill, dim3(blocks_for(total, B)), dim3(B), 0, stream, total, F.d_blk.ptr, 0.);
+    clear_once(F.cleared, F.d_blk.ptr, total);
     hipLaunchKernelGGL(k_scatter_values, dim3(blocks_for(nnz, B)), dim3(B), 0, stream, nnz, d_values.ptr,
                        F.d_blk_pos.ptr, F.d_blk.ptr);
     hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, stream, 2, C.flags.ptr, 0);
@@ -2244,7 +2252,7 @@ void Operator::prepare_storage(hipStream_t stream)
   const int64_t total = dia ? int64_t(F.ndiag) * n : int64_t(F.d_sell_vals.count);
   if (!square()) {
     // an operator between two spaces: its SELL values for apply(); no Jacobi scaling, no solver copy
-    hipLaunchKernelGGL(k_fill, dim3(blocks_for(total, B)), dim3(B), 0, stream, total, dst, 0.);
+    clear_once(F.cleared, dst, total);
     hipLaunchKernelGGL(k_scatter_values, dim3(blocks_for(nnz, B)), dim3(B), 0, stream, nnz, d_values.ptr,
                        F.d_sell_pos.ptr, dst);
     HGDT_HIP(hipGetLastError());
@@ -2261,7 +2269,7 @@ void Operator::prepare_storage(hipStream_t stream)
   } else {
     if (values_stale)
       materialize_values(stream);
-    hipLaunchKernelGGL(k_fill, dim3(blocks_for(total, B)), dim3(B), 0, stream, total, dst, 0.);
+    clear_once(F.cleared, dst, total);
     hipLaunchKernelGGL(k_scatter_values, dim3(blocks_for(nnz, B)), dim3(B), 0, stream, nnz, d_values.ptr,
                        dia ? F.d_dia_pos.ptr : F.d_sell_pos.ptr, dst);
     hipLaunchKernelGGL(k_fill_int, dim3(blocks_for(nflags, B)), dim3(B), 0, stream, int(nflags), C.flags.ptr, 0);
@@ -2301,7 +2309,7 @@ void Operator::prepare_storage(hipStream_t stream)
   } else {
     C.scaled_pad = 0;
     F.d_scaled.allocate(std::max<int64_t>(total, 1));
-    hipLaunchKernelGGL(k_fill, dim3(blocks_for(total, B)), dim3(B), 0, stream, total, F.d_scaled.ptr, 0.);
+    clear_once(F.scaled_cleared, F.d_scaled.ptr, total);
     hipLaunchKernelGGL(k_scale_values, dim3(blocks_for(n, B)), dim3(B), 0, stream, n, d_row_ptr.ptr, d_cols.ptr,
                        d_values.ptr, F.d_sell_pos.ptr, F.d_dh.ptr, F.d_scaled.ptr);
   }
@@ -2444,7 +2452,7 @@ static ResidentPlan& resident_plan(Operator& op)
   return plan;
 }
 
-static bool resident_solve(Operator& op, const PcgParams& P, hipStream_t stream)
+static std::unique_ptr<ResidentLaunch> resident_solve(Operator& op, const PcgParams& P, hipStream_t stream)
 {
   const SolverFormat& F = op.fmt;
   SolverCache& C = cache_of(op);
@@ -2456,9 +2464,9 @@ static bool resident_solve(Operator& op, const PcgParams& P, hipStream_t stream)
   R.blk_ne = P.blk_ne, R.blk_mn = P.blk_mn, R.blk_sym = F.symmetric, R.blk_nb = P.blk_nb, R.blk_mir = P.blk_mir;
   R.dg_ref = F.d_mf_ref.ptr, R.dh = P.dh;
   R.r = P.r, R.x = P.x, R.x_out = P.q, R.r_pub[0] = P.p, R.r_pub[1] = P.p2, R.part2 = P.part2;
-  R.S = P.S, R.max_iter = P.max_iter;
-  return resident_run(C.resident, R, F.format == HGDT_FORMAT_MATRIX_FREE ? mf_params(op) : MfParams{}, stream,
-                      C.host_scalars[0]);
+  R.S = P.S, R.result = C.host_scalars[0], R.max_iter = P.max_iter;
+  return std::make_unique<ResidentLaunch>(C.resident, R, F.format == HGDT_FORMAT_MATRIX_FREE ? mf_params(op) : MfParams{},
+                                          stream);
 }
 
 void Operator::apply_inverse(const double* b, double* x, const hgdt_solver_options& opt, hgdt_solver_stats& st,
@@ -2535,23 +2543,12 @@ void Operator::apply_inverse(const double* b, double* x, const hgdt_solver_optio
   // one whose update met the tolerance (the stopping test is the first thing a step does)
   const int chunk = opt.check_every + (opt.check_every & 1);
   // in one launch where the vectors fit on the chip (a timed solve issues the kernel that is timed)
-  const bool solved = !opt.time_spmv && resident_plan(*this).usable && resident_solve(*this, P, stream);
-  last_workgroups = solved ? C.resident.workgroups : 0;
-  if (!solved && graph && (C.graph == nullptr || C.graph_x != x || C.graph_chunk != chunk || C.graph_version != C.version
-                || C.graph_b != b || C.graph_maxit != opt.max_iter)) {
-    if (C.graph)
-      HGDT_HIP(hipGraphExecDestroy(C.graph));
-    C.graph = nullptr;
-    hipGraph_t g;
-    HGDT_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
-    for (int it = 0; it < chunk; ++it)
-      launch_iteration(*this, P, it & 1, stream, nullptr, nullptr);
-    HGDT_HIP(hipStreamEndCapture(stream, &g));
-    HGDT_HIP(hipGraphInstantiate(&C.graph, g, nullptr, nullptr, 0));
-    HGDT_HIP(hipGraphDestroy(g));
-    C.graph_x = x, C.graph_b = b, C.graph_chunk = chunk, C.graph_version = C.version;
-    C.graph_maxit = opt.max_iter;
-  }
+  bool solved = !opt.time_spmv && resident_plan(*this).usable;
+  if (solved && C.resident.skip > 0)
+    --C.resident.skip, solved = false;
+  std::unique_ptr<ResidentLaunch> launch; // (goes after the exit passes are queued and waited for)
+  if (solved)
+    launch = resident_solve(*this, P, stream);
   size_t nev = 0;
   int64_t issued = 0; // iterations launched so far
   std::vector<int64_t> timed_iter;
@@ -2647,7 +2644,22 @@ void Operator::apply_inverse(const double* b, double* x, const hgdt_solver_optio
   const int64_t max_chunks = (opt.max_iter + 1 + chunk - 1) / chunk + 1;
   int cur = 0;
   int64_t launched = 0;
-  if (!solved) {
+  auto iterate = [&]() {
+    if (graph && (C.graph == nullptr || C.graph_x != x || C.graph_chunk != chunk || C.graph_version != C.version
+                  || C.graph_b != b || C.graph_maxit != opt.max_iter)) {
+      if (C.graph)
+        HGDT_HIP(hipGraphExecDestroy(C.graph));
+      C.graph = nullptr;
+      hipGraph_t g;
+      HGDT_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
+      for (int it = 0; it < chunk; ++it)
+        launch_iteration(*this, P, it & 1, stream, nullptr, nullptr);
+      HGDT_HIP(hipStreamEndCapture(stream, &g));
+      HGDT_HIP(hipGraphInstantiate(&C.graph, g, nullptr, nullptr, 0));
+      HGDT_HIP(hipGraphDestroy(g));
+      C.graph_x = x, C.graph_b = b, C.graph_chunk = chunk, C.graph_version = C.version;
+      C.graph_maxit = opt.max_iter;
+    }
     launch_chunk();
     ++launched;
     HGDT_HIP(hipMemcpyAsync(C.host_scalars[cur], d_scalars.ptr, sizeof(PcgScalars) * ninst, hipMemcpyDeviceToHost,
@@ -2676,7 +2688,45 @@ void Operator::apply_inverse(const double* b, double* x, const hgdt_solver_optio
         compact(C.host_scalars[cur]);
       cur = nxt;
     }
-  } else if (ninst > 1) {
+  };
+  if (!solved)
+    iterate();
+  // the exit passes; behind a launch that gave up they leave x as it was, and follow the three kernels' iterations again
+  while (true) {
+    hipLaunchKernelGGL(k_cg_finish, dim3(blocks_for(n, 256)), dim3(256), 0, stream, n, fmt.d_dh.ptr,
+                       solved ? d_q.ptr : x, x, solved ? C.resident.gave_up.ptr : nullptr);
+    HGDT_HIP(hipGetLastError());
+    // true residual |b - A x| / |b| of every instance at exit, with the unscaled operator (one application and
+    // one pass over b and A x, over all blocks whatever the narrowed launches held)
+    if (opt.true_residual) {
+      if (C.host_true_capacity < ninst) {
+        if (C.host_true)
+          HGDT_HIP(hipHostFree(C.host_true));
+        C.host_true = nullptr;
+        HGDT_HIP(hipHostMalloc((void**)&C.host_true, sizeof(double) * ninst));
+        C.host_true_capacity = ninst;
+      }
+      apply(x, d_q.ptr, stream);
+      PcgParams T = make_params(*this);
+      T.b = b, T.ax = d_q.ptr, T.part3 = P.part3, T.S = P.S;
+      dispatch_items(fmt.V.items, [&](auto IT) {
+        constexpr int I = decltype(IT)::value;
+        hipLaunchKernelGGL((k_true_residual<I>), dim3(hw_blocks(fmt.V.nblocks)), dim3(fmt.V.block), 0, stream, T);
+      });
+      hipLaunchKernelGGL(k_true_reduce, dim3(unsigned(ninst)), dim3(256), 0, stream, T, C.host_true);
+      HGDT_HIP(hipGetLastError());
+    }
+    HGDT_HIP(hipEventRecord(C.t1, stream));
+    HGDT_HIP(hipEventSynchronize(C.t1));
+    if (!solved || !resident_gave_up(C.resident))
+      break;
+    solved = false;
+    launch.reset();
+    iterate();
+  }
+  launch.reset();
+  last_workgroups = solved ? C.resident.workgroups : 0;
+  if (solved && ninst > 1) {
     // the workgroups of an instance end with it: counted as narrowings while others went on
     int64_t most = 0;
     for (int i = 0; i < ninst; ++i)
@@ -2684,33 +2734,6 @@ void Operator::apply_inverse(const double* b, double* x, const hgdt_solver_optio
     for (int i = 0; i < ninst; ++i)
       compactions += C.host_scalars[0][i].iters < most;
   }
-  hipLaunchKernelGGL(k_cg_finish, dim3(blocks_for(n, 256)), dim3(256), 0, stream, n, fmt.d_dh.ptr,
-                     solved ? d_q.ptr : x, x);
-  HGDT_HIP(hipGetLastError());
-  // true residual |b - A x| / |b| of every instance at exit, with the unscaled operator (one application and
-  // one pass over b and A x, over all blocks whatever the narrowed launches held)
-  if (opt.true_residual) {
-    if (C.host_true_capacity < ninst) {
-      if (C.host_true)
-        HGDT_HIP(hipHostFree(C.host_true));
-      C.host_true = nullptr;
-      HGDT_HIP(hipHostMalloc((void**)&C.host_true, sizeof(double) * ninst));
-      C.host_true_capacity = ninst;
-    }
-    C.true_relres.allocate(size_t(ninst));
-    apply(x, d_q.ptr, stream);
-    PcgParams T = make_params(*this);
-    T.b = b, T.ax = d_q.ptr, T.part3 = P.part3, T.S = P.S;
-    dispatch_items(fmt.V.items, [&](auto IT) {
-      constexpr int I = decltype(IT)::value;
-      hipLaunchKernelGGL((k_true_residual<I>), dim3(hw_blocks(fmt.V.nblocks)), dim3(fmt.V.block), 0, stream, T);
-    });
-    hipLaunchKernelGGL(k_true_reduce, dim3(unsigned(ninst)), dim3(256), 0, stream, T, C.true_relres.ptr);
-    HGDT_HIP(hipGetLastError());
-    HGDT_HIP(hipMemcpyAsync(C.host_true, C.true_relres.ptr, sizeof(double) * ninst, hipMemcpyDeviceToHost, stream));
-  }
-  HGDT_HIP(hipEventRecord(C.t1, stream));
-  HGDT_HIP(hipEventSynchronize(C.t1));
   if (graph) {
     HGDT_HIP(hipEventRecord(C.join, stream));
     HGDT_HIP(hipStreamWaitEvent(user_stream, C.join, 0));
