@@ -949,12 +949,14 @@ __global__ void __launch_bounds__(256) k_inner_local(FaceParams P)
 // inside's frame, the in_out block, stored transposed by the outside): the matrix is symmetric bit for bit.
 // Against k_inner_local and k_gather_values this evaluates every intersection twice, but needs 52 registers for
 // accumulators instead of 128 (2 waves per SIMD instead of 1) and neither writes and reads back the blocks of the
-// intersections (512 bytes each) nor reads a list of contributions (4 bytes each).  P1 on 82 944 tetrahedra (6.4 million
-// entries): 77 + 58 us -> 54 us.  Bound by the arithmetic and by chains of loads that two waves per SIMD do not hide.
+// intersections (512 bytes each) nor reads a list of contributions (4 bytes each).  On simplices the sums over a face's
+// points are taken once per form (the normal derivatives are constant), and the rows of 16 elements leave through LDS in
+// whole lines.  P1 on 82 944 tetrahedra (6.4 million entries): 77 + 58 us -> 54 us, with the last two 47 us.  Bound by the
+// geometries, which every element has evaluated by its four lanes and by those of its neighbours.
 struct DgRows {
   int64_t ne;
   const int32_t* code;
-  const int64_t* row0;
+  const int64_t* row0; // ne + 1
   const double* staging;
   int64_t bnd_base;
   int has_element, has_boundary; // staged element / boundary blocks
@@ -980,12 +982,17 @@ __global__ void __launch_bounds__(256) k_dg_rows(FaceParams P, DgRows R)
   constexpr int D = T::D, ND = Basis<GEOM, 1>::ND, NF = T::SIMPLEX ? D + 1 : 2 * D;
   constexpr int NU = ND * (ND + 1) / 2;
   static_assert(ND <= 4 && NF <= 4, "one lane per face, 4 lanes per element");
+  // the rows of a wave's 16 elements, one contiguous range of values (with 2 gaps per 32: fewer bank conflicts)
+  constexpr int RANGE = 16 * ND * ND * (1 + NF);
+  __shared__ double rows[4][RANGE + RANGE / 16];
   const int64_t t = xcd_index(4 * R.ne);
-  if (t >= 4 * R.ne) // (whole elements)
+  const int lane = threadIdx.x & 63;
+  if (t - lane >= 4 * R.ne)
     return;
-  const int64_t E = t >> 2;
+  const bool live = t < 4 * R.ne; // (whole elements)
+  const int64_t E = min(t >> 2, R.ne - 1);
   const int f = int(t & 3);
-  const int32_t code = f < NF ? R.code[E * NF + f] : ScatterMaps::NO_FACE;
+  const int32_t code = live && f < NF ? R.code[E * NF + f] : ScatterMaps::NO_FACE;
   const bool outside = code & 1;
   double own[NU], C[ND][ND]; // own block; in_out block (rows of the inside)
 #pragma unroll
@@ -1053,59 +1060,117 @@ __global__ void __launch_bounds__(256) k_dg_rows(FaceParams P, DgRows R)
         pen = (prm * ((delta_plus * delta_minus) / (delta_plus + delta_minus))) / F.h;
       }
       const double wo = outside ? wp : -1.0 * wm; // of the own block
-      for (int q = 0; q < Q.npts; ++q) {
-        double s, tt, wq;
-        face_qp<D - 1>(P.qtab, Q, q, s, tt, wq);
-        double pin[ND], pout[ND];
-        if constexpr (T::SIMPLEX) {
+      if constexpr (T::SIMPLEX) {
+        // sums over the points of the basis functions (by face corner; row 3: the function that vanishes there) and of
+        // their products
+        double m1[4] = {0., 0., 0., 0.}, m2[3][3];
+#pragma unroll
+        for (int a = 0; a < 3; ++a)
+#pragma unroll
+          for (int c = 0; c < 3; ++c)
+            m2[a][c] = 0.;
+        for (int q = 0; q < Q.npts; ++q) {
+          double s, tt, wq;
+          face_qp<D - 1>(P.qtab, Q, q, s, tt, wq);
           const double lam[3] = {D == 2 ? 1. - s : 1. - s - tt, s, tt};
 #pragma unroll
-          for (int i = 0; i < ND; ++i) {
-            pin[i] = win_at[i] == 0 ? lam[0] : win_at[i] == 1 ? lam[1] : win_at[i] == 2 ? lam[2] : 0.;
-            pout[i] = wout_at[i] == 0 ? lam[0] : wout_at[i] == 1 ? lam[1] : wout_at[i] == 2 ? lam[2] : 0.;
-          }
-        } else {
-          double X[D], Gin[ND][D], Gout[ND][D];
-          F.point(s, tt, X);
-          eval_at<GEOM, 1>(gin, X, pin, Gin);
-          eval_at<GEOM, 1>(gout, X, pout, Gout);
+          for (int a = 0; a < D; ++a) {
+            m1[a] += lam[a] * wq;
 #pragma unroll
-          for (int i = 0; i < ND; ++i) {
-            fin[i] = flux<D>(kin, Gin[i], n, Kin);
-            fout[i] = flux<D>(kout, Gout[i], n, Kout);
+            for (int c = a; c < D; ++c)
+              m2[a][c] += lam[a] * lam[c] * wq;
           }
         }
-        const double factor = F.ie * wq;
-        double ps[ND];
-#pragma unroll
-        for (int i = 0; i < ND; ++i)
-          ps[i] = outside ? pout[i] : pin[i];
+        const double factor = sc * F.ie;
+        auto pick = [](int k, double a, double c, double d) { return k == 0 ? a : k == 1 ? c : k == 2 ? d : 0.; };
         if (coupling) {
-          double fs[ND];
+          double pin[ND], pout[ND];
 #pragma unroll
-          for (int i = 0; i < ND; ++i)
-            fs[i] = outside ? fout[i] : fin[i];
+          for (int i = 0; i < ND; ++i) {
+            pin[i] = factor * pick(win_at[i], m1[0], m1[1], m1[2]);
+            pout[i] = factor * pick(wout_at[i], m1[0], m1[1], m1[2]);
+          }
 #pragma unroll
-          for (int i = 0, k = 0; i < ND; ++i)
+          for (int i = 0, k = 0; i < ND; ++i) {
+            const double psi = outside ? pout[i] : pin[i], fsi = prm * wo * (outside ? fout[i] : fin[i]);
 #pragma unroll
             for (int j = i; j < ND; ++j, ++k)
-              own[k] += sc * ((wo * fs[j] * ps[i] + prm * wo * ps[j] * fs[i]) * factor);
+              own[k] += wo * (outside ? fout[j] : fin[j]) * psi + (outside ? pout[j] : pin[j]) * fsi;
+          }
 #pragma unroll
           for (int i = 0; i < ND; ++i)
 #pragma unroll
             for (int j = 0; j < ND; ++j)
-              C[i][j] += sc * ((-1.0 * wp * fout[j] * pin[i] + prm * wm * pout[j] * fin[i]) * factor);
+              C[i][j] += -1.0 * wp * fout[j] * pin[i] + prm * wm * pout[j] * fin[i];
         } else {
+          const double pf = pen * factor;
 #pragma unroll
-          for (int i = 0, k = 0; i < ND; ++i)
+          for (int i = 0, k = 0; i < ND; ++i) {
+            // row of the products for the own vertex i, and for the inside's vertex i
+            const int wi = outside ? wout_at[i] : win_at[i];
+            double ro[3], ri[3];
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+              const double x0 = m2[0][c], x1 = c < 1 ? m2[0][1] : m2[1][c], x2 = c < 2 ? m2[c][2] : m2[2][2];
+              ro[c] = pf * pick(wi, x0, x1, x2);
+              ri[c] = -pf * pick(win_at[i], x0, x1, x2);
+            }
 #pragma unroll
             for (int j = i; j < ND; ++j, ++k)
-              own[k] += sc * ((pen * ps[j] * ps[i]) * factor);
-#pragma unroll
-          for (int i = 0; i < ND; ++i)
+              own[k] += pick(outside ? wout_at[j] : win_at[j], ro[0], ro[1], ro[2]);
 #pragma unroll
             for (int j = 0; j < ND; ++j)
-              C[i][j] += sc * ((-1.0 * pen * pout[j] * pin[i]) * factor);
+              C[i][j] += pick(wout_at[j], ri[0], ri[1], ri[2]);
+          }
+        }
+      } else {
+        for (int q = 0; q < Q.npts; ++q) {
+          double s, tt, wq;
+          face_qp<D - 1>(P.qtab, Q, q, s, tt, wq);
+          double pin[ND], pout[ND];
+          {
+            double X[D], Gin[ND][D], Gout[ND][D];
+            F.point(s, tt, X);
+            eval_at<GEOM, 1>(gin, X, pin, Gin);
+            eval_at<GEOM, 1>(gout, X, pout, Gout);
+#pragma unroll
+            for (int i = 0; i < ND; ++i) {
+              fin[i] = flux<D>(kin, Gin[i], n, Kin);
+              fout[i] = flux<D>(kout, Gout[i], n, Kout);
+            }
+          }
+          const double factor = F.ie * wq;
+          double ps[ND];
+#pragma unroll
+          for (int i = 0; i < ND; ++i)
+            ps[i] = outside ? pout[i] : pin[i];
+          if (coupling) {
+            double fs[ND];
+#pragma unroll
+            for (int i = 0; i < ND; ++i)
+              fs[i] = outside ? fout[i] : fin[i];
+#pragma unroll
+            for (int i = 0, k = 0; i < ND; ++i)
+#pragma unroll
+              for (int j = i; j < ND; ++j, ++k)
+                own[k] += sc * ((wo * fs[j] * ps[i] + prm * wo * ps[j] * fs[i]) * factor);
+#pragma unroll
+            for (int i = 0; i < ND; ++i)
+#pragma unroll
+              for (int j = 0; j < ND; ++j)
+                C[i][j] += sc * ((-1.0 * wp * fout[j] * pin[i] + prm * wm * pout[j] * fin[i]) * factor);
+          } else {
+#pragma unroll
+            for (int i = 0, k = 0; i < ND; ++i)
+#pragma unroll
+              for (int j = i; j < ND; ++j, ++k)
+                own[k] += sc * ((pen * ps[j] * ps[i]) * factor);
+#pragma unroll
+            for (int i = 0; i < ND; ++i)
+#pragma unroll
+              for (int j = 0; j < ND; ++j)
+                C[i][j] += sc * ((-1.0 * pen * pout[j] * pin[i]) * factor);
+          }
         }
       }
     }
@@ -1126,7 +1191,10 @@ __global__ void __launch_bounds__(256) k_dg_rows(FaceParams P, DgRows R)
     rank_own += id[k] >= 0 && id[k] < int(E);
     rank += id[k] >= 0 && id[k] < nbr;
   }
-  double* __restrict__ out = R.values + R.row0[E];
+  const int64_t begin = R.row0[(t - lane) >> 2], end = R.row0[min(((t - lane) >> 2) + 16, R.ne)];
+  double* const mine = rows[threadIdx.x >> 6];
+  auto place = [](int k) { return k + ((k >> 5) << 1); };
+  const int at0 = int(R.row0[E] - begin);
   const int L = blocks * ND;
 #pragma unroll
   for (int i = 0, k = 0; i < ND; ++i)
@@ -1142,11 +1210,11 @@ __global__ void __launch_bounds__(256) k_dg_rows(FaceParams P, DgRows R)
   // lane i stores row i of the own block
 #pragma unroll
   for (int i = 0; i < ND; ++i)
-    if (f == i) {
+    if (live && f == i) {
 #pragma unroll
       for (int j = 0; j < ND; ++j) {
         const int a = i < j ? i : j, b = i < j ? j : i;
-        out[i * L + rank_own * ND + j] = own[a * ND - a * (a - 1) / 2 + b - a];
+        mine[place(at0 + i * L + rank_own * ND + j)] = own[a * ND - a * (a - 1) / 2 + b - a];
       }
     }
   if (nbr >= 0) {
@@ -1154,8 +1222,14 @@ __global__ void __launch_bounds__(256) k_dg_rows(FaceParams P, DgRows R)
     for (int i = 0; i < ND; ++i)
 #pragma unroll
       for (int j = 0; j < ND; ++j)
-        out[i * L + rank * ND + j] = outside ? C[j][i] : C[i][j];
+        mine[place(at0 + i * L + rank * ND + j)] = outside ? C[j][i] : C[i][j];
   }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  double* __restrict__ out = R.values + begin;
+  for (int k = lane; k < int(end - begin); k += 64)
+    out[k] = mine[place(k)];
 }
 
 // block K of the four blocks of an inner intersection between elements of types GIN (inside) and GOUT

@@ -299,7 +299,7 @@ struct ScatterMaps {
   // 2 (inner intersection) + (1: the element is its outside), or -1 - (boundary intersection), or NO_FACE
   static constexpr int32_t NO_FACE = INT32_MIN;
   DeviceArray<int32_t> d_face_code;
-  DeviceArray<int64_t> d_elem_row; // first CSR slot of every element
+  DeviceArray<int64_t> d_elem_row; // first CSR slot of every element, and the end
   bool dg_rows = false;
   bool built = false;
   int nforms_built = -1; // which form set the maps were built for (element/face/source presence)

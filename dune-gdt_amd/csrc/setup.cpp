@@ -715,7 +715,7 @@ void Operator::build_scatter_maps()
                                    nf <= 4 && has_c && nin < (int64_t(1) << 29) && n == ls * ne};
   if (rows_of_blocks) {
     std::vector<int32_t> code(size_t(ne) * nf, ScatterMaps::NO_FACE);
-    std::vector<int64_t> first(ne);
+    std::vector<int64_t> first(ne + 1, nnz);
     parallel_for(ne, [&](int64_t e0, int64_t e1) {
       for (int64_t e = e0; e < e1 && rows_of_blocks; ++e) {
         int64_t col[5] = {e}, cnt = 1;
