@@ -951,11 +951,14 @@ __global__ void __launch_bounds__(256) k_inner_local(FaceParams P)
 // accumulators instead of 128 (2 waves per SIMD instead of 1) and neither writes and reads back the blocks of the
 // intersections (512 bytes each) nor reads a list of contributions (4 bytes each).  On simplices the sums over a face's
 // points are taken once per form (the normal derivatives are constant), and the rows of 16 elements leave through LDS in
-// whole lines.  P1 on 82 944 tetrahedra (6.4 million entries): 77 + 58 us -> 54 us, with the last two 47 us.  Bound by the
-// geometries, which every element has evaluated by its four lanes and by those of its neighbours.
+// whole lines.  On simplices the geometry is read from a table made once per operator (112 bytes per tetrahedron): an
+// element's four lanes and those of its neighbours would each evaluate it.  P1 on 82 944 tetrahedra (6.4 million entries):
+// 77 + 58 us -> 54 us, with the sums and whole lines 47 us, with the table 41 us, of which the 53 MB of values take 11.
+// Bound by loads and arithmetic that two waves per SIMD (220 registers) do not overlap.
 struct DgRows {
   int64_t ne;
   const int32_t* code;
+  const double* simplex;
   const int64_t* row0; // ne + 1
   const double* staging;
   int64_t bnd_base;
@@ -975,6 +978,30 @@ __device__ __forceinline__ double lane_of_4(double v)
   return __hiloint2double(lane_of_4<K>(__double2hiint(v)), lane_of_4<K>(__double2loint(v)));
 }
 
+// geometry of a grid's simplices, as ScatterMaps::d_simplex holds it
+template <int GEOM>
+__global__ void __launch_bounds__(256) k_simplex_geometry(const double* __restrict__ coords, const int32_t* __restrict__ conn,
+                                                          int64_t ne, double* __restrict__ out)
+{
+  constexpr int D = Traits<GEOM>::D;
+  const int64_t e = xcd_index(ne);
+  if (e >= ne)
+    return;
+  Geo<D> g;
+  load_geometry<GEOM>(coords, conn, e, g);
+#pragma unroll
+  for (int a = 0; a < D; ++a)
+#pragma unroll
+    for (int b = 0; b < D; ++b)
+      out[int64_t(a * D + b) * ne + e] = g.Ji[a][b];
+  out[int64_t(D * D) * ne + e] = g.det;
+  for (int f = 0; f <= D; ++f) {
+    FaceFrame<D> F;
+    face_frame<GEOM>(coords, conn, e, f, F);
+    out[int64_t(D * D + 1 + f) * ne + e] = F.h;
+  }
+}
+
 template <int GEOM>
 __global__ void __launch_bounds__(256) k_dg_rows(FaceParams P, DgRows R)
 {
@@ -992,8 +1019,9 @@ __global__ void __launch_bounds__(256) k_dg_rows(FaceParams P, DgRows R)
   const bool live = t < 4 * R.ne; // (whole elements)
   const int64_t E = min(t >> 2, R.ne - 1);
   const int f = int(t & 3);
-  const int32_t code = live && f < NF ? R.code[E * NF + f] : ScatterMaps::NO_FACE;
-  const bool outside = code & 1;
+  const int2 entry = live && f < NF ? reinterpret_cast<const int2*>(R.code)[E * NF + f] : make_int2(ScatterMaps::NO_FACE, 0);
+  const int32_t code = entry.x;
+  const bool outside = entry.y & 1;
   double own[NU], C[ND][ND]; // own block; in_out block (rows of the inside)
 #pragma unroll
   for (int k = 0; k < NU; ++k)
@@ -1005,31 +1033,55 @@ __global__ void __launch_bounds__(256) k_dg_rows(FaceParams P, DgRows R)
       C[i][j] = 0.;
   int nbr = -1;
   if (code >= 0) {
-    const int64_t fi = code >> 1;
-    const int64_t e = P.faces[4 * fi + 0], o = P.faces[4 * fi + 2];
-    nbr = int(outside ? e : o);
+    nbr = code;
+    const int64_t e = outside ? nbr : E, o = outside ? E : nbr;
+    const int fe = (entry.y >> 1) & 7;
     Geo<D> gin, gout;
-    load_geometry<GEOM>(P.coords, P.conn, e, gin);
-    load_geometry<GEOM>(P.coords, P.conn, o, gout);
     FaceFrame<D> F;
-    face_frame<GEOM>(P.coords, P.conn, e, P.faces[4 * fi + 1], F);
-    const double* n = F.n;
     // simplices: the basis functions at a point of the face are the point's barycentric coordinates; which of them belongs
     // to a vertex of the elements (3: none, the vertex is opposite to the face)
     int win_at[ND], wout_at[ND];
     if constexpr (T::SIMPLEX) {
-      const int fe = P.faces[4 * fi + 1];
-      int32_t v[3] = {-1, -1, -1};
+      const int64_t ne = R.ne;
 #pragma unroll
-      for (int k = 0; k < D; ++k)
-        v[k] = P.conn[e * T::NV + face_vertex<GEOM>(fe, k)];
+      for (int a = 0; a < D; ++a)
+#pragma unroll
+        for (int c = 0; c < D; ++c) {
+          gin.Ji[a][c] = R.simplex[int64_t(a * D + c) * ne + e];
+          gout.Ji[a][c] = R.simplex[int64_t(a * D + c) * ne + o];
+        }
+      F.h = R.simplex[(D * D + 1 + fe) * ne + e];
+      // the gradient of the coordinate that vanishes on the face points inward, one over the height long: the
+      // integration element is |det J| over the height
+      double gr[D], len = 0.;
+#pragma unroll
+      for (int c = 0; c < D; ++c) {
+        double first = 0.;
+#pragma unroll
+        for (int a = 0; a < D; ++a)
+          first -= gin.Ji[a][c];
+        gr[c] = first;
+#pragma unroll
+        for (int a = 0; a < D; ++a)
+          gr[c] = D - fe == a + 1 ? gin.Ji[a][c] : gr[c];
+        len += gr[c] * gr[c];
+      }
+      len = sqrt(len);
+      F.ie = R.simplex[int64_t(D * D) * ne + e] * len;
+#pragma unroll
+      for (int c = 0; c < D; ++c)
+        F.n[c] = -gr[c] / len;
 #pragma unroll
       for (int i = 0; i < ND; ++i) {
-        const int32_t a = P.conn[e * T::NV + i], b = P.conn[o * T::NV + i];
-        win_at[i] = a == v[0] ? 0 : a == v[1] ? 1 : a == v[2] ? 2 : 3;
-        wout_at[i] = b == v[0] ? 0 : b == v[1] ? 1 : b == v[2] ? 2 : 3;
+        win_at[i] = i == D - fe ? 3 : i - (i > D - fe ? 1 : 0);
+        wout_at[i] = (entry.y >> (4 + 2 * i)) & 3;
       }
+    } else {
+      load_geometry<GEOM>(P.coords, P.conn, e, gin);
+      load_geometry<GEOM>(P.coords, P.conn, o, gout);
+      face_frame<GEOM>(P.coords, P.conn, e, fe, F);
     }
+    const double* n = F.n;
     for (int fm = 0; fm < P.nforms; ++fm) {
       const double kin = P.kappa[fm] ? P.kappa[fm][e] : P.kappa_value[fm];
       const double kout = P.kappa[fm] ? P.kappa[fm][o] : P.kappa_value[fm];
@@ -2317,7 +2369,19 @@ void launch_assembly(Operator& op, hipStream_t stream, bool matrix)
   }
   if (rows) {
     C.faces = M.d_inner.ptr, C.coords = g.d_coords.ptr, C.conn = g.d_conn.ptr, C.qtab = op.d_qtab_line.ptr;
-    DgRows R{g.ne, M.d_face_code.ptr, M.d_elem_row.ptr, op.d_staging.ptr, M.bnd_base, !op.eforms.empty(),
+    if (g.ref.geom != HGDT_QUAD && !M.d_simplex.ptr) { // (set-up)
+      DeviceArray<double>& G = op.maps.d_simplex;
+      const int D = g.ref.dim;
+      G.allocate(size_t(D * D + 2 + D) * g.ne);
+      const dim3 all(xcd_grid(g.ne, 256));
+      if (D == 2)
+        hipLaunchKernelGGL(k_simplex_geometry<HGDT_TRI>, all, dim3(256), 0, stream, g.d_coords.ptr, g.d_conn.ptr, g.ne, G.ptr);
+      else
+        hipLaunchKernelGGL(k_simplex_geometry<HGDT_TET>, all, dim3(256), 0, stream, g.d_coords.ptr, g.d_conn.ptr, g.ne, G.ptr);
+      HGDT_HIP(hipGetLastError());
+      HGDT_HIP(hipStreamSynchronize(stream)); // other streams may assemble next
+    }
+    DgRows R{g.ne, M.d_face_code.ptr, M.d_simplex.ptr, M.d_elem_row.ptr, op.d_staging.ptr, M.bnd_base, !op.eforms.empty(),
              !op.bforms.empty() && nbd > 0, op.d_values.ptr};
     const dim3 grid(xcd_grid(4 * g.ne, 256));
     switch (g.ref.geom) {

@@ -296,10 +296,12 @@ struct ScatterMaps {
   DeviceArray<uint32_t> d_rhs_ptr, d_rhs_contrib;
   DeviceArray<int32_t> d_inner, d_bnd; // packed (e_in, f_in, e_out, f_out) / (e, f)
   // discontinuous spaces whose rows hold the element's and its neighbours' blocks and nothing else: per element and face
-  // 2 (inner intersection) + (1: the element is its outside), or -1 - (boundary intersection), or NO_FACE
+  // the neighbour, or -1 - (boundary intersection), or NO_FACE; and for an inner intersection 1 (the element is its
+  // outside) + 2 (local face of the inside) + 16 (simplices: corner of the face of the outside's vertices, 2 bits each)
   static constexpr int32_t NO_FACE = INT32_MIN;
   DeviceArray<int32_t> d_face_code;
   DeviceArray<int64_t> d_elem_row; // first CSR slot of every element, and the end
+  DeviceArray<double> d_simplex; // their geometry, entry-major: inverse Jacobian, |det J|, diameters of the faces
   bool dg_rows = false;
   bool built = false;
   int nforms_built = -1; // which form set the maps were built for (element/face/source presence)

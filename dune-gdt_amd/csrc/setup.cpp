@@ -714,7 +714,9 @@ void Operator::build_scatter_maps()
   std::atomic<bool> rows_of_blocks{s.kind == HGDT_DISCONTINUOUS_LAGRANGE && !g.mixed && square() && !borrowed && ls <= 4 &&
                                    nf <= 4 && has_c && nin < (int64_t(1) << 29) && n == ls * ne};
   if (rows_of_blocks) {
-    std::vector<int32_t> code(size_t(ne) * nf, ScatterMaps::NO_FACE);
+    std::vector<int32_t> code(2 * size_t(ne) * nf, ScatterMaps::NO_FACE);
+    const bool simplex = g.ref.geom == HGDT_TRI || g.ref.geom == HGDT_TET;
+    const int nv = g.ref.nverts, D = g.ref.dim;
     std::vector<int64_t> first(ne + 1, nnz);
     parallel_for(ne, [&](int64_t e0, int64_t e1) {
       for (int64_t e = e0; e < e1 && rows_of_blocks; ++e) {
@@ -725,10 +727,22 @@ void Operator::build_scatter_maps()
           if (o >= 0) {
             const int32_t fi = o > e ? inner_index[e * nf + f] : inner_index[o * nf + g.nbface[e * nf + f]];
             ok = ok && fi >= 0 && (o > e ? M.inner_out[fi] == o : M.inner_in[fi] == o && M.inner_out[fi] == e);
-            code[e * nf + f] = 2 * fi + (o > e ? 0 : 1);
             col[cnt++] = o;
+            if (!ok)
+              break;
+            const int64_t in = M.inner_in[fi], out = M.inner_out[fi];
+            const int fin = M.inner_fin[fi];
+            int32_t bits = (o > e ? 0 : 1) | fin << 1;
+            for (int i = 0; simplex && i < nv; ++i) { // corner of the face that vertex i of the outside is (3: none)
+              int corner = 3;
+              for (int c = 0; c < D; ++c)
+                if (g.conn[out * nv + i] == g.conn[in * nv + c + (c >= D - fin ? 1 : 0)])
+                  corner = c;
+              bits |= corner << (4 + 2 * i);
+            }
+            code[2 * (e * nf + f)] = int32_t(o), code[2 * (e * nf + f) + 1] = bits;
           } else if (bnd_index[e * nf + f] >= 0) {
-            code[e * nf + f] = -1 - bnd_index[e * nf + f];
+            code[2 * (e * nf + f)] = -1 - bnd_index[e * nf + f];
           }
         }
         std::sort(col, col + cnt);
@@ -749,6 +763,7 @@ void Operator::build_scatter_maps()
     }
   }
   M.dg_rows = rows_of_blocks;
+  M.d_simplex.release();
   d_staging.allocate(std::max<int64_t>(M.staging_size, 1));
   M.built = true;
   M.signature = signature;
