@@ -24,7 +24,8 @@
 //
 // Measured (us per iteration, three kernels -> one launch): Q1 32^2 15 -> 2.7, 128^2 14 -> 4.5, 701x523 18 -> 7.8, 1023^2
 // 33 -> 11.8, P1 48^3 x 6 18 -> 7.0, eight of these in a batch 33 -> 9.4, 100^3 x 6 34 -> 19, 128^3 x 6 54 -> 27; SELL: P1
-// triangles of a mesh with 160 401 vertices 18 -> 7.0, P2 triangles with 90 201 DoFs 18 -> 7.5.
+// triangles of a mesh with 160 401 vertices 18 -> 7.0, P2 triangles with 90 201 DoFs 18 -> 7.5; Q1 hexahedra (13 upper
+// diagonals, read in every step) 20^3 15.2 -> 6.8, 40^3 16.1 -> 10.3, 63^3 21.7 -> 16.3.
 // What bounds an iteration now: small problems two exchanges of 1-2.5 us, the barriers and sums around them; 4096 rows
 // per workgroup LDS (13 reads of 8 bytes per row at 128 B per clock: 1.4 us) and registers (a variant that spilled 46 took
 // 19 us instead of 11.8 at 1023^2: the scratch of 256 workgroups evicts L2); 128^3 x 6 the published p (17 MB of
@@ -49,7 +50,7 @@ namespace {
 
 constexpr bool q_in_lds(int slots, int nu, bool far)
 {
-  return far || slots > 8 || (slots == 8 && nu == 4);
+  return far || slots > 8 || (slots == 8 && nu >= 4);
 }
 
 // PCG of the tasks of one workgroup, one after the other.  Lane t holds rows t, t + T, ... of the workgroup,
@@ -391,7 +392,7 @@ __global__ void __launch_bounds__(T) k_pcg_resident(ResidentParams P)
       };
       if constexpr (FAR)
         far_ask(0, 0);
-      constexpr int G = S < 2 || (KEEP && S == 8 && NU == 4) ? 1 : 2; // slots whose loads are in flight together
+      constexpr int G = S < 2 || NU > 4 || (KEEP && S == 8 && NU == 4) ? 1 : 2; // slots whose loads are in flight together
 #pragma unroll
       for (int s0 = 0; s0 < S; s0 += G) {
         double ml[G][MU], mu[G][MU], xl[G][MU], xu[G][MU], xc[G];
@@ -630,6 +631,22 @@ Kernel kernel_for(int slots, int lg, bool same)
   return nullptr;
 }
 
+// up to RES_WIDE strict upper slots (Q1 on hexahedra): the matrix is read in every step
+constexpr int RES_WIDE = 13;
+Kernel wide_kernel(int slots, int lg, bool same)
+{
+  if (same)
+    switch (slots * 16 + lg) {
+      case 16:
+        return k_pcg_resident<RES_LANES, 1, 0, true, RES_WIDE, 0>;
+      case 33:
+        return k_pcg_resident<RES_LANES, 2, 1, true, RES_WIDE, 0>;
+      case 66:
+        return k_pcg_resident<RES_LANES, 4, 2, true, RES_WIDE, 0>;
+    }
+  return nullptr;
+}
+
 // FAR: blocks of RES_FAR_BLOCK lanes and 4 rows per lane
 Kernel far_kernel(int slots)
 {
@@ -658,7 +675,7 @@ Kernel kernel_of(int slots, int lg, bool same, int nu)
     }
     return nullptr;
   }
-  return nu <= 3 ? kernel_for<3>(slots, lg, same) : kernel_for<4>(slots, lg, same);
+  return nu <= 3 ? kernel_for<3>(slots, lg, same) : nu <= 4 ? kernel_for<4>(slots, lg, same) : wide_kernel(slots, lg, same);
 }
 
 // CUs of a device in use by resident launches of this process
@@ -707,10 +724,16 @@ static int64_t team_of(int64_t rows, int slots, int lanes = RES_LANES)
 // short, few rows the steps between them.  Measured (Q1, us per iteration with 1 / 2 / 4 / 8 rows per lane): 1 089 rows
 // 4.5 / 4.2 / 2.7 / 4.3 (one workgroup: no exchange); 4 096 4.2 / 3.9 / 4.3 / 4.4; 16 384 5.0 / 4.4 / 5.0 / 6.2; 65 536 6.4 / 5.3 / 5.3 / 6.7; 131 044 8.0 / 7.9 / 5.7 / 7.1;
 // 262 144 - / - / 7.8 / 7.5.  SELL: 160 401 rows of 7 entries - / 8.5 / 7.6 / 13.4, 90 201 of 11 8.6 / 8.0 / 14.8 / 23
-static bool enough_rows(int64_t rows, int slots, int cus, bool sell)
+// More than 4 upper slots (hexahedra): 1 000 rows 6.6 / 4.6 / 7.5, 2 197 6.8 / 8.1 / 10.9, 19 683 7.1 / 8.4 / 11.0, 35 937
+// 9.3 / 9.2 / 11.7, 68 921 12.5 / 10.5 / 12.2, 132 651 - / 14.8 / 13.8 / 20.7, 300 763 - / - / 17.2 / 23.0 (three kernels:
+// 13.6, 15.7, 15.7, 15.1, 16.0, 17.9, 25); 8 rows per lane are not compiled.
+enum RowKind { ROWS_DIA, ROWS_WIDE, ROWS_SELL };
+static bool enough_rows(int64_t rows, int slots, int cus, RowKind kind)
 {
   const int64_t w = team_of(rows, slots);
-  if (sell) // (a row costs more: 9 to 20 scattered reads of LDS)
+  if (kind == ROWS_WIDE)
+    return slots == 1 ? w <= 1 || (w > 2 && w <= cus / 5) : slots == 2 ? w <= cus / 3 : w <= cus;
+  if (kind == ROWS_SELL) // (a row costs more: 9 to 20 scattered reads of LDS)
     return slots == 1 ? w <= cus / 16 : slots <= 4 ? w <= cus / 2 : w <= cus;
   return slots == 1 ? w <= 1 : slots == 2 ? w <= (rows <= 4 * RES_LANES ? 1 : cus / 8) : slots == 4 ? w <= cus / 4 : w <= cus;
 }
@@ -751,28 +774,30 @@ double resident_schedule(const std::vector<int64_t>& row0, const std::vector<int
 }
 
 // us per iteration of one workgroup with 1, 2, 4, 8, 16 rows per lane (measured)
-static double step_of(int slots)
+static double step_of(int slots, RowKind kind = ROWS_DIA)
 {
+  if (kind == ROWS_WIDE)
+    return slots == 1 ? 3.3 : slots == 2 ? 4.6 : 7.5;
   return slots == 1 ? 1.8 : slots == 2 ? 2.1 : slots == 4 ? 2.7 : slots == 8 ? 4.3 : 10.;
 }
 
 // rows per lane: -1 when no choice of `fits` (LDS, compiled variant) takes all instances
 template <class F>
-static int choose_slots(const std::vector<int64_t>& row0, bool sell, bool given, F fits)
+static int choose_slots(const std::vector<int64_t>& row0, RowKind kind, bool given, F fits)
 {
   const int cus = device_cus();
   int best = -1;
   double time = 0.;
   for (int s : {1, 2, 4, 8, 16}) {
     if (row0.size() == 2) {
-      if (enough_rows(row0[1] - row0[0], s, cus, sell) && fits(s))
+      if (enough_rows(row0[1] - row0[0], s, cus, kind) && fits(s))
         return s;
       continue;
     }
     std::vector<int> teams;
     for (size_t i = 0; i + 1 < row0.size(); ++i)
       teams.push_back(int(std::min<int64_t>(team_of(row0[i + 1] - row0[i], s), 1 << 20)));
-    const double t = resident_schedule(row0, teams, step_of(s), nullptr, nullptr);
+    const double t = resident_schedule(row0, teams, step_of(s, kind), nullptr, nullptr);
     if (t >= 0. && (best < 0 || t < time) && fits(s))
       best = s, time = t;
   }
@@ -825,10 +850,12 @@ int64_t resident_padding(const std::vector<int64_t>& row0, const std::vector<std
 ResidentShape resident_shape_dia(const std::vector<int64_t>& row0, const std::vector<std::vector<int64_t>>& s_offs,
                                  int s_nu)
 {
-  if (s_nu < 0 || s_nu > 4)
+  if (s_nu < 0 || s_nu > RES_WIDE)
     return {};
   const int64_t reach = reach_of(row0, s_offs);
-  const int s = choose_slots(row0, false, false, [&](int k) { return lds_of(k, reach, s_nu) <= RES_LDS && !(s_nu == 0 && k > 8); });
+  const int s = choose_slots(row0, s_nu > 4 ? ROWS_WIDE : ROWS_DIA, false, [&](int k) {
+    return lds_of(k, reach, s_nu) <= RES_LDS && !(s_nu == 0 && k > 8) && !(s_nu > 4 && k > 4);
+  });
   if (s > 0)
     return {RES_LANES, std::min(s, 8)}; // (16 rows per lane: two blocks of 8 each)
   if (far_slots(row0, s_offs, s_nu))
@@ -935,7 +962,7 @@ void resident_plan_dia(ResidentPlan& plan, const Operator& op, const std::vector
     return;
   }
   const bool same = bv == RES_LANES && F.A.block == bv && F.A.items == iv;
-  if (s_nu < 0 || s_nu > 4 || RES_LANES % bv != 0 || !(same || (F.A.items == 1 && ba <= 1024 && (ba & (ba - 1)) == 0)))
+  if (s_nu < 0 || s_nu > RES_WIDE || RES_LANES % bv != 0 || !(same || (F.A.items == 1 && ba <= 1024 && (ba & (ba - 1)) == 0)))
     return;
   const std::vector<int64_t>& row0 = op.space->inst_dof;
   int lg = 0;
@@ -944,7 +971,7 @@ void resident_plan_dia(ResidentPlan& plan, const Operator& op, const std::vector
   if (lg > 0 && bv != RES_LANES)
     return;
   const int64_t reach = reach_of(row0, s_offs);
-  const int slots = choose_slots(row0, false, true, [&](int k) {
+  const int slots = choose_slots(row0, s_nu > 4 ? ROWS_WIDE : ROWS_DIA, true, [&](int k) {
     // (a diagonal matrix holds no slot to stream)
     return (int64_t(k) * RES_LANES) % ba == 0 && kernel_of(k, lg, same, s_nu) && lds_of(k, reach, s_nu) <= RES_LDS &&
            !(s_nu == 0 && k > 8);
@@ -955,7 +982,7 @@ void resident_plan_dia(ResidentPlan& plan, const Operator& op, const std::vector
   if (!list_tasks(op, slots, RES_LANES, tasks))
     return;
   plan.slots = slots, plan.lg_items = lg, plan.same_blocks = same, plan.nu = s_nu;
-  plan.step = step_of(plan.slots);
+  plan.step = step_of(plan.slots, s_nu > 4 ? ROWS_WIDE : ROWS_DIA);
   resident_finish(plan, op, tasks, lds_of(slots, reach, s_nu), F.A.nblocks, F.V.nblocks);
 }
 
@@ -973,7 +1000,7 @@ static void halo_of(const Operator& op, int64_t r0, int64_t r1, std::vector<int3
 int resident_items_sell(const Operator& op)
 {
   const std::vector<int64_t>& row0 = op.space->inst_dof;
-  const int s = choose_slots(row0, true, false, [&](int k) {
+  const int s = choose_slots(row0, ROWS_SELL, false, [&](int k) {
     if (k > 8)
       return false;
     // p of the own rows and the halo in LDS

@@ -16,7 +16,9 @@
 //
 // Jacobi-PCG runs as CG on the symmetrically scaled matrix D^{-1/2} A D^{-1/2} (same iterates in
 // exact arithmetic; the scaled matrix has a unit diagonal that is never stored or read, and the
-// preconditioner costs no vector), three launches per iteration, each one pass over its vectors:
+// preconditioner costs no vector).  A solve whose vectors fit on the chip is one launch (resident.hip,
+// resident_dg.hip); the others, timed ones, and those whose launch gave up take three launches per
+// iteration, each one pass over its vectors:
 //   k_cg_direction : stopping test from the previous update's partials; p = r + beta p into the other
 //                    of two p buffers; every second step x += the two updates deferred since
 //   k_cg_spmv      : q = Ah p and the block partials of p.q (k_cg_spmv_win: the same with the p entries

@@ -42,6 +42,17 @@ def test_one_launch_equals_three_kernels(hgdt_mod, kind, cells, workgroups):
     assert wg > 0 and (workgroups is None or wg == workgroups)
 
 
+@pytest.mark.parametrize("cells,taken", [
+    ([1, 1, 1], True), ([2, 3, 2], True), ([7, 7, 7], True), ([12, 9, 15], True), ([30, 31, 29], True),
+    ([55, 60, 61], True), ([61, 59, 120], True), ([96, 96, 20], False)])
+def test_thirteen_upper_diagonals(hgdt_mod, cells, taken):
+    """Q1 on hexahedra: the matrix read in every step; planes too large for LDS are left to the three kernels"""
+    print(f"case hex {cells}", flush=True)
+    space, op = _poisson(hgdt_mod, "hex", 1, cells, 13)
+    op.assemble()
+    assert (_both(hgdt_mod, op) > 0) == taken
+
+
 @pytest.mark.parametrize("apply,vector,taken", [
     ((64, 1), (64, 1), True), ((1024, 1), (512, 1), True), ((128, 1), (256, 1), True), ((512, 2), (512, 2), True),
     ((512, 8), (512, 8), True), ((256, 1), (256, 4), False), ((512, 4), (512, 2), False), ((512, 1), (64, 8), False),
