@@ -28,8 +28,8 @@
 // diagonals, read in every step) 20^3 15.2 -> 6.8, 40^3 16.1 -> 10.3, 63^3 21.7 -> 16.3.
 // What bounds an iteration now: small problems two exchanges of 1-2.5 us, the barriers and sums around them; 4096 rows
 // per workgroup LDS (13 reads of 8 bytes per row at 128 B per clock: 1.4 us) and registers (a variant that spilled 46 took
-// 19 us instead of 11.8 at 1023^2: the scratch of 256 workgroups evicts L2); 128^3 x 6 the published p (17 MB of
-// write-through stores at about 2.5 TB/s) and the matrix (68 MB read past L2).
+// 19 us instead of 11.8 at 1023^2: the scratch of 256 workgroups evicts L2); 128^3 x 6 the memory
+// behind the L2 caches (104 MB of matrix and far p read, 17 MB of p written per iteration: 4.3 TB/s, the rate of a copy).
 //
 // All workgroups of a team must be on the chip together: the host launches at most one per CU and counts the
 // CUs of all running launches of the process.  A wait that outlasts its limit (another process holds the
