@@ -22,7 +22,7 @@
 // the operator's and the vector partition, sums over the partials), so a solve gives the same bits on either path,
 // alone or in a batch.
 //
-// Measured (us per iteration, three kernels -> one launch): Q1 32^2 15 -> 2.7, 128^2 14 -> 4.5, 701x523 18 -> 7.8, 1023^2
+// Measured (us per iteration, three kernels -> one launch): Q1 32^2 15 -> 2.3, 128^2 14 -> 4.5, 701x523 18 -> 7.8, 1023^2
 // 33 -> 11.8, P1 48^3 x 6 18 -> 7.0, eight of these in a batch 33 -> 9.4, 100^3 x 6 34 -> 19, 128^3 x 6 54 -> 27; SELL: P1
 // triangles of a mesh with 160 401 vertices 18 -> 7.0, P2 triangles with 90 201 DoFs 18 -> 7.5; Q1 hexahedra (13 upper
 // diagonals, read in every step) 20^3 15.2 -> 6.8, 40^3 16.1 -> 10.3, 63^3 21.7 -> 16.3.

@@ -13,7 +13,7 @@
 // D^{-1/2}.  The sums of p.q and of the norms are those of the workgroups in their order: the three kernels
 // add the same terms in another order, so a solve agrees with theirs up to round-off and not bit for bit.
 // Measured (us per iteration, three kernels -> one launch): element blocks 256 x 192 elements 17.7 -> 5.1, matrix-free
-// 512 x 512 elements 23.6 -> 9.0.  What bounds an iteration now: the two exchanges (2.4-3.5 us each with 96-256
+// 512 x 512 elements 23.6 -> 8.7.  What bounds an iteration now: the two exchanges (2.4-3.5 us each with 96-256
 // workgroups) and the barriers around them.  More than 131 072 elements with their blocks do not fit in the
 // registers of 256 CUs, and reading 168 MB of blocks per step instead leaves nothing to gain; matrix-free 262 144 elements.
 
