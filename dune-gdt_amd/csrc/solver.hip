@@ -1480,6 +1480,15 @@ void RowPartition::build_counts(const std::vector<int64_t>& inst_dof, const std:
 static bool blk_wanted(const Operator& op);
 static int kernel_format(const Operator& op);
 
+// the same as resident_shape below once C.sell_items is known for the pattern (its slices need not be built yet)
+static ResidentShape resident_shape_sell(const Operator& op)
+{
+  const SolverCache& C = *op.solver_cache;
+  if (op.launch[3].user || op.launch[4].user || !op.square() || !C.sell_items)
+    return {};
+  return {RES_BLOCK, C.sell_items};
+}
+
 // row blocks that suit a solve in one launch (resident.hip; the operator's and the vector kernels' alike); none: the
 // caller chose shapes, or the storage (once it is known) or size does not fit
 static ResidentShape resident_shape(const Operator& op)
@@ -1488,7 +1497,7 @@ static ResidentShape resident_shape(const Operator& op)
   if (op.launch[3].user || op.launch[4].user || !op.square())
     return {};
   if (op.fmt.format == HGDT_FORMAT_SELL && op.fmt.structure_ready)
-    return C.sell_items ? ResidentShape{RES_BLOCK, C.sell_items} : ResidentShape{};
+    return resident_shape_sell(op);
   if (!op.fmt.valid || op.fmt.format != HGDT_FORMAT_DIA || kernel_format(op) != FMT_DIAS)
     return {};
   if (C.s_nu != C.shape_nu || C.s_offs != C.shape_offs) // (a batch's shape is a search over its instances)
@@ -1496,18 +1505,21 @@ static ResidentShape resident_shape(const Operator& op)
   return C.shape_dia;
 }
 
-// row-block partitions of the operator (host set-up, O(number of blocks))
-static void build_partitions(Operator& op)
+// row-block partitions of the operator (host set-up, O(number of blocks)), resident: its resident_shape.  The default
+// shape of the application depends on the caller's choice for either kernel, so a choice for the vector kernels alone can
+// change the operator's row blocks too: SELL slices follow these and are dropped with them, whatever the cause (the caller
+// goes through prepare_storage before they are read).
+static void build_partitions(Operator& op, const ResidentShape& resident)
 {
   SolverFormat& F = op.fmt;
   SolverCache& C = cache_of(op);
   const Space& s = *op.space;
+  const int sliced_block = F.A.block, sliced_items = F.A.items;
   // default launch shapes: one row per lane for the operator application (many blocks keep enough
   // loads in flight); the vector kernels take ~1024 blocks so that every block's reduction of an
   // instance's partials stays small
   if (!op.launch[3].user)
     op.launch[3].block = 256, op.launch[3].items = 1;
-  const ResidentShape resident = resident_shape(op);
   if (resident.block)
     op.launch[3].block = resident.block, op.launch[3].items = resident.items;
   // the matrix-free kernels give every lane one row (continuous spaces, at most 256 lanes per block) or one
@@ -1535,6 +1547,8 @@ static void build_partitions(Operator& op)
   F.d_inst_row0.upload(s.inst_dof);
   if (mf)
     mf_block_table(op);
+  if (F.format == HGDT_FORMAT_SELL && (F.A.block != sliced_block || F.A.items != sliced_items))
+    F.structure_ready = F.valid = false;
   F.partitions_ready = true;
   ++C.version; // captured graphs hold the launch shapes
 }
@@ -1920,9 +1934,8 @@ static void build_structure(Operator& op)
   } else {
     F.format = HGDT_FORMAT_SELL;
     C.sell_items = op.square() ? resident_items_sell(op) : 0;
-    F.structure_ready = true;
-    if (resident_shape(op) != C.shaped_for)
-      build_partitions(op); // (the slices follow the row blocks)
+    if (resident_shape_sell(op) != C.shaped_for)
+      build_partitions(op, resident_shape_sell(op)); // (the slices follow the row blocks)
     std::vector<int64_t> slice_ptr{0}, bslice0;
     for (int64_t b = 0; b < F.A.nblocks; ++b) {
       bslice0.push_back(int64_t(slice_ptr.size()) - 1);
@@ -2004,6 +2017,8 @@ static PcgParams make_params(Operator& op)
 {
   SolverFormat& F = op.fmt;
   SolverCache& C = cache_of(op);
+  if (F.format == HGDT_FORMAT_SELL && C.block_slice0.count != size_t(F.A.nblocks) + 1)
+    HGDT_THROW(HGDT_ERR_OPERATOR, "the slices of the SELL storage do not follow the operator's row blocks");
   PcgParams P{};
   P.n = op.n;
   P.a_nb = int(F.A.nblocks);
@@ -2076,11 +2091,11 @@ bool Operator::direct_applicable()
       return false;
   if (!(requested_format == HGDT_FORMAT_AUTO || requested_format == HGDT_FORMAT_DIA) || !allow_symmetric)
     return false;
+  SolverCache& C = cache_of(*this);
   if (!fmt.partitions_ready)
-    build_partitions(*this);
+    build_partitions(*this, resident_shape(*this));
   if (!fmt.structure_ready)
     build_structure(*this);
-  SolverCache& C = cache_of(*this);
   if (fmt.format != HGDT_FORMAT_DIA || fmt.ndiag != 15)
     return false;
   std::vector<DirectInst> rec(g.ninst());
@@ -2170,8 +2185,10 @@ void Operator::materialize_values(hipStream_t stream)
 void Operator::prepare_solver(hipStream_t stream)
 {
   prepare_storage(stream);
-  if (resident_shape(*this) != cache_of(*this).shaped_for) // default shapes follow the storage
-    build_partitions(*this);
+  if (const ResidentShape shape = resident_shape(*this); shape != cache_of(*this).shaped_for) {
+    build_partitions(*this, shape); // default shapes follow the storage
+    prepare_storage(stream);        // (and SELL slices the row blocks)
+  }
   // column windows for the current row blocks, on the device once the staged application is chosen
   // (set-up, never captured)
   SolverCache& C = cache_of(*this);
@@ -2187,7 +2204,7 @@ void Operator::prepare_storage(hipStream_t stream)
   SolverFormat& F = fmt;
   SolverCache& C = cache_of(*this);
   if (!F.partitions_ready)
-    build_partitions(*this);
+    build_partitions(*this, resident_shape(*this));
   if (!F.structure_ready)
     build_structure(*this);
   if (F.valid)
