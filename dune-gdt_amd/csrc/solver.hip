@@ -50,6 +50,7 @@
 
 #include "hgdt_internal.hpp"
 #include "block_reduce.hpp"
+#include "index_math.hpp"
 #include "resident.hpp"
 
 namespace hgdt {
@@ -308,23 +309,34 @@ __device__ __forceinline__ void apply_rows(const PcgParams& P, const double* __r
   }
 }
 
-// y = A x, one row per lane: a row block of 1 << lg rows per lane is handled by as many workgroups
-template <int FMT>
-__global__ void __launch_bounds__(1024) k_apply(PcgParams P, int lg, const double* __restrict__ x, double* __restrict__ y)
+// y = A x, one row per lane.  PLAIN: row blocks of as many rows as a workgroup has lanes.  Otherwise (several rows per
+// lane in the solver's kernels) `per` workgroups share a row block, as apply_split says.
+// Both are bound by the requests to L1 and L2 (values and x of 8 bytes per entry).  Measured (us per call): Q1 on 96^3
+// hexahedra, row blocks of 256 x 1, 36.2 in the plain form and 36.75 in the other (its division of the workgroup's number
+// ahead of the first load); P1 on 112 x 100 x 112 x 6 tetrahedra, row blocks of 768 x 4, 30.4 with workgroups of 768 lanes
+// and 29.2 with 256, which leave the CUs in smaller pieces.
+template <int FMT, bool PLAIN>
+__global__ void __launch_bounds__(1024) k_apply(PcgParams P, unsigned per, unsigned inv, const double* __restrict__ x,
+                                                double* __restrict__ y)
 {
-  const int w = logical_block(P.a_nb << lg);
+  const int w = logical_block(PLAIN ? P.a_nb : P.a_nb * int(per));
   if (w < 0)
     return;
-  const int b = w >> lg;
+  const int b = PLAIN || inv == 0 ? w : int(__umulhi(unsigned(w), inv));
   const int inst = P.a_inst[b];
-  const int64_t rb = P.a_row0[b], r1 = P.a_row0[b + 1], r0 = rb + int64_t(w - (b << lg)) * blockDim.x;
-  if (r0 >= r1)
-    return;
+  const int64_t rb = P.a_row0[b], r1 = P.a_row0[b + 1];
   const double* vals = (FMT == FMT_SELL) ? P.sell_vals : P.dia;
-  double acc[1];
-  apply_rows<FMT, 1, false>(P, vals, b, inst, rb, r0, r1, [&](int64_t c) { return x[c]; }, acc);
-  if (r0 + threadIdx.x < r1)
-    y[r0 + threadIdx.x] = acc[0];
+  auto rows = [&](int64_t r0) {
+    double acc[1];
+    apply_rows<FMT, 1, false>(P, vals, b, inst, rb, r0, r1, [&](int64_t c) { return x[c]; }, acc);
+    if (r0 + threadIdx.x < r1)
+      y[r0 + threadIdx.x] = acc[0];
+  };
+  if constexpr (PLAIN)
+    rows(rb);
+  else
+    for (int64_t r0 = rb + int64_t(w - b * int(per)) * blockDim.x; r0 < r1; r0 += int64_t(per) * blockDim.x)
+      rows(r0);
 }
 
 // 4 x 4 element blocks: y = A x over the 4 rows of element E (lane per element).  Each row sums its
@@ -2351,11 +2363,8 @@ void Operator::apply(const double* x, double* y, hipStream_t stream)
     return;
   }
   PcgParams P = make_params(*this);
-  const int block = fmt.A.block;
-  int lg = 0; // (items is a power of two)
-  while ((1 << lg) < fmt.A.items)
-    ++lg;
-  const unsigned grid = hw_blocks(fmt.A.nblocks << lg);
+  const ApplySplit split = apply_split(fmt.A.block, fmt.A.items, fmt.A.nblocks);
+  const unsigned grid = hw_blocks(fmt.A.nblocks * split.per);
   const int kf = kernel_format(*this);
   if (kf == FMT_BLK) {
     const unsigned g1 = xcd_grid(fmt.blk_ne, 256);
@@ -2366,12 +2375,16 @@ void Operator::apply(const double* x, double* y, hipStream_t stream)
     HGDT_HIP(hipGetLastError());
     return;
   }
+  auto launch = [&](auto plain, auto several) {
+    hipLaunchKernelGGL(fmt.A.items == 1 ? plain : several, dim3(grid), dim3(split.lanes), 0, stream, P, split.per, split.inv,
+                       x, y);
+  };
   if (kf == FMT_DIA)
-    hipLaunchKernelGGL(k_apply<FMT_DIA>, dim3(grid), dim3(block), 0, stream, P, lg, x, y);
+    launch(k_apply<FMT_DIA, true>, k_apply<FMT_DIA, false>);
   else if (kf == FMT_DIAS)
-    hipLaunchKernelGGL(k_apply<FMT_DIAS>, dim3(grid), dim3(block), 0, stream, P, lg, x, y);
+    launch(k_apply<FMT_DIAS, true>, k_apply<FMT_DIAS, false>);
   else
-    hipLaunchKernelGGL(k_apply<FMT_SELL>, dim3(grid), dim3(block), 0, stream, P, lg, x, y);
+    launch(k_apply<FMT_SELL, true>, k_apply<FMT_SELL, false>);
   HGDT_HIP(hipGetLastError());
 }
 
