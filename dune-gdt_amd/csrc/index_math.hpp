@@ -24,4 +24,12 @@ constexpr ApplySplit apply_split(int block, int items, int64_t nblocks)
   return {lanes, uint32_t(per), uint32_t(((uint64_t(1) << 32) + uint64_t(per) - 1) / uint64_t(per))};
 }
 
+// One-launch solves of general storage and of discontinuous spaces address the values that workgroups exchange from the
+// start of a vector of n doubles with 32-bit byte offsets, as one scalar base and an offset per lane.  Vectors beyond 4 GB
+// (batches: no single instance on the chip is that large) take the kernels per iteration.
+constexpr bool reached_by_32_bits(int64_t n)
+{
+  return n <= (int64_t(1) << 32) / int64_t(sizeof(double));
+}
+
 } // namespace hgdt

@@ -43,6 +43,7 @@
 #include <map>
 #include <mutex>
 
+#include "index_math.hpp"
 #include "resident_device.hpp"
 
 namespace hgdt {
@@ -999,6 +1000,8 @@ static void halo_of(const Operator& op, int64_t r0, int64_t r1, std::vector<int3
 
 int resident_items_sell(const Operator& op)
 {
+  if (!reached_by_32_bits(op.n))
+    return 0;
   const std::vector<int64_t>& row0 = op.space->inst_dof;
   const int s = choose_slots(row0, ROWS_SELL, false, [&](int k) {
     if (k > 8)
@@ -1030,7 +1033,8 @@ void resident_plan_sell(ResidentPlan& plan, const Operator& op)
   plan.usable = false;
   const SolverFormat& F = op.fmt;
   const int slots = F.V.items;
-  if (F.V.block != RES_LANES || F.A.block != RES_LANES || F.A.items != slots || slots > RES_MAX_SLOTS)
+  if (F.V.block != RES_LANES || F.A.block != RES_LANES || F.A.items != slots || slots > RES_MAX_SLOTS ||
+      !reached_by_32_bits(op.n))
     return;
   int lg = 0;
   while ((1 << lg) < slots)

@@ -20,6 +20,7 @@
 #include <algorithm>
 #include <cmath>
 
+#include "index_math.hpp"
 #include "mf_params.hpp"
 #include "resident_device.hpp"
 
@@ -567,7 +568,7 @@ void resident_plan_dg(ResidentPlan& plan, const Operator& op)
   const std::vector<int64_t>& row0 = sp.inst_dof;
   const int ninst = int(row0.size()) - 1;
   const bool mf = F.format == HGDT_FORMAT_MATRIX_FREE;
-  if (op.n % 4 != 0 || op.n / 4 >= (int64_t(1) << 30) || (mf ? F.mf_kind != MFK_DG_QUAD : F.blk_mn > 4))
+  if (op.n % 4 != 0 || !reached_by_32_bits(op.n) || (mf ? F.mf_kind != MFK_DG_QUAD : F.blk_mn > 4))
     return;
   for (int in = 0; in < ninst; ++in)
     if (row0[in + 1] == row0[in] || row0[in] % 4 != 0 || (mf && !on_lattice(op, in)))

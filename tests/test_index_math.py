@@ -38,3 +38,23 @@ def test_workgroups_of_an_application(tmp_path):
           return 1;
         }
       }""")
+
+
+def test_rows_reached_by_32_bit_offsets(tmp_path):
+    """the byte offset of a lane's value, computed in 32 bits, is the one in 64 bits for every row of every vector that is
+    admitted: 4 n DoFs by element too, up to the last (2^29 rows: 4 GB)"""
+    _run(tmp_path, r"""
+  int64_t largest = 0;
+  for (int64_t n = 4; n <= (int64_t(1) << 32); n += n < 1024 ? 4 : n / 64) {
+    for (int64_t m = n - 1; m <= n + 1; ++m)
+      if (reached_by_32_bits(m)) {
+        largest = m > largest ? m : largest;
+        if (int64_t(uint32_t(m - 1) * uint32_t(sizeof(double))) != (m - 1) * int64_t(sizeof(double)))
+          return 1;
+      }
+  }
+  const int64_t limit = int64_t(1) << 29;
+  if (!reached_by_32_bits(limit) || reached_by_32_bits(limit + 1) || reached_by_32_bits(2 * limit) || largest > limit)
+    return 1;
+  if (int64_t(uint32_t(limit - 1) * 8u) != (limit - 1) * 8 || int64_t(uint32_t(limit) * 8u) == limit * 8)
+    return 1;""")
