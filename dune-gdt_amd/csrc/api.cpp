@@ -1289,6 +1289,14 @@ hgdt_status hgdt_operator_solve_workgroups(hgdt_operator op, int32_t* workgroups
   });
 }
 
+hgdt_status hgdt_operator_set_solve_wait(hgdt_operator op, double seconds)
+{
+  return guarded([&] {
+    require(op && seconds >= 0. && seconds <= 1e6, HGDT_ERR_INVALID_ARGUMENT, "a wait of 0 to 1e6 seconds is needed");
+    op->op->solve_wait = seconds;
+  });
+}
+
 hgdt_status hgdt_operator_instance_true_residuals(hgdt_operator op, double* relres)
 {
   return guarded([&] {

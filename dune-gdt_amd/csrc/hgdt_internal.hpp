@@ -479,6 +479,7 @@ struct Operator {
   std::vector<int64_t> last_iters;
   std::vector<double> last_relres;
   std::vector<double> last_true_relres; // |b - A x| / |b| at exit (-1: not computed)
+  double solve_wait = 4.;               // seconds that a workgroup of a solve in one launch waits for another
   int32_t last_workgroups = 0;          // of the last solve in one launch (0: kernels per iteration)
 
   // Structured assembly (P1 on the Kuhn tetrahedra of axis-parallel lattices with Laplace element forms and

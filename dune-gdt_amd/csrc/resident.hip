@@ -929,6 +929,10 @@ void resident_finish(ResidentPlan& plan, const Operator& op, const std::vector<R
   plan.task_start.upload(start);
   plan.n_a = n_a, plan.n_v = n_v;
   plan.exchanges = std::any_of(teams.begin(), teams.end(), [](int t) { return t > 1; });
+  // (the first workgroup has the first rows of the largest instance, so others wait for it if any wait at all)
+  start[0] = start[1];
+  plan.start_without = std::move(start);
+  plan.d_start_without.release();
   plan.cus = device_cus();
   plan.kernel = plan.dg ? resident_dg_kernel(plan)
                         : reinterpret_cast<const void*>(plan.far ? far_kernel(plan.slots)
@@ -1116,7 +1120,11 @@ ResidentLaunch::ResidentLaunch(ResidentPlan& plan, ResidentParams P, const MfPar
   P.sell_local = plan.sell_local.ptr, P.halo_rows = plan.halo_rows.ptr, P.publish = plan.publish.ptr;
   P.tasks = plan.tasks.ptr, P.task_start = plan.task_start.ptr;
   P.gave_up = {plan.gave_up.ptr, plan.host_gave_up}, P.flags = plan.gave_up.ptr + 1;
-  P.wait_ticks = int64_t(4) * 100000000; // 4 s
+  if (P.wait_ticks == 0 && plan.exchanges) {
+    if (!plan.d_start_without.ptr)
+      plan.d_start_without.upload(plan.start_without);
+    P.task_start = plan.d_start_without.ptr;
+  }
   *plan.host_gave_up = 0;
   const int64_t nx = int64_t(plan.exchange.count);
   if (plan.exchanges)

@@ -82,7 +82,7 @@ struct ResidentParams {
   const int32_t* task_start; // per workgroup
   int* flags;          // FAR: per workgroup, the step whose p it has published
   ResidentFlags gave_up;
-  int64_t wait_ticks;  // limit of one wait, in ticks of the 100 MHz counter
+  int64_t wait_ticks;  // limit of one wait, in ticks of the 100 MHz counter; 0: a launch that exchanges gives up
 };
 
 // launch plan of an operator: kept with its solver data, rebuilt when partitions or storage change
@@ -107,6 +107,9 @@ struct ResidentPlan {
   DeviceArray<uint32_t> publish;
   DeviceArray<ResidentTask> tasks;
   DeviceArray<int32_t> task_start;
+  // the same with no task for the first workgroup, which the others of its instance then wait for (waits of length 0)
+  std::vector<int32_t> start_without;
+  DeviceArray<int32_t> d_start_without;
   DeviceArray<double> exchange; // g1, g2
   DeviceArray<int> gave_up;    // and the flags of the workgroups behind it
   int* host_gave_up = nullptr;

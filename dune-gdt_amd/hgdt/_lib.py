@@ -205,6 +205,7 @@ SIGNATURES = {
     "hgdt_operator_instance_stats": (ctypes.c_int, [_vp, _pi64, _pdbl]),
     "hgdt_operator_instance_true_residuals": (ctypes.c_int, [_vp, _pdbl]),
     "hgdt_operator_solve_workgroups": (ctypes.c_int, [_vp, _pi32]),
+    "hgdt_operator_set_solve_wait": (ctypes.c_int, [_vp, _dbl]),
     "hgdt_space_error_norms_noalloc": (ctypes.c_int, [_vp, _vp, _i32, _vp, _vp, _vp, _dbl, _pdbl, _vp]),
     "hgdt_noalloc_scratch_bytes": (ctypes.c_int, [_pi64]),
     "hgdt_operator_assembly_info": (ctypes.c_int, [_vp, _pi32, _pi32]),

@@ -1053,6 +1053,11 @@ class MatrixOperator:
         L.call("hgdt_operator_solve_workgroups", self._h, ctypes.byref(w))
         return int(w.value)
 
+    def set_solve_wait(self, seconds):
+        """how long a workgroup of a solve in one launch waits for the others (4 s by default) before the solve, and the
+        next 16, take kernels per iteration; 0: every launch whose workgroups wait gives up"""
+        L.call("hgdt_operator_set_solve_wait", self._h, float(seconds))
+
     def adjoint_log_diffusion_gradient(self, u, lam, form_index=0, stream=None):
         """grad_e = -kappa_e lambda_e^T Khat_e u_e (no reference counterpart)."""
         u = _dvec(u, self.shape[0], "u")

@@ -460,6 +460,12 @@ hgdt_status hgdt_operator_instance_stats(hgdt_operator op, int64_t* iterations, 
 hgdt_status hgdt_operator_instance_true_residuals(hgdt_operator op, double* relres);
 /* workgroups of the launch that ran the last apply_inverse as a whole (0: it issued kernels per iteration) */
 hgdt_status hgdt_operator_solve_workgroups(hgdt_operator op, int32_t* workgroups);
+/* How long a workgroup of a solve in one launch waits for the others (4 s by default; no reference counterpart).
+ * They have to be on the GPU together: the library counts the CUs of this process's solves, but another process
+ * may hold some.  When a wait ends, the solve goes on from its start with kernels per iteration, and so do the next
+ * 16 solves of the operator.  0: the launch is made without one of its workgroups, so that it always gives up (for tests
+ * of what follows); a solve in which no workgroup waits for another is not affected. */
+hgdt_status hgdt_operator_set_solve_wait(hgdt_operator op, double seconds);
 
 /* Adjoint element kernel (no reference counterpart): for the Laplace form appended at position
  * `form_index` among the element forms, with per-element diffusion kappa_e,
