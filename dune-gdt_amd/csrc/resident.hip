@@ -996,16 +996,46 @@ void resident_plan_dia(ResidentPlan& plan, const Operator& op, const std::vector
   resident_finish(plan, op, tasks, lds_of(slots, reach, s_nu), F.A.nblocks, F.V.nblocks);
 }
 
-// columns of the rows [r0, r1) that lie outside them, ascending
-static void halo_of(const Operator& op, int64_t r0, int64_t r1, std::vector<int32_t>& halo)
-{
-  halo.clear();
-  for (int64_t k = op.row_ptr[r0]; k < op.row_ptr[r1]; ++k)
-    if (op.cols[k] < r0 || op.cols[k] >= r1)
-      halo.push_back(op.cols[k]);
-  std::sort(halo.begin(), halo.end());
-  halo.erase(std::unique(halo.begin(), halo.end()), halo.end());
-}
+// Columns of a block of rows that lie outside it, ascending, and the place of each in this list, by a table over the rows
+// of an instance (at most what 256 workgroups hold).  All entries listed and sorted, and a search per entry, took 34 ms of
+// the first solve of P2 on 300 x 350 x 2 triangles (60 ms with three steps), the tables take 12.
+class Halo {
+  const Operator& op_;
+  std::vector<int32_t> place_; // -1: not in the list
+  int64_t lo_ = 0;             // first row of the instance
+
+public:
+  std::vector<int32_t> list;
+  explicit Halo(const Operator& op)
+    : op_(op)
+  {
+  }
+  // rows [r0, r1) of the instance with the rows [lo, hi); false: a column of another instance (a caller's matrix)
+  bool of(int64_t r0, int64_t r1, int64_t lo, int64_t hi)
+  {
+    for (int32_t c : list)
+      place_[c - lo_] = -1;
+    list.clear();
+    lo_ = lo;
+    if (int64_t(place_.size()) < hi - lo)
+      place_.resize(hi - lo, -1);
+    for (int64_t k = op_.row_ptr[r0]; k < op_.row_ptr[r1]; ++k) {
+      const int32_t c = op_.cols[k];
+      if (c < lo || c >= hi)
+        return false;
+      if ((c < r0 || c >= r1) && place_[c - lo] < 0)
+        place_[c - lo] = 0, list.push_back(c);
+    }
+    std::sort(list.begin(), list.end());
+    for (size_t i = 0; i < list.size(); ++i)
+      place_[list[i] - lo] = int32_t(i);
+    return true;
+  }
+  int32_t place(int32_t c) const
+  {
+    return place_[c - lo_];
+  }
+};
 
 int resident_items_sell(const Operator& op)
 {
@@ -1017,18 +1047,18 @@ int resident_items_sell(const Operator& op)
       return false;
     // p of the own rows and the halo in LDS
     const int64_t R = int64_t(k) * RES_LANES;
-    std::vector<int64_t> first;
+    std::vector<std::pair<int64_t, size_t>> blocks; // first row, instance
     for (size_t in = 0; in + 1 < row0.size(); ++in)
       for (int64_t r = row0[in]; r < row0[in + 1]; r += R)
-        first.push_back(r);
-    first.push_back(row0.back());
+        blocks.push_back({r, in});
     std::atomic<int64_t> most{0};
-    parallel_for(int64_t(first.size()) - 1, [&](int64_t b0, int64_t b1) {
-      std::vector<int32_t> halo;
+    parallel_for(int64_t(blocks.size()), [&](int64_t b0, int64_t b1) {
+      Halo halo(op);
       for (int64_t b = b0; b < b1; ++b) {
-        halo_of(op, first[b], first[b + 1], halo);
+        const int64_t r = blocks[b].first, lo = row0[blocks[b].second], hi = row0[blocks[b].second + 1];
+        const int64_t size = halo.of(r, std::min(r + R, hi), lo, hi) ? int64_t(halo.list.size()) : RES_LDS;
         int64_t m = most;
-        while (m < int64_t(halo.size()) && !most.compare_exchange_weak(m, int64_t(halo.size())))
+        while (m < size && !most.compare_exchange_weak(m, size))
           ;
       }
     });
@@ -1054,51 +1084,63 @@ void resident_plan_sell(ResidentPlan& plan, const Operator& op)
   if (!list_tasks(op, slots, RES_LANES, tasks))
     return;
   const int64_t R = int64_t(slots) * RES_LANES, nt = int64_t(tasks.size());
-  std::vector<std::vector<int32_t>> halo(nt);
-  parallel_for(nt, [&](int64_t b0, int64_t b1) {
-    for (int64_t b = b0; b < b1; ++b)
-      halo_of(op, tasks[b].row0, tasks[b].row0 + tasks[b].rows, halo[b]);
-  });
-  // the rows that other workgroups read
-  std::vector<uint8_t> read(std::max<int64_t>(op.n, 1), 0);
-  std::vector<int32_t> rows;
-  int64_t most = 0, slices = 0;
-  for (int64_t b = 0; b < nt; ++b) {
-    tasks[b].halo0 = int32_t(rows.size()), tasks[b].nhalo = int32_t(halo[b].size());
-    tasks[b].slice0 = int32_t(slices);
-    slices += (tasks[b].rows + 63) / 64;
-    most = std::max<int64_t>(most, tasks[b].nhalo);
-    for (int32_t c : halo[b])
-      read[c] = 1;
-    rows.insert(rows.end(), halo[b].begin(), halo[b].end());
-  }
-  if (slices != F.nslices || (R + most) * int64_t(sizeof(double)) > RES_LDS)
-    return;
-  std::vector<uint32_t> pub(nt * RES_LANES, 0u);
-  std::vector<uint16_t> local(std::max<size_t>(F.d_sell_vals.count, 1), 0);
+  const std::vector<int64_t>& row0 = op.space->inst_dof;
   std::vector<int64_t> slice_ptr(F.nslices + 1);
   F.d_slice_ptr.download(slice_ptr.data());
+  int64_t slices = 0;
+  for (ResidentTask& K : tasks) {
+    K.slice0 = int32_t(slices);
+    slices += (K.rows + 63) / 64;
+  }
+  if (slices != F.nslices)
+    return;
+  std::vector<std::vector<int32_t>> halo(nt);
+  std::vector<uint16_t> local(std::max<size_t>(F.d_sell_vals.count, 1), 0);
+  std::atomic<bool> fits{true};
   parallel_for(nt, [&](int64_t b0, int64_t b1) {
-    for (int64_t b = b0; b < b1; ++b) {
+    Halo h(op);
+    for (int64_t b = b0; b < b1 && fits; ++b) {
       const ResidentTask& K = tasks[b];
-      const std::vector<int32_t>& h = halo[b];
+      if (!h.of(K.row0, K.row0 + K.rows, row0[K.inst], row0[K.inst + 1]) ||
+          (R + int64_t(h.list.size())) * int64_t(sizeof(double)) > RES_LDS) {
+        fits = false;
+        return;
+      }
+      halo[b] = h.list;
       for (int o = 0; o < K.rows; ++o) {
         const int64_t i = K.row0 + o;
-        if (read[i])
-          pub[b * RES_LANES + o % RES_LANES] |= 1u << (o / RES_LANES);
         const int64_t sl = K.slice0 + o / 64;
         const int64_t w = (slice_ptr[sl + 1] - slice_ptr[sl]) / 64, len = op.row_ptr[i + 1] - op.row_ptr[i];
         for (int64_t k = 0; k < w; ++k) {
           int64_t at = o; // padding: the own row, as the columns of the storage
           if (k < len) {
             const int32_t c = op.cols[op.row_ptr[i] + k];
-            at = (c >= K.row0 && c < K.row0 + K.rows) ? c - K.row0
-                                                      : R + (std::lower_bound(h.begin(), h.end(), c) - h.begin());
+            at = (c >= K.row0 && c < K.row0 + K.rows) ? c - K.row0 : R + h.place(c);
           }
           local[slice_ptr[sl] + k * 64 + o % 64] = uint16_t(at);
         }
       }
     }
+  });
+  if (!fits)
+    return;
+  // the rows that other workgroups read
+  std::vector<uint8_t> read(std::max<int64_t>(op.n, 1), 0);
+  std::vector<int32_t> rows;
+  int64_t most = 0;
+  for (int64_t b = 0; b < nt; ++b) {
+    tasks[b].halo0 = int32_t(rows.size()), tasks[b].nhalo = int32_t(halo[b].size());
+    most = std::max<int64_t>(most, tasks[b].nhalo);
+    for (int32_t c : halo[b])
+      read[c] = 1;
+    rows.insert(rows.end(), halo[b].begin(), halo[b].end());
+  }
+  std::vector<uint32_t> pub(nt * RES_LANES, 0u);
+  parallel_for(nt, [&](int64_t b0, int64_t b1) {
+    for (int64_t b = b0; b < b1; ++b)
+      for (int o = 0; o < tasks[b].rows; ++o)
+        if (read[tasks[b].row0 + o])
+          pub[b * RES_LANES + o % RES_LANES] |= 1u << (o / RES_LANES);
   });
   plan.sell_local.upload(local);
   if (rows.empty())
