@@ -1332,7 +1332,7 @@ hgdt_status hgdt_operator_set_launch(hgdt_operator op, int32_t kernel, int32_t b
     Launch& L = op->op->launch[kernel];
     if ((kernel == 3 || kernel == 4) && (L.block != block_size || L.items != items_per_thread)) {
       op->op->fmt.partitions_ready = false;
-      if (kernel == 3 && op->op->fmt.format == HGDT_FORMAT_SELL) { // SELL slices follow the A partition
+      if (kernel == 3 && op->op->fmt.format == HGDT_FORMAT_SELL) { // (format_info is refused until the next application)
         op->op->fmt.structure_ready = false;
         op->op->fmt.valid = false;
       }

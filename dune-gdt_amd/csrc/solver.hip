@@ -1402,7 +1402,7 @@ struct SolverCache {
   ResidentShape shape_dia;
   std::vector<std::vector<int64_t>> shape_offs;
   int shape_nu = -1;
-  int sell_items = 0; // SELL: rows per lane that suit a solve in one launch (0: none)
+  int sell_items = 0; // SELL: rows per lane that suit a solve in one launch (0: none, -1: not looked for yet)
   ~SolverCache()
   {
     for (auto& h : host_scalars)
@@ -1492,15 +1492,6 @@ void RowPartition::build_counts(const std::vector<int64_t>& inst_dof, const std:
 static bool blk_wanted(const Operator& op);
 static int kernel_format(const Operator& op);
 
-// the same as resident_shape below once C.sell_items is known for the pattern (its slices need not be built yet)
-static ResidentShape resident_shape_sell(const Operator& op)
-{
-  const SolverCache& C = *op.solver_cache;
-  if (op.launch[3].user || op.launch[4].user || !op.square() || !C.sell_items)
-    return {};
-  return {RES_BLOCK, C.sell_items};
-}
-
 // row blocks that suit a solve in one launch (resident.hip; the operator's and the vector kernels' alike); none: the
 // caller chose shapes, or the storage (once it is known) or size does not fit
 static ResidentShape resident_shape(const Operator& op)
@@ -1508,8 +1499,11 @@ static ResidentShape resident_shape(const Operator& op)
   SolverCache& C = *op.solver_cache;
   if (op.launch[3].user || op.launch[4].user || !op.square())
     return {};
-  if (op.fmt.format == HGDT_FORMAT_SELL && op.fmt.structure_ready)
-    return resident_shape_sell(op);
+  if (op.fmt.format == HGDT_FORMAT_SELL && op.fmt.valid) {
+    if (C.sell_items < 0)
+      C.sell_items = resident_items_sell(op);
+    return C.sell_items ? ResidentShape{RES_BLOCK, C.sell_items} : ResidentShape{};
+  }
   if (!op.fmt.valid || op.fmt.format != HGDT_FORMAT_DIA || kernel_format(op) != FMT_DIAS)
     return {};
   if (C.s_nu != C.shape_nu || C.s_offs != C.shape_offs) // (a batch's shape is a search over its instances)
@@ -1517,16 +1511,31 @@ static ResidentShape resident_shape(const Operator& op)
   return C.shape_dia;
 }
 
+// first slice of every row block of the SELL storage.  The slices are 64 rows of an instance each, whatever the row blocks
+// (of a multiple of 64 rows) are: only this table follows them
+static void build_block_slices(Operator& op)
+{
+  const SolverFormat& F = op.fmt;
+  const std::vector<int64_t>& row0 = op.space->inst_dof;
+  std::vector<int64_t> first(F.A.nblocks + 1);
+  int64_t slices = 0; // of the instances before
+  for (size_t in = 0; in + 1 < row0.size(); ++in) {
+    for (int64_t b = F.A.inst_block0[in]; b < F.A.inst_block0[in + 1]; ++b)
+      first[b] = slices + (F.A.row0[b] - row0[in]) / 64;
+    slices += (row0[in + 1] - row0[in] + 63) / 64;
+  }
+  first[F.A.nblocks] = slices;
+  cache_of(op).block_slice0.upload(first);
+}
+
 // row-block partitions of the operator (host set-up, O(number of blocks)), resident: its resident_shape.  The default
 // shape of the application depends on the caller's choice for either kernel, so a choice for the vector kernels alone can
-// change the operator's row blocks too: SELL slices follow these and are dropped with them, whatever the cause (the caller
-// goes through prepare_storage before they are read).
+// change the operator's row blocks too, and with them what follows them.
 static void build_partitions(Operator& op, const ResidentShape& resident)
 {
   SolverFormat& F = op.fmt;
   SolverCache& C = cache_of(op);
   const Space& s = *op.space;
-  const int sliced_block = F.A.block, sliced_items = F.A.items;
   // default launch shapes: one row per lane for the operator application (many blocks keep enough
   // loads in flight); the vector kernels take ~1024 blocks so that every block's reduction of an
   // instance's partials stays small
@@ -1559,14 +1568,14 @@ static void build_partitions(Operator& op, const ResidentShape& resident)
   F.d_inst_row0.upload(s.inst_dof);
   if (mf)
     mf_block_table(op);
-  if (F.format == HGDT_FORMAT_SELL && (F.A.block != sliced_block || F.A.items != sliced_items))
-    F.structure_ready = F.valid = false;
+  if (F.format == HGDT_FORMAT_SELL && F.structure_ready)
+    build_block_slices(op);
   F.partitions_ready = true;
   ++C.version; // captured graphs hold the launch shapes
 }
 
 // storage structure of the operator (host set-up): DIA offsets and CSR -> DIA positions, or the
-// SELL-64 slices of the A partition
+// SELL-64 slices of the instances
 // element-block storage is the default for discontinuous spaces with 4 DoFs per element
 static bool blk_wanted(const Operator& op)
 {
@@ -1945,47 +1954,41 @@ static void build_structure(Operator& op)
     F.d_dia.allocate(std::max<int64_t>(int64_t(nd) * op.n, 1));
   } else {
     F.format = HGDT_FORMAT_SELL;
-    C.sell_items = op.square() ? resident_items_sell(op) : 0;
-    if (resident_shape_sell(op) != C.shaped_for)
-      build_partitions(op, resident_shape_sell(op)); // (the slices follow the row blocks)
-    std::vector<int64_t> slice_ptr{0}, bslice0;
-    for (int64_t b = 0; b < F.A.nblocks; ++b) {
-      bslice0.push_back(int64_t(slice_ptr.size()) - 1);
-      for (int64_t r = F.A.row0[b]; r < F.A.row0[b + 1]; r += 64) {
+    C.sell_items = -1;
+    std::vector<int64_t> slice_ptr{0}, slice_row0;
+    for (int in = 0; in < ninst; ++in)
+      for (int64_t r = s.inst_dof[in]; r < s.inst_dof[in + 1]; r += 64) {
         int64_t w = 0;
-        for (int64_t i = r; i < std::min(r + 64, F.A.row0[b + 1]); ++i)
+        for (int64_t i = r; i < std::min(r + 64, s.inst_dof[in + 1]); ++i)
           w = std::max(w, op.row_ptr[i + 1] - op.row_ptr[i]);
+        slice_row0.push_back(r);
         slice_ptr.push_back(slice_ptr.back() + 64 * w);
       }
-    }
-    bslice0.push_back(int64_t(slice_ptr.size()) - 1);
+    slice_row0.push_back(op.n);
     F.nslices = int64_t(slice_ptr.size()) - 1;
     const int64_t total = slice_ptr.back();
     std::vector<int32_t> scols(std::max<int64_t>(total, 1));
     std::vector<int64_t> pos(std::max<int64_t>(op.nnz, 1));
-    parallel_for(F.A.nblocks, [&](int64_t b0, int64_t b1) {
-      for (int64_t b = b0; b < b1; ++b) {
-        int64_t sl = bslice0[b];
-        for (int64_t r = F.A.row0[b]; r < F.A.row0[b + 1]; r += 64, ++sl) {
-          const int64_t w = (slice_ptr[sl + 1] - slice_ptr[sl]) / 64;
-          for (int64_t i = r; i < r + 64; ++i) {
-            const int lane = int(i - r);
-            const int64_t len = (i < F.A.row0[b + 1]) ? op.row_ptr[i + 1] - op.row_ptr[i] : 0;
-            for (int64_t k = 0; k < w; ++k) {
-              const int64_t at = slice_ptr[sl] + k * 64 + lane;
-              if (k < len) {
-                scols[at] = op.cols[op.row_ptr[i] + k];
-                pos[op.row_ptr[i] + k] = at;
-              } else {
-                scols[at] = int32_t(std::min<int64_t>(i, op.ncols - 1)); // padding: zero value, valid column
-              }
+    parallel_for(F.nslices, [&](int64_t s0, int64_t s1) {
+      for (int64_t sl = s0; sl < s1; ++sl) {
+        const int64_t r = slice_row0[sl], w = (slice_ptr[sl + 1] - slice_ptr[sl]) / 64;
+        for (int64_t i = r; i < r + 64; ++i) {
+          const int lane = int(i - r);
+          const int64_t len = (i < slice_row0[sl + 1]) ? op.row_ptr[i + 1] - op.row_ptr[i] : 0;
+          for (int64_t k = 0; k < w; ++k) {
+            const int64_t at = slice_ptr[sl] + k * 64 + lane;
+            if (k < len) {
+              scols[at] = op.cols[op.row_ptr[i] + k];
+              pos[op.row_ptr[i] + k] = at;
+            } else {
+              scols[at] = int32_t(std::min<int64_t>(i, op.ncols - 1)); // padding: zero value, valid column
             }
           }
         }
       }
     });
     F.d_slice_ptr.upload(slice_ptr);
-    C.block_slice0.upload(bslice0);
+    build_block_slices(op);
     F.d_sell_cols.upload(scols);
     F.d_sell_pos.upload(pos);
     F.d_sell_vals.allocate(std::max<int64_t>(total, 1));
@@ -2197,10 +2200,8 @@ void Operator::materialize_values(hipStream_t stream)
 void Operator::prepare_solver(hipStream_t stream)
 {
   prepare_storage(stream);
-  if (const ResidentShape shape = resident_shape(*this); shape != cache_of(*this).shaped_for) {
+  if (const ResidentShape shape = resident_shape(*this); shape != cache_of(*this).shaped_for)
     build_partitions(*this, shape); // default shapes follow the storage
-    prepare_storage(stream);        // (and SELL slices the row blocks)
-  }
   // column windows for the current row blocks, on the device once the staged application is chosen
   // (set-up, never captured)
   SolverCache& C = cache_of(*this);
@@ -2355,7 +2356,7 @@ void Operator::prepare_storage(hipStream_t stream)
 
 void Operator::apply(const double* x, double* y, hipStream_t stream)
 {
-  prepare_solver(stream);
+  prepare_storage(stream); // (the solver's own row blocks and column windows are made for the first solve)
   if (fmt.format == HGDT_FORMAT_MATRIX_FREE) {
     MfVectors v;
     v.x = x, v.y = y;
