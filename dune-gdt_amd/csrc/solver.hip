@@ -1504,8 +1504,8 @@ static ResidentShape resident_shape(const Operator& op)
       C.sell_items = resident_items_sell(op);
     return C.sell_items ? ResidentShape{RES_BLOCK, C.sell_items} : ResidentShape{};
   }
-  if (!op.fmt.valid || op.fmt.format != HGDT_FORMAT_DIA || kernel_format(op) != FMT_DIAS)
-    return {};
+  if (!op.fmt.valid || op.fmt.format != HGDT_FORMAT_DIA || kernel_format(op) != FMT_DIAS || op.column_staging == 1)
+    return {}; // (column staging asked for: row blocks of one row per lane)
   if (C.s_nu != C.shape_nu || C.s_offs != C.shape_offs) // (a batch's shape is a search over its instances)
     C.shape_dia = resident_shape_dia(op.space->inst_dof, C.s_offs, C.s_nu), C.shape_offs = C.s_offs, C.shape_nu = C.s_nu;
   return C.shape_dia;
@@ -2576,8 +2576,10 @@ void Operator::apply_inverse(const double* b, double* x, const hgdt_solver_optio
   // current scalars in record 0 after each chunk; the last step of a solve runs in the chunk after the
   // one whose update met the tolerance (the stopping test is the first thing a step does)
   const int chunk = opt.check_every + (opt.check_every & 1);
-  // in one launch where the vectors fit on the chip (a timed solve issues the kernel that is timed)
-  bool solved = !opt.time_spmv && resident_plan(*this).usable;
+  // in one launch where the vectors fit on the chip (a timed solve issues the kernel that is timed, one for which the
+  // caller asked for column staging the kernel that has it)
+  const bool staged = kernel_format(*this) == FMT_DIAS && win_lds_bytes(*this) > 0 && C.win.ptr;
+  bool solved = !opt.time_spmv && !(staged && column_staging == 1) && resident_plan(*this).usable;
   if (solved && C.resident.skip > 0)
     --C.resident.skip, solved = false;
   std::unique_ptr<ResidentLaunch> launch; // (goes after the exit passes are queued and waited for)
@@ -2815,7 +2817,7 @@ void Operator::apply_inverse(const double* b, double* x, const hgdt_solver_optio
   // inside the application for the matrix-free SWIPDG operator) and the update (32 B per row)
   st.iteration_bytes = fmt.step_bytes + (fused_dir ? 0 : 36 * n) + 32 * n;
   st.compactions = compactions;
-  st.column_staged = (kernel_format(*this) == FMT_DIAS && win_lds_bytes(*this) > 0 && C.win.ptr) ? 1 : 0;
+  st.column_staged = staged && !solved ? 1 : 0;
   if (!st.converged) {
     if (st.breakdown)
       HGDT_THROW(HGDT_ERR_SOLVER_FAILED, "Jacobi-PCG breakdown: p.Ap <= 0 (matrix not SPD)");

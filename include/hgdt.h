@@ -438,8 +438,9 @@ typedef struct hgdt_solver_stats {
   int32_t column_staged;  /* 1: the solver's operator application ran with column staging (see
                              hgdt_operator_set_column_staging) */
   int32_t restarts;       /* restarts from the true residual taken (options.restarts) */
-  int64_t iteration_bytes; /* algorithmic bytes of one PCG iteration over all instances: the application
-                              (step_bytes), the direction update (36 B per DoF on average over the two
+  int64_t iteration_bytes; /* algorithmic bytes of one PCG iteration over all instances by kernels per iteration
+                              (a solve in one launch keeps the vectors on the chip and moves less): the
+                              application (step_bytes), the direction update (36 B per DoF on average over the two
                               parities of the deferred iterate update, none when the application does it)
                               and the update (32 B per DoF) */
 } hgdt_solver_stats;
@@ -488,8 +489,9 @@ hgdt_status hgdt_operator_get_launch(hgdt_operator op, int32_t kernel, int32_t* 
  * the one above).  With symmetric DIA storage, one row per lane (kernel 3 with items_per_thread 1), at most
  * 8 strict upper diagonals and the stencil's column offsets in at most 4 windows no wider than the block,
  * the entries of p a row block needs are loaded into LDS once per block and read from there.  mode -1
- * (default): staged when the application moves more than 256 MiB (beyond the GPU's last-level cache);
- * 0: never; 1: wherever it applies.  Results are the same bits either way. */
+ * (default): staged when the application moves more than 256 MiB (beyond the GPU's last-level cache) and the
+ * solve is not one launch as a whole; 0: never; 1: wherever it applies, with kernels per iteration (and default
+ * row blocks of one row per lane).  Results are the same bits either way for the same launch shapes. */
 hgdt_status hgdt_operator_set_column_staging(hgdt_operator op, int32_t mode);
 
 #ifdef __cplusplus

@@ -64,3 +64,31 @@ def test_vector_shape_of_a_used_operator(hgdt_mod, case, first):
     x = op.apply_inverse("rhs").cpu().numpy()
     assert np.linalg.norm(b - A @ x) <= 2e-10 * np.linalg.norm(b)
     assert torch.equal(op.apply(v), before)
+
+
+@pytest.mark.parametrize("shapes", [None, ((256, 1), (256, 1))])
+def test_column_staging_asked_for(hgdt_mod, shapes):
+    """mode 1 runs the staged application (kernels per iteration) wherever it applies, also where the solve would be one
+    launch; the other modes leave that to the size; storage without diagonals has nothing to stage"""
+    H = hgdt_mod
+    print(f"case column staging {shapes}", flush=True)
+    kappa = torch.from_numpy(H.fields.lognormal(7, 150 * 131)).cuda()
+    op = hgdt_problem(H, "heat_q1", [150, 131], kappa)[2]
+    if shapes:
+        op.set_launch(3, *shapes[0])
+        op.set_launch(4, *shapes[1])
+    op.assemble()
+    xs = []
+    for mode in (1, 0, 1, -1):
+        op.set_column_staging(mode)
+        xs.append(op.apply_inverse("rhs"))
+        assert op.last_solve["column_staged"] == (mode == 1), mode
+        assert (op.solve_workgroups() == 0) == (mode == 1), mode
+    assert torch.equal(xs[0], xs[2]) and torch.equal(xs[1], xs[3])
+    if shapes:
+        assert torch.equal(xs[0], xs[1])
+    op.set_column_staging(1)
+    op.set_format("sell64")
+    op.apply_inverse("rhs")
+    assert op.last_solve["column_staged"] == 0
+    assert shapes or op.solve_workgroups() > 0  # (general storage in one launch: blocks of 512 lanes)
