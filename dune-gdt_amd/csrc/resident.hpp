@@ -42,11 +42,11 @@ struct ResidentFlags {
 
 struct ResidentParams {
   int64_t n;
-  int ninst;
+  int zero_place; // discontinuous spaces: place of the zeros in p
   const int64_t* inst_row0;
   // launch shapes whose block partials (and therefore bits) the solve reproduces: vector blocks of v_block lanes and
   // 1 << v_lg_items rows per lane, operator blocks the same or of a_rows lanes with one row each
-  int a_rows, v_block, same_blocks;
+  int a_rows, v_block;
   // scaled symmetric DIA: strict upper slots
   int s_nu;
   const int64_t* s_off;
@@ -56,10 +56,9 @@ struct ResidentParams {
   const uint16_t* sell_local;
   const int32_t* halo_rows;
   const uint32_t* publish; // per workgroup and lane: the slots whose rows other workgroups read
-  // discontinuous spaces: elements of a workgroup, in order (-1: none; bit 30: read by other workgroups), place of the zeros
-  // in p; the scaled element blocks as the storage has them; reference data of the matrix-free operator
+  // discontinuous spaces: elements of a workgroup, in order (-1: none; bit 30: read by other workgroups); the scaled element
+  // blocks as the storage has them; reference data of the matrix-free operator
   const int32_t* dg_elements;
-  int zero_place;
   int blk_mn, blk_sym;
   int64_t blk_ne;
   const int32_t* blk_nb;

@@ -2490,9 +2490,8 @@ static std::unique_ptr<ResidentLaunch> resident_solve(Operator& op, const PcgPar
   const SolverFormat& F = op.fmt;
   SolverCache& C = cache_of(op);
   ResidentParams R{};
-  R.n = op.n, R.ninst = P.ninst, R.inst_row0 = P.inst_row0;
+  R.n = op.n, R.inst_row0 = P.inst_row0;
   R.a_rows = F.A.block * F.A.items, R.v_block = F.V.block;
-  R.same_blocks = C.resident.same_blocks;
   R.s_nu = P.s_nu, R.s_off = P.s_off, R.scaled = P.scaled, R.dsq = P.dsq, R.slice_ptr = P.slice_ptr;
   R.blk_ne = P.blk_ne, R.blk_mn = P.blk_mn, R.blk_sym = F.symmetric, R.blk_nb = P.blk_nb, R.blk_mir = P.blk_mir;
   R.dg_ref = F.d_mf_ref.ptr, R.dh = P.dh;
