@@ -28,6 +28,7 @@ sys.path.insert(0, os.path.join(ROOT, "dune-gdt_amd"))
 
 METRIC = "DoFs/s assembly+CG @1e-10 rel. residual FP64; batched/adjoint vs plain; % HBM peak"
 HBM_PEAK_GBS = 8000.0
+HBM_COPY_GBS = 4730.0  # what a large copy reaches (read + written)
 
 
 def log(msg):
@@ -222,28 +223,33 @@ def traffic_record(config, mf):
     return pmc_record(f"pmc_{'mf' if mf else 'cg_spmv'}_{config}.json")
 
 
-def pmc_record(name):
+def pmc_record(name, key="hbm_bytes_per_launch"):
     tfile = os.path.join(ROOT, "profiles", name)
     if not os.path.exists(tfile):
         return None, None
     with open(tfile) as f:
         d = json.load(f)
     src = f"profiles/{os.path.basename(tfile)} (rocprofv3 --pmc FETCH_SIZE, WRITE_SIZE; {d.get('date', 'undated')})"
-    return d.get("hbm_bytes_per_launch"), src
+    return d.get(key), src
 
 
 def one_launch_record(config, mf, stats, workgroups, step_bytes):
-    """the solves in one launch: their time against the bytes of an application per iteration (the matrix, p read and
-    the product written: what a solve that keeps nothing on the chip between two steps would have to move at least; with
-    the matrix in registers none of it is moved and the exchanges between the workgroups bound the step)"""
+    """the solves in one launch: the bytes that the counters saw per iteration (profiles/) over the time of the timed
+    steps' iterations.  Vectors, and the matrix where it fits, stay on the chip, so what an application alone would move
+    (application_bytes) is no measure of the launch; where the bytes moved are few, the exchanges between the workgroups
+    bound an iteration and not the memory"""
     iters = sum(s["iterations"] for s in stats)
     us = sum(s["solve_ms"] for s in stats) * 1e3
-    traffic, src = pmc_record(f"pmc_resident{'_mf' if mf else ''}_{config}.json")
-    rate = iters * step_bytes / (us * 1e-6) / 1e9
-    return {"kernel": "k_pcg_resident_dg" if config == "c3" else "k_pcg_resident", "workgroups": workgroups,
+    moved, src = pmc_record(f"pmc_resident{'_mf' if mf else ''}_{config}.json", "bytes_per_iteration")
+    rate = iters * moved / (us * 1e-6) / 1e9 if moved else None
+    per_launch = iters / len(stats)
+    return {"bound": "hbm" if rate and rate > 0.5 * HBM_COPY_GBS else "exchanges between workgroups",
+            "kernel": "k_pcg_resident_dg" if config == "c3" else "k_pcg_resident", "workgroups": workgroups,
             "avg_launch_us": us / len(stats), "us_per_iteration": us / iters, "achieved": rate, "peak": HBM_PEAK_GBS,
-            "unit": "GB/s", "frac": rate / HBM_PEAK_GBS, "bytes_per_launch": iters // len(stats) * step_bytes,
-            "traffic": traffic, "traffic_source": src,
+            "unit": "GB/s", "frac": rate / HBM_PEAK_GBS if rate else None,
+            "bytes_per_launch": int(per_launch * moved) if moved else None,
+            "traffic": moved * per_launch if moved else None, "traffic_source": src,
+            "application_bytes": step_bytes,
             "timing": "HIP events around the timed steps' solves (initial residual, the launch, exit passes)"}
 
 
@@ -370,8 +376,13 @@ def run_single(hgdt, torch, args, config, fmt, steps, warmup, spmv_sample):
     asm_bytes = op.assembly_bytes()
     it_bytes = int(stats[-1]["iteration_bytes"])
     mean_iters = float(np.mean([s["iterations"] for s in stats]))
-    total = asm_bytes + mean_iters * it_bytes
-    step_rate = total / (ms_per_step * 1e-3) / 1e9
+    basis = ("algorithmic bytes of the assembly and of the step's iterations (operator application, direction update, "
+             "update; the formats' compulsory bytes, as the roofline's)")
+    if workgroups:  # in one launch: what the counters saw (nothing where there is no such record)
+        it_bytes = pmc_record(f"pmc_resident{'_mf' if mf else ''}_{config}.json", "bytes_per_iteration")[0]
+        basis = "algorithmic bytes of the assembly, and the bytes that the counters saw per iteration of the launch,"
+    total = asm_bytes + mean_iters * it_bytes if it_bytes else None
+    step_rate = total / (ms_per_step * 1e-3) / 1e9 if total else None
     res = {
         "value": n / (ms_per_step * 1e-3), "ms_per_step": ms_per_step,
         "config": {"workload": workload, "dofs": n, "elements": grid.num_elements, "nnz": op.nnz,
@@ -388,17 +399,16 @@ def run_single(hgdt, torch, args, config, fmt, steps, warmup, spmv_sample):
                                "from the end of "
                                "the kernel before the application (the direction update; for a matrix-free application "
                                "fused with it, the previous iteration's update) to the application's end"},
-        "step_hbm": {"achieved": step_rate, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": step_rate / HBM_PEAK_GBS,
+        "step_hbm": {"achieved": step_rate, "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                     "frac": step_rate / HBM_PEAK_GBS if step_rate else None,
                      "bytes_per_step": total, "assembly_bytes": asm_bytes, "iteration_bytes": it_bytes,
-                     "basis": "algorithmic bytes of the assembly and of the step's iterations (operator application, "
-                              "direction update, update; the formats' compulsory bytes, as the roofline's) over "
-                              "ms_per_step; the solve's set-up and exit passes (initial residual, the solver's scaled "
-                              "copy, true residual) are not counted"},
+                     "basis": basis + " over ms_per_step; the solve's set-up and exit passes (initial residual, the "
+                                      "solver's scaled copy, true residual) are not counted"},
     }
     if workgroups:
         # the timed steps' dominant kernel; the application of the three-kernel iteration beside it
         res["roofline_application"] = res["roofline"]
-        res["roofline"] = {"bound": "hbm", **one_launch_record(config, mf, stats, workgroups, step_bytes)}
+        res["roofline"] = one_launch_record(config, mf, stats, workgroups, step_bytes)
     return res, (grid, space, op, kappa, x)
 
 
