@@ -19,8 +19,8 @@
 // caches are coherent; as every value is its own flag, no order between different addresses is needed beyond that.
 //
 // Every value is computed by the operations of the three kernels in their order (row sums, block partials in
-// the operator's and the vector partition, sums over the partials), so a solve gives the same bits on either path,
-// alone or in a batch.
+// the operator's and the vector partition, sums over the partials), so for the same launch shapes a solve gives the same
+// bits on either path, alone or in a batch.  (The default shapes follow the size: of the instance, or of the batch.)
 //
 // Measured (us per iteration, three kernels -> one launch): Q1 32^2 15 -> 2.3, 128^2 14 -> 4.5, 701x523 18 -> 7.8, 1023^2
 // 33 -> 11.8, P1 48^3 x 6 18 -> 7.0, eight of these in a batch 33 -> 9.4, 100^3 x 6 34 -> 19, 128^3 x 6 54 -> 27; SELL: P1
@@ -32,8 +32,9 @@
 // behind the L2 caches (104 MB of matrix and far p read, 17 MB of p written per iteration: 4.3 TB/s, the rate of a copy).
 //
 // All workgroups of a team must be on the chip together: the host launches at most one per CU and counts the
-// CUs of all running launches of the process.  A wait that outlasts its limit (another process holds the
-// CUs) sets a flag at which every workgroup ends; the caller then solves with the three kernels.
+// CUs of all running launches of the process.  A wait that outlasts its limit (Operator::solve_wait: another process holds
+// the CUs, or in a batch a partner is still busy with an earlier instance) sets a flag at which every workgroup ends; the
+// caller then solves with the three kernels.
 
 #include <algorithm>
 #include <atomic>

@@ -11,7 +11,9 @@
 // A workgroup's elements are a rectangle of the lattice where there is one (halo: its perimeter), else consecutive.
 // The matrix-free solve runs in the unscaled variables (r, z = D^{-1} r, p): neighbours then need z alone, not also their
 // D^{-1/2}.  The sums of p.q and of the norms are those of the workgroups in their order: the three kernels
-// add the same terms in another order, so a solve agrees with theirs up to round-off and not bit for bit.
+// add the same terms in another order, so a solve agrees with theirs up to round-off and not bit for bit.  One instance that is
+// too large changes the elements per lane (matrix-free) or the path (blocks) of its whole batch, and with them the
+// rounding of the others.
 // Measured (us per iteration, three kernels -> one launch): element blocks 256 x 192 elements 17.7 -> 5.1, matrix-free
 // 512 x 512 elements 23.6 -> 8.7.  What bounds an iteration now: the two exchanges (2.4-3.5 us each with 96-256
 // workgroups) and the barriers around them.  More than 131 072 elements with their blocks do not fit in the

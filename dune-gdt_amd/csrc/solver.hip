@@ -311,7 +311,8 @@ __device__ __forceinline__ void apply_rows(const PcgParams& P, const double* __r
 
 // y = A x, one row per lane.  PLAIN: row blocks of as many rows as a workgroup has lanes.  Otherwise (several rows per
 // lane in the solver's kernels) `per` workgroups share a row block, as apply_split says.
-// Both are bound by the requests to L1 and L2 (values and x of 8 bytes per entry).  Measured (us per call): Q1 on 96^3
+// Both are bound by the memory behind the L2 caches (Q1 on 96^3 hexahedra: 151 MB in 38 us, 1.3 times the compulsory bytes;
+// 27 us while the last-level cache holds the operator).  Measured (us per call, operators in turn): Q1 on 96^3
 // hexahedra, row blocks of 256 x 1, 36.2 in the plain form and 36.75 in the other (its division of the workgroup's number
 // ahead of the first load); P1 on 112 x 100 x 112 x 6 tetrahedra, row blocks of 768 x 4, 30.4 with workgroups of 768 lanes
 // and 29.2 with 256, which leave the CUs in smaller pieces.

@@ -158,7 +158,9 @@ def save_table(op, choice, table_file):
 
 
 def tune_assembly(op, repeats=3, verbose=False):
-    """Pick the block size of the element / intersection / scatter kernels (one launch shape each)."""
+    """Pick the block size of the element / intersection / scatter kernels (one launch shape each).  Symmetric forms on
+    discontinuous order-1 spaces of triangles, quadrilaterals and tetrahedra are assembled by one kernel of a fixed shape:
+    there the scatter kernel's choice has no effect, the intersection kernel's only on the boundary."""
     best = {}
     for kernel in (L.KERNEL_ELEMENT, L.KERNEL_INTERSECTION, L.KERNEL_GATHER):
         results = {}
