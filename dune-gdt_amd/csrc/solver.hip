@@ -2498,7 +2498,7 @@ static std::unique_ptr<ResidentLaunch> resident_solve(Operator& op, const PcgPar
   R.dg_ref = F.d_mf_ref.ptr, R.dh = P.dh;
   R.r = P.r, R.x = P.x, R.x_out = P.q, R.r_pub[0] = P.p, R.r_pub[1] = P.p2, R.part2 = P.part2;
   R.S = P.S, R.result = C.host_scalars[0], R.max_iter = P.max_iter;
-  R.wait_ticks = int64_t(op.solve_wait * 1e8);
+  R.wait_ticks = op.solve_wait > 0. ? std::max(int64_t(1), int64_t(op.solve_wait * 1e8)) : 0; // (0 leaves a workgroup out)
   return std::make_unique<ResidentLaunch>(C.resident, R, F.format == HGDT_FORMAT_MATRIX_FREE ? mf_params(op) : MfParams{},
                                           stream);
 }

@@ -141,3 +141,17 @@ def test_solves_that_exceed_the_cus_together(hgdt_mod):
     [t.join() for t in th]
     for k in range(2):
         assert len(got[k]) == 4 and all(torch.equal(x, alone[k]) for x in got[k]) and min(groups[k]) > 0
+
+
+def test_shortest_wait(hgdt_mod):
+    """a limit below the clock's resolution is a limit, not 0: the launch is complete, and waits of some microseconds end
+    before the clock is looked at"""
+    print("case shortest wait", flush=True)
+    op = _operator(hgdt_mod, "dia")
+    want = op.apply_inverse("rhs", time_spmv=8)
+    op.set_solve_wait(1e-12)
+    groups = []
+    for _ in range(40):  # (were one to give up all the same, the 17th after it is tried again)
+        assert torch.equal(op.apply_inverse("rhs"), want)
+        groups.append(op.solve_workgroups())
+    assert max(groups) > 1
